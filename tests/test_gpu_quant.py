@@ -99,6 +99,26 @@ def test_act_quant_matches_oracle(gpu, block, pow2):
     assert bits_equal(np_(deq), od)
 
 
+@pytest.mark.parametrize("rows,n,block,shift", [(1, 8, 8, 0), (3, 48, 16, 0), (7, 192, 64, 0), (33, 512, 256, 0),
+                                                (2, 1024, 512, 0), (300, 896, 128, 0), (5, 96, 24, 0), (3, 64, 4, 0),
+                                                (3, 1024, 1024, 0), (4, 256, 32, 1)])
+@pytest.mark.parametrize("pow2", [True, False])
+def test_act_quant_block_lengths_and_alignment(gpu, rows, n, block, shift, pow2):
+    # blocks of 1, 2, 4, ... 64 lanes of 8 values (partial workgroups among them), and the block lengths
+    # and the unaligned x that take one thread per block: all as the oracle, bit for bit
+    x = (data.normal((rows, n), 1.0, seed=rows + n) * torch.logspace(-4, 4, n)).to(torch.bfloat16)
+    x[-1, -1] = float("inf")
+    x[0, 0] = float("nan")
+    buf = torch.zeros(rows * n + 8, dtype=torch.bfloat16, device=gpu)
+    xg = buf[shift:shift + rows * n].view(rows, n)
+    xg.copy_(x)
+    codes, scales, deq = ops.act_quant(xg, block, pow2, want_deq=True)
+    oc, os_, od = oracle.act_quant(x.float().numpy(), block, pow2)
+    assert np.array_equal(np_(scales), os_)
+    assert np.array_equal(np_(codes), oc)
+    assert bits_equal(np_(deq), od)
+
+
 def test_stbl_act_quant_fp8_inplace(gpu):
     # the reference engine's form (stbl/kernels.cu:54-63): fp32 buffer of bf16 values, block 32
     x = (data.normal((4, 256), 3.0, seed=7)).to(torch.bfloat16).float()
