@@ -124,7 +124,8 @@ __device__ __forceinline__ float e2m1_value(uint32_t c) {
 __device__ __forceinline__ float round_fp4(float v) {
     const float a = fabsf(v);
     const float step = a < 2.f ? .5f : (a < 4.f ? 1.f : 2.f);
-    return copysignf(rintf(a / step) * step, v);
+    const float inv = a < 2.f ? 2.f : (a < 4.f ? 1.f : .5f);  // 1 / step, exact
+    return copysignf(rintf(a * inv) * step, v);
 }
 
 // e2m1 code of a grid value (ref/kernel.py:75-77): magnitude index | sign bit << 3.

@@ -85,6 +85,34 @@ def test_quant_fp8_e8m0_matches_oracle(gpu, rows, k):
 
 
 
+@pytest.mark.parametrize("rows,k,shift", [(1, 128, 0), (129, 132, 0), (127, 1412, 0), (200, 130, 0), (130, 260, 1),
+                                          (256, 384, 2)])
+def test_quant_fp8_b128_edges_and_alignment(gpu, rows, k, shift):
+    # whole and partial blocks read 16 bytes at a time, and the k and the unaligned w that are read value
+    # by value; an infinity gives its block the scale +Inf, a NaN is skipped by the maximum
+    w = data.weight(rows, k, seed=rows + k) * torch.logspace(-6, 6, k)
+    w[0, 0], w[-1, -1] = float("nan"), float("inf")
+    buf = torch.zeros(rows * k + 4, device=gpu)
+    wg = buf[shift:shift + rows * k].view(rows, k)
+    wg.copy_(w)
+    codes, scales = ops.quant_fp8_b128(wg)
+    oc, os_ = oracle.quant_fp8_b128(w.numpy())
+    assert np.array_equal(np_(scales), os_)
+    assert np.array_equal(np_(codes), oc)
+
+
+@pytest.mark.parametrize("rows,k,shift", [(1, 32, 0), (33, 160, 0), (95, 2304, 0), (64, 128, 1)])
+def test_quant_fp8_e8m0_edges_and_alignment(gpu, rows, k, shift):
+    w = data.weight(rows, k, seed=rows + k) * torch.logspace(-6, 6, k)
+    w[0, 0], w[-1, -1] = float("nan"), float("-inf")
+    buf = torch.zeros(rows * k + 4, device=gpu)
+    wg = buf[shift:shift + rows * k].view(rows, k)
+    wg.copy_(w)
+    codes, scales = ops.quant_fp8_e8m0(wg)
+    oc, os_ = oracle.quant_fp8_e8m0_b32(w.numpy())
+    assert np.array_equal(np_(codes), oc) and np.array_equal(np_(scales), os_)
+
+
 @pytest.mark.parametrize("block,pow2", [(32, True), (128, True), (128, False)])
 def test_act_quant_matches_oracle(gpu, block, pow2):
     x = (data.normal((5, 1024), 1.0, seed=block) * torch.logspace(-3, 3, 1024)).to(torch.bfloat16)
