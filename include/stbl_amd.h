@@ -155,6 +155,14 @@ enum { STBL_AMD_FP4 = 0, STBL_AMD_FP8 = 1, STBL_AMD_FP8_E8M0 = 2 };
  * NULL) and returns the slot size. Replaces the gate|up|down slot of stbl/model.cu:374-381. */
 uint64_t stbl_amd_expert_layout(int fmt, int dim, int inter, uint64_t *offsets);
 
+/* An expert's fp32 gate and up [inter x dim] and down [dim x inter] quantized into its slot (the layout
+ * above, each matrix as stbl_amd_quant_fp4 / _fp8_b128 / _fp8_e8m0 quantizes it) in one launch; bytes
+ * between the parts are left alone. slot and weights 16-byte aligned and not overlapping; dim and inter
+ * % 32 == 0 (FP4, FP8_E8M0) or % 4 == 0 (FP8). No counterpart in the reference, whose weights arrive
+ * quantized (tools/convert_official.py:53-54). */
+int stbl_amd_quant_expert(int fmt, void *slot, const float *w_gate, const float *w_up, const float *w_down, int dim,
+                          int inter, hipStream_t st);
+
 /* One expert FFN on m <= 4 tokens (stbl/model.cu:516-547 for one expert):
  * y[t] = bf16(down . act(swiglu(bf16(gate . act(x_t)), bf16(up . act(x_t)), weight, limit)))
  * where act is act_quant(., 32, ue8m0, inplace) when `official`, else the identity, and swiglu is

@@ -47,6 +47,7 @@ SIGNATURES = {
     "stbl_amd_dequant_gguf17": (I, [P, P, I, I, P]),
     "stbl_amd_dequant_fp8": (I, [P, P, P, I, I, I, P]),
     "stbl_amd_expert_layout": (U64, [I, I, I, PU64]),
+    "stbl_amd_quant_expert": (I, [I, P, P, P, P, I, I, P]),
     "stbl_amd_expert_ffn": (I, [I, P, P, P, I, I, I, F, F, I, I, P, P]),
     "stbl_amd_moe_experts": (I, [I, P, P, I, I, I, PP, I, PI, PF, I, I, I, F, I, I, P, P]),
     "stbl_amd_moe_experts_phase": (I, [I, P, P, I, I, I, PP, I, PI, PF, I, I, I, F, I, I, PI, I, P, P]),

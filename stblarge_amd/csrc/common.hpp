@@ -120,21 +120,6 @@ __device__ __forceinline__ float e2m1_value(uint32_t c) {
     return (c & 8u) ? -mag : mag;
 }
 
-// Onto the e2m1 grid, ties to even (ref/kernel.py:48-52); v is within [-6, 6].
-__device__ __forceinline__ float round_fp4(float v) {
-    const float a = fabsf(v);
-    const float step = a < 2.f ? .5f : (a < 4.f ? 1.f : 2.f);
-    const float inv = a < 2.f ? 2.f : (a < 4.f ? 1.f : .5f);  // 1 / step, exact
-    return copysignf(rintf(a * inv) * step, v);
-}
-
-// e2m1 code of a grid value (ref/kernel.py:75-77): magnitude index | sign bit << 3.
-__device__ __forceinline__ uint32_t fp4_code(float q) {
-    const float a = fabsf(q);
-    const uint32_t m = a <= 1.5f ? (uint32_t)(a * 2.f) : (a <= 3.f ? (uint32_t)(a + 2.f) : (a <= 4.f ? 6u : 7u));
-    return m | ((__float_as_uint(q) >> 28) & 8u);
-}
-
 // ---- wave reductions -----------------------------------------------------------------------------
 
 __device__ __forceinline__ float wave_sum(float v) {

@@ -9,6 +9,7 @@
 // All are bound by their bytes; the quantizers read each value once, in 16-byte loads.
 #include "common.hpp"
 #include "abi_util.hpp"
+#include "expert_layout.hpp"
 
 namespace stbl {
 
@@ -137,30 +138,65 @@ __global__ void k_act_quant(const uint16_t *x, int n_blocks, int block, int pow2
 
 // ---- weight quantizers ---------------------------------------------------------------------------
 
+// The matrices of one launch: a matrix on its own, or the three of an expert, whose launch then fills
+// the GPU to the end once instead of three times (quantizing a 7168 x 2048 expert into its slot: three FP8
+// launches and six copies of their outputs 69.1 us, one launch 37.7).
+struct QuantJob {
+    const float *w;
+    uint8_t *codes;
+    void *scales;
+    int rows, k;
+    uint32_t first;  // the matrix's first workgroup; past every workgroup for an unused entry
+};
+struct QuantJobs {
+    QuantJob j[3];
+};
+
+// This workgroup's matrix, and its index among the matrix's workgroups in `b`.
+__device__ __forceinline__ const QuantJob &quant_job(const QuantJobs &jobs, uint32_t &b) {
+    const int m = (blockIdx.x >= jobs.j[1].first) + (blockIdx.x >= jobs.j[2].first);
+    b = blockIdx.x - jobs.j[m].first;
+    return jobs.j[m];
+}
+
 // FP4 e2m1 with E8M0 scales per 32 along K. Four lanes per group of 32, 8 values (two 16-byte loads)
-// each: a wave reads 2 KB and writes 256 bytes of codes (element 2i in the low nibble) in contiguous
-// runs, and the group's maximum comes over two DPP moves. s is a power of two, so w times its exact
-// inverse is w / s. Bound by its bytes: 7168 x 2048 23.3 -> 14.6 us (4.6 TB/s) against one thread per group (128 bytes
-// apart, so each load of a wave touched 64 lines).
-__global__ __launch_bounds__(256) void k_quant_fp4(const float *__restrict__ w, size_t n8, uint8_t *__restrict__ codes,
-                                                   uint8_t *__restrict__ scales) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const bool ok = i < n8;  // n8 is a multiple of 4: a group's lanes are all in or all out
-    const f32x4 *src = (const f32x4 *)(w + (ok ? i : 0) * 8);
-    const f32x4 a = __builtin_nontemporal_load(src), b = __builtin_nontemporal_load(src + 1);
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    float amax = 0.f;
+// each, two groups per lane: a wave reads 2 KB and writes 256 bytes of codes (element 2i in the low
+// nibble) in contiguous runs, and a group's maximum comes over two DPP moves. s is a power of two, so w
+// times its exact inverse is w / s. Bound by its bytes: 7168 x 2048 23.3 us with one thread per group
+// (128 bytes apart, so each load of a wave touched 64 lines), 20.5 with 16 consecutive values a lane,
+// 16.6 with 4, 15.8 with 8 rounded in software, 14.2 (4.7 TB/s) so.
+__global__ __launch_bounds__(256) void k_quant_fp4(QuantJobs jobs) {
+    uint32_t wg;
+    const QuantJob &J = quant_job(jobs, wg);
+    const size_t n8 = (size_t)J.rows * (J.k >> 3);  // a multiple of 4: a group's lanes are all in or all out
+    const size_t i0 = (size_t)wg * 512 + threadIdx.x;
+    f32x4 v[2][2];
 #pragma unroll
-    for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(v[j]));
-    amax = fmaxf(group_max(amax, 4), 6.0f * 0x1p-126f);
-    const float s = pow2_ceil(amax * (float)(1.0 / 6.0));
-    const float inv = pow2_inverse(s);
-    uint32_t word = 0;
+    for (int q = 0; q < 2; q++) {
+        const f32x4 *src = (const f32x4 *)J.w + 2 * (i0 + 256 * q < n8 ? i0 + 256 * q : 0);
+        v[q][0] = __builtin_nontemporal_load(src);
+        v[q][1] = __builtin_nontemporal_load(src + 1);
+    }
 #pragma unroll
-    for (int j = 0; j < 8; j++) word |= fp4_code(round_fp4(fminf(fmaxf(v[j] * inv, -6.f), 6.f))) << (4 * j);
-    if (!ok) return;
-    *(uint32_t *)(codes + i * 4) = word;
-    if ((threadIdx.x & 3) == 0) scales[i >> 2] = (uint8_t)((__float_as_uint(s) >> 23) & 0xffu);
+    for (int q = 0; q < 2; q++) {
+        const size_t i = i0 + 256 * q;
+        float amax = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(v[q][j >> 2][j & 3]));
+        amax = fmaxf(group_max(amax, 4), 6.0f * 0x1p-126f);
+        const float s = pow2_ceil(amax * (float)(1.0 / 6.0));
+        const float inv = pow2_inverse(s);
+        // v_cvt_scalef32_pk_fp4_f32 at scale 1 rounds to nearest, ties to the even code, as ref/kernel.py:48-52
+        // does (8 instead of about 140 VALU operations a lane)
+        auto at = [&](int j) { return fminf(fmaxf(v[q][j >> 2][j & 3] * inv, -6.f), 6.f); };
+        uint32_t out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0, at(0), at(1), 1.0f, 0);
+        out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, at(2), at(3), 1.0f, 1);
+        out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, at(4), at(5), 1.0f, 2);
+        out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, at(6), at(7), 1.0f, 3);
+        if (i >= n8) return;
+        *(uint32_t *)(J.codes + i * 4) = out;
+        if ((threadIdx.x & 3) == 0) ((uint8_t *)J.scales)[i >> 2] = (uint8_t)((__float_as_uint(s) >> 23) & 0xffu);
+    }
 }
 
 // FP8 e4m3 with one fp32 scale per 128x128 block (partial blocks at the edges): s = amax / 448 and
@@ -169,15 +205,16 @@ __global__ __launch_bounds__(256) void k_quant_fp4(const float *__restrict__ w, 
 // together (rows and columns past the edge reload the last ones, which changes no maximum). k % 4 == 0,
 // w 16-byte and codes 4-byte aligned. 7168 x 2048: 73.9 us with two scalar passes over the block by 256
 // threads, 16.1 us (4.6 TB/s) so.
-__global__ __launch_bounds__(512) void k_quant_fp8_b128_x4(const float *__restrict__ w, int rows, int k,
-                                                           uint8_t *__restrict__ codes, float *__restrict__ scales) {
+__global__ __launch_bounds__(512) void k_quant_fp8_b128_x4(QuantJobs jobs) {
     __shared__ float red[8];
-    const int bi = blockIdx.y, bj = blockIdx.x, kb = gridDim.x;
+    uint32_t wg;
+    const QuantJob &J = quant_job(jobs, wg);
+    const int rows = J.rows, k = J.k, kb = (k + 127) >> 7, bi = (int)(wg / kb), bj = (int)(wg % kb);
     const int r0 = bi * 128 + (threadIdx.x >> 5), c0 = bj * 128 + (threadIdx.x & 31) * 4, c = min(c0, k - 4);
     f32x4 v[8];
 #pragma unroll
     for (int i = 0; i < 8; i++)
-        v[i] = __builtin_nontemporal_load((const f32x4 *)(w + (size_t)min(r0 + 16 * i, rows - 1) * k + c));
+        v[i] = __builtin_nontemporal_load((const f32x4 *)(J.w + (size_t)min(r0 + 16 * i, rows - 1) * k + c));
     float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; i++)
@@ -189,12 +226,12 @@ __global__ __launch_bounds__(512) void k_quant_fp8_b128_x4(const float *__restri
 #pragma unroll
     for (int i = 0; i < 8; i++) amax = fmaxf(amax, red[i]);
     const float s = __fdiv_rn(fmaxf(amax, 1e-4f), 448.0f);
-    if (threadIdx.x == 0) scales[(size_t)bi * kb + bj] = s;
+    if (threadIdx.x == 0) ((float *)J.scales)[wg] = s;
     if (c0 >= k) return;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         if (r0 + 16 * i >= rows) return;
-        *(uint32_t *)(codes + (size_t)(r0 + 16 * i) * k + c0) =
+        *(uint32_t *)(J.codes + (size_t)(r0 + 16 * i) * k + c0) =
             e4m3x4_sat(__fdiv_rn(v[i].x, s), __fdiv_rn(v[i].y, s), __fdiv_rn(v[i].z, s), __fdiv_rn(v[i].w, s));
     }
 }
@@ -227,15 +264,17 @@ __global__ __launch_bounds__(256) void k_quant_fp8_b128(const float *w, int rows
 // columns of rows l / 8, l / 8 + 8, ... (rows past the edge reload the last one), so every load reads
 // eight whole 128-byte lines, and the block is read once. w 16-byte, codes 4-byte aligned. 5120 x 2304:
 // 35.6 us with two scalar passes by 256 threads, 12.2 us (4.8 TB/s) so.
-__global__ __launch_bounds__(256) void k_quant_fp8_e8m0_x4(const float *__restrict__ w, int rows, int k,
-                                                           uint8_t *__restrict__ codes, uint8_t *__restrict__ scales) {
-    const int bi = blockIdx.y, bj = blockIdx.x * 4 + (threadIdx.x >> 6), kb = k >> 5;
+__global__ __launch_bounds__(256) void k_quant_fp8_e8m0_x4(QuantJobs jobs) {
+    uint32_t wg;
+    const QuantJob &J = quant_job(jobs, wg);
+    const int rows = J.rows, k = J.k, kb = k >> 5, kw = (kb + 3) >> 2;  // kw: workgroups (four blocks) per block row
+    const int bi = (int)(wg / kw), bj = (int)(wg % kw) * 4 + (threadIdx.x >> 6);
     if (bj >= kb) return;  // the whole wave
     const int lane = threadIdx.x & 63, r0 = bi * 32 + (lane >> 3), c0 = bj * 32 + (lane & 7) * 4;
     f32x4 v[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        v[i] = __builtin_nontemporal_load((const f32x4 *)(w + (size_t)min(r0 + 8 * i, rows - 1) * k + c0));
+        v[i] = __builtin_nontemporal_load((const f32x4 *)(J.w + (size_t)min(r0 + 8 * i, rows - 1) * k + c0));
     float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -243,11 +282,11 @@ __global__ __launch_bounds__(256) void k_quant_fp8_e8m0_x4(const float *__restri
         for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(v[i][j]));
     const float s = pow2_ceil(fmaxf(group_max(amax, kWave), 1e-4f) * (1.0f / 448.0f));
     const float inv = pow2_inverse(s);
-    if (lane == 0) scales[(size_t)bi * kb + bj] = (uint8_t)((__float_as_uint(s) >> 23) & 0xffu);
+    if (lane == 0) ((uint8_t *)J.scales)[(size_t)bi * kb + bj] = (uint8_t)((__float_as_uint(s) >> 23) & 0xffu);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         if (r0 + 8 * i >= rows) return;
-        *(uint32_t *)(codes + (size_t)(r0 + 8 * i) * k + c0) =
+        *(uint32_t *)(J.codes + (size_t)(r0 + 8 * i) * k + c0) =
             e4m3x4_sat(v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv);
     }
 }
@@ -357,6 +396,28 @@ __global__ void k_axpy(float *y, const float *x, float a, int n) {
 
 static inline unsigned grid_for(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
+// Quantizes n <= 3 matrices to one format (ExpertFmt) in one launch; each as its kernel above needs it.
+static hipError_t launch_quant(int fmt, const QuantJob *jobs, int n, hipStream_t st) {
+    QuantJobs all = {};
+    uint32_t wgs = 0;
+    for (int i = 0; i < 3; i++) {
+        if (i >= n) {
+            all.j[i].first = UINT32_MAX;
+            continue;
+        }
+        all.j[i] = jobs[i];
+        all.j[i].first = wgs;
+        const size_t rows = jobs[i].rows, k = jobs[i].k;
+        if (fmt == EXPERT_FP4) wgs += grid_for(rows * (k / 16), 256);
+        else if (fmt == EXPERT_FP8) wgs += (uint32_t)(((rows + 127) / 128) * ((k + 127) / 128));
+        else wgs += (uint32_t)(((rows + 31) / 32) * ((k / 32 + 3) / 4));
+    }
+    if (fmt == EXPERT_FP4) hipLaunchKernelGGL(k_quant_fp4, dim3(wgs), dim3(256), 0, st, all);
+    else if (fmt == EXPERT_FP8) hipLaunchKernelGGL(k_quant_fp8_b128_x4, dim3(wgs), dim3(512), 0, st, all);
+    else hipLaunchKernelGGL(k_quant_fp8_e8m0_x4, dim3(wgs), dim3(256), 0, st, all);
+    return hipGetLastError();
+}
+
 }  // namespace stbl
 
 using namespace stbl;
@@ -438,19 +499,18 @@ int stbl_amd_act_quant(const void *x, int rows, int n, int block, int pow2, void
 int stbl_amd_quant_fp4(void *codes, void *scales, const float *w, int rows, int k, hipStream_t st) {
     if (!codes || !scales || !w || rows <= 0 || k <= 0 || k % 32) return abi_fail(hipErrorInvalidValue, "quant_fp4: need k %% 32 == 0");
     if (!aligned16(codes) || !aligned16(w)) return abi_fail(hipErrorInvalidValue, "quant_fp4: codes and w must be 16-byte aligned");
-    const size_t n8 = (size_t)rows * (k / 8);
-    hipLaunchKernelGGL(k_quant_fp4, dim3(grid_for(n8, 256)), dim3(256), 0, st, w, n8, (uint8_t *)codes,
-                       (uint8_t *)scales);
-    return abi_status(hipGetLastError(), "quant_fp4 launch");
+    const QuantJob job = {w, (uint8_t *)codes, scales, rows, k, 0};
+    return abi_status(launch_quant(EXPERT_FP4, &job, 1, st), "quant_fp4 launch");
 }
 
 int stbl_amd_quant_fp8_b128(void *codes, float *scales, const float *w, int rows, int k, hipStream_t st) {
     if (!codes || !scales || !w || rows <= 0 || k <= 0) return abi_fail(hipErrorInvalidValue, "quant_fp8_b128: bad arguments");
-    const dim3 grid((k + 127) / 128, (rows + 127) / 128);
-    if (k % 4 == 0 && aligned16(w) && ((uintptr_t)codes & 3) == 0)
-        hipLaunchKernelGGL(k_quant_fp8_b128_x4, grid, dim3(512), 0, st, w, rows, k, (uint8_t *)codes, scales);
-    else
-        hipLaunchKernelGGL(k_quant_fp8_b128, grid, dim3(256), 0, st, w, rows, k, (uint8_t *)codes, scales);
+    if (k % 4 == 0 && aligned16(w) && ((uintptr_t)codes & 3) == 0) {
+        const QuantJob job = {w, (uint8_t *)codes, scales, rows, k, 0};
+        return abi_status(launch_quant(EXPERT_FP8, &job, 1, st), "quant_fp8_b128 launch");
+    }
+    hipLaunchKernelGGL(k_quant_fp8_b128, dim3((k + 127) / 128, (rows + 127) / 128), dim3(256), 0, st, w, rows, k,
+                       (uint8_t *)codes, scales);
     return abi_status(hipGetLastError(), "quant_fp8_b128 launch");
 }
 
@@ -458,13 +518,30 @@ int stbl_amd_quant_fp8_b128(void *codes, float *scales, const float *w, int rows
 int stbl_amd_quant_fp8_e8m0(void *codes, void *scales, const float *w, int rows, int k, hipStream_t st) {
     if (!codes || !scales || !w || rows <= 0 || k <= 0 || k % 32)
         return abi_fail(hipErrorInvalidValue, "quant_fp8_e8m0: need k %% 32 == 0");
-    if (aligned16(w) && ((uintptr_t)codes & 3) == 0)
-        hipLaunchKernelGGL(k_quant_fp8_e8m0_x4, dim3((k / 32 + 3) / 4, (rows + 31) / 32), dim3(256), 0, st, w, rows, k,
-                           (uint8_t *)codes, (uint8_t *)scales);
-    else
-        hipLaunchKernelGGL(k_quant_fp8_e8m0, dim3(k / 32, (rows + 31) / 32), dim3(256), 0, st, w, rows, k,
-                           (uint8_t *)codes, (uint8_t *)scales);
+    if (aligned16(w) && ((uintptr_t)codes & 3) == 0) {
+        const QuantJob job = {w, (uint8_t *)codes, scales, rows, k, 0};
+        return abi_status(launch_quant(EXPERT_FP8_E8M0, &job, 1, st), "quant_fp8_e8m0 launch");
+    }
+    hipLaunchKernelGGL(k_quant_fp8_e8m0, dim3(k / 32, (rows + 31) / 32), dim3(256), 0, st, w, rows, k, (uint8_t *)codes,
+                       (uint8_t *)scales);
     return abi_status(hipGetLastError(), "quant_fp8_e8m0 launch");
+}
+
+int stbl_amd_quant_expert(int fmt, void *slot, const float *w_gate, const float *w_up, const float *w_down, int dim,
+                          int inter, hipStream_t st) {
+    const int step = fmt == EXPERT_FP8 ? 4 : 32;
+    if (fmt != EXPERT_FP4 && fmt != EXPERT_FP8 && fmt != EXPERT_FP8_E8M0)
+        return abi_fail(hipErrorInvalidValue, "quant_expert: unknown format %d", fmt);
+    if (!slot || !w_gate || !w_up || !w_down || dim <= 0 || inter <= 0 || dim % step || inter % step)
+        return abi_fail(hipErrorInvalidValue, "quant_expert: need dim and inter %% %d == 0 (dim=%d inter=%d)", step, dim, inter);
+    if (!aligned16(slot) || !aligned16(w_gate) || !aligned16(w_up) || !aligned16(w_down))
+        return abi_fail(hipErrorInvalidValue, "quant_expert: slot and weights must be 16-byte aligned");
+    const ExpertLayout L = expert_layout(fmt, dim, inter);
+    uint8_t *base = (uint8_t *)slot;
+    const QuantJob jobs[3] = {{w_gate, base + L.off[0], base + L.off[1], inter, dim, 0},
+                              {w_up, base + L.off[2], base + L.off[3], inter, dim, 0},
+                              {w_down, base + L.off[4], base + L.off[5], dim, inter, 0}};
+    return abi_status(launch_quant(fmt, jobs, 3, st), "quant_expert launch");
 }
 
 int stbl_amd_dequant_fp4(float *out, const void *codes, const void *scales, int rows, int k, hipStream_t st) {

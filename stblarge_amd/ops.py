@@ -362,8 +362,35 @@ def pack_slot(parts, fmt, dim, inter, out=None):
     return slot
 
 
+def _quant_into_slot(w_gate, w_up, w_down, fmt, out):
+    """Whether stbl_amd_quant_expert takes these weights and this slot as they are: 16-byte aligned fp32
+    device matrices of an expert's three shapes, and a contiguous slot on their device that shares no
+    memory with them. Anything else (a host slot, a strided one, a wrong shape) goes matrix by matrix,
+    which copies, or raises."""
+    ws = (w_gate, w_up, w_down)
+    for w in ws:
+        _need(w, torch.float32, "w", 2)
+    inter, dim = w_gate.shape
+    step = {FP4: 32, FP8: 4, FP8_E8M0: 32}[fmt]
+    if (w_up.shape != w_gate.shape or w_down.shape != (dim, inter) or not inter or not dim or dim % step or inter % step
+            or any(w.data_ptr() % 16 or w.device != w_gate.device for w in ws)):
+        return False
+    if out is None:
+        return True
+    return (out.is_cuda and out.device == w_gate.device and out.dtype == torch.uint8 and out.dim() == 1
+            and out.is_contiguous() and out.data_ptr() % 16 == 0 and out.numel() >= expert_layout(fmt, dim, inter)[0]
+            and all(w.untyped_storage().data_ptr() != out.untyped_storage().data_ptr() for w in ws))
+
+
 def quant_expert(w_gate, w_up, w_down, fmt, out=None):
     """Quantize fp32 gate/up [inter, dim] and down [dim, inter] on the device into one slot."""
+    if _quant_into_slot(w_gate, w_up, w_down, fmt, out):
+        inter, dim = w_gate.shape
+        nbytes, _ = expert_layout(fmt, dim, inter)
+        slot = out if out is not None else torch.zeros(nbytes, dtype=torch.uint8, device=w_gate.device)
+        _lib.check(_lib.load().stbl_amd_quant_expert(fmt, _ptr(slot), _ptr(w_gate), _ptr(w_up), _ptr(w_down), dim, inter,
+                                                     _stream()), "quant_expert")
+        return slot
     q = {FP4: quant_fp4, FP8: quant_fp8_b128, FP8_E8M0: quant_fp8_e8m0}[fmt]
     parts = []
     for w in (w_gate, w_up, w_down):

@@ -62,6 +62,22 @@ def test_quant_fp4_matches_oracle(gpu, rows, k):
     assert np.array_equal(np_(scales), os_)
 
 
+def test_quant_fp4_ties_and_neighbours(gpu):
+    # every multiple of 1/64 of the scale up to 6 with both signs, each next to its fp32 neighbours (so
+    # all ties and both sides of them), under scales 2^-20 .. 2^20, with NaN and infinities
+    grid = np.arange(-384, 385, dtype=np.float32) / 64
+    vals = np.concatenate([grid, np.nextafter(grid, np.float32(9)), np.nextafter(grid, np.float32(-9)), [-0.0, 0.0]])
+    vals = np.resize(vals.astype(np.float32), (75, 31))
+    rows = np.concatenate([np.full((75, 1), 6, np.float32), vals], 1)  # the group's maximum is 6: its scale 1
+    w = np.concatenate([rows * np.float32(2.0 ** e) for e in range(-20, 21, 5)], 0)
+    w[0, 3], w[1, 4], w[2, 5] = np.nan, np.inf, -np.inf
+    codes, scales = ops.quant_fp4(torch.from_numpy(w).to(gpu))
+    with np.errstate(invalid="ignore"):
+        oc, os_ = oracle.quant_fp4(w)
+    assert np.array_equal(np_(scales), os_)
+    assert np.array_equal(np_(codes), oc)
+
+
 @pytest.mark.parametrize("rows,k", [(130, 260), (2048, 7168), (7168, 2048)])
 def test_quant_fp8_b128_matches_oracle(gpu, rows, k):
     w = data.weight(rows, k, seed=3 * rows + k)
@@ -111,6 +127,33 @@ def test_quant_fp8_e8m0_edges_and_alignment(gpu, rows, k, shift):
     codes, scales = ops.quant_fp8_e8m0(wg)
     oc, os_ = oracle.quant_fp8_e8m0_b32(w.numpy())
     assert np.array_equal(np_(codes), oc) and np.array_equal(np_(scales), os_)
+
+
+@pytest.mark.parametrize("fmt,dim,inter", [(0, 96, 32), (0, 7168, 2048), (1, 260, 132), (1, 7168, 2048), (1, 130, 66),
+                                           (2, 160, 96), (2, 5120, 2304)])
+@pytest.mark.parametrize("where", ["new", "given", "host", "shared"])
+def test_quant_expert_equals_its_matrices(gpu, fmt, dim, inter, where):
+    # the one-launch form and the one that copies matrix by matrix (dims the launch does not take, a slot
+    # in host memory, a slot sharing the weights' memory) write what the quantizers give for each matrix,
+    # and nothing between the parts
+    ws = [data.weight(r, k, seed=r + k + i, device=gpu) for i, (r, k) in enumerate(((inter, dim), (inter, dim), (dim, inter)))]
+    q = {0: ops.quant_fp4, 1: ops.quant_fp8_b128, 2: ops.quant_fp8_e8m0}[fmt]
+    parts = [t for w in ws for t in q(w)]
+    n, _ = ops.expert_layout(fmt, dim, inter)
+    fill = 0 if where == "new" else 77
+    want = ops.pack_slot(parts, fmt, dim, inter, out=torch.full((n,), fill, dtype=torch.uint8, device=gpu))
+    out = None
+    if where == "given":
+        out = torch.full((n + 256,), fill, dtype=torch.uint8, device=gpu)[256:]
+    elif where == "host":
+        out = torch.full((n,), fill, dtype=torch.uint8)
+    elif where == "shared":
+        buf = torch.empty(n + ws[2].numel() * 4, dtype=torch.uint8, device=gpu)  # n is a multiple of 256
+        ws[2] = buf[n:].view(torch.float32).view(ws[2].shape).copy_(ws[2])
+        out = buf[:n].fill_(fill)
+    got = ops.quant_expert(*ws, fmt, out=out)
+    assert out is None or got is out
+    assert np.array_equal(np_(got), np_(want))
 
 
 @pytest.mark.parametrize("block,pow2", [(32, True), (128, True), (128, False)])
