@@ -239,9 +239,9 @@ int stbl_amd_gemm(int fmt, void *y, const void *codes, const void *scales, const
 int stbl_amd_gemm_q(int fmt, void *y, const void *codes, const void *scales, const void *aq, const void *as, int m,
                     int n, int k, int act_block, int y_f32, void *work, hipStream_t st);
 
-/* Scratch bytes for stbl_amd_gemm and stbl_amd_gemm_q with m activation rows (n, k as in the call);
- * a workspace of that size also serves every call with fewer rows. The same bytes serve the packed
- * variants below. */
+/* Scratch bytes for stbl_amd_gemm, stbl_amd_gemm_q and the _rows variants with m activation rows (n, k as
+ * in the call); a workspace of that size also serves every call with fewer rows. The same bytes serve
+ * the packed variants below. */
 uint64_t stbl_amd_gemm_work_bytes(int m, int n, int k);
 
 /* No counterpart in the reference: for callers whose GEMM weights are static (an expert's matrices
@@ -257,6 +257,15 @@ int stbl_amd_gemm_q_packed(int fmt, void *y, const void *packed, const void *sca
                            int m, int n, int k, int act_block, int y_f32, void *work, hipStream_t st);
 int stbl_amd_gemm_packed(int fmt, void *y, const void *packed, const void *scales, const void *x, int m, int n, int k,
                          int act_block, int y_f32, void *work, hipStream_t st);
+
+/* stbl_amd_gemm / stbl_amd_gemm_q (packed != 0: on weight codes from stbl_amd_gemm_pack) on up to 8192 rows
+ * in one call: the weights pass through the GPU once per 64 or 128 columns, not once per 64 rows. Every
+ * full 64 rows' results are those of a call on them alone, bit for bit; a shorter last part is summed
+ * as the others are. The rows of ref/kernel.py:85-102's a, whose number is not limited. */
+int stbl_amd_gemm_rows(int fmt, int packed, void *y, const void *codes, const void *scales, const void *x, int m, int n,
+                       int k, int act_block, int y_f32, void *work, hipStream_t st);
+int stbl_amd_gemm_q_rows(int fmt, int packed, void *y, const void *codes, const void *scales, const void *aq, const void *as,
+                         int m, int n, int k, int act_block, int y_f32, void *work, hipStream_t st);
 
 /* act_quant(x, block, "ue8m0") (ref/kernel.py:35-45) as the GEMM consumes it: x bf16 [rows][k] ->
  * e4m3 codes [rows][k] and E8M0 scale bytes [rows][k/block]; block 32 or 128. Non-finite values as

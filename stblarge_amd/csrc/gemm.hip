@@ -1,4 +1,4 @@
-// Multi-token expert GEMM on CDNA4 scaled MFMA: Y[m][n] = sum_k Aq[m][k] * Wdeq[n][k], M <= 64.
+// Multi-token expert GEMM on CDNA4 scaled MFMA: Y[m][n] = sum_k Aq[m][k] * Wdeq[n][k].
 //
 // Reference: fp8_gemm / fp4_gemm of ref/kernel.py:85-102 with M = 64 rows of activations:
 //   A = act_quant(X, block, "ue8m0") (e4m3 codes, power-of-two scales per `block` along K),
@@ -8,20 +8,17 @@
 //   k_act_quant_e4m3  X bf16 -> e4m3 codes + E8M0 scale bytes, one 16-lane group per block of 128
 //                     (or 4 lanes per block of 32); the e4m3 rounding uses v_cvt_pk_fp8_f32, which
 //                     equals the round-to-nearest-even encoder bit for bit on every bf16 input;
-//                     k_act_quant_e4m3_ops the same codes in MFMA operand order, for k_gemm_one;
-//   k_gemm            v_mfma_scale_f32_16x16x128_f8f6f4 with A = e4m3 activations and B = the e4m3 or
+//                     k_act_quant_e4m3_ops the same codes in MFMA operand order;
+//   k_gemm, ...       v_mfma_scale_f32_16x16x128_f8f6f4 with A = e4m3 activations and B = the e4m3 or
 //                     e2m1 weights. The activation scales (powers of two) and the FP4 weight scales
 //                     (E8M0) are the MFMA's own per-32 scale operands, so the hardware applies them
 //                     exactly; the FP8 weights' fp32 block scale multiplies each 128-K step's product
-//                     in fp32. Split K: each workgroup writes its K slice's partial tile and
-//                     k_gemm_reduce adds the slices in order (the kernel boundary is the
-//                     synchronization point); stbl_amd_gemm_q takes already quantized activations,
-//                     stbl_amd_gemm quantizes X first (one more launch).
-//   k_gemm_one        the same products in one launch over all of K, for m > 32 and K % 512 == 0
-//                     (the configurations' shapes): small tiles, half-line-balanced operand loads
-//                     and scales loaded four steps at a time;
+//                     in fp32. gemm_plan chooses between them: k_gemm_one (the configurations' shapes)
+//                     and k_gemm_waves, one launch over all of K by waves that each take a part of it;
+//                     k_gemm and k_gemm_reduce, split K; k_gemm_tile, many rows through LDS, on operands
+//                     laid out by k_gemm_prep;
 //   k_gemm_pack       the weight codes rearranged once into MFMA operand order (WOPS below), which
-//                     both GEMM kernels then read as one contiguous kilobyte per wave load.
+//                     every kernel reads to the same results bit for bit.
 // Operand layout of the 16x16x128 f8f6f4 MFMA (probed on gfx950): lane l = r + 16 g holds row r of A
 // (column r of B); e4m3 operands hold K bytes [16g, 16g+16) and [64+16g, 64+16g+16) of the 128-K
 // step, e2m1 operands K elements [32g, 32g+32) (low nibble first); the lane's E8M0 scale covers K
@@ -35,6 +32,19 @@ namespace stbl {
 
 constexpr int kGemmMaxM = 64;
 constexpr int kGemmMaxN = 1 << 20;
+constexpr int kGemmMaxRows = 8192;  // of stbl_amd_gemm_rows
+
+// ---- operand order --------------------------------------------------------------------------------
+
+// WOPS: weights in MFMA operand order. Per group G of 16 columns and 128-K step s, the 64 lanes'
+// 16-byte operand pieces lie in lane order: FP4 one kilobyte, lane r + 16 g holding bytes [16g,
+// 16g + 16) of column 16 G + r's 64-byte step; FP8 two kilobytes, the first holding bytes [16g, 16g
+// + 16) and the second [64 + 16g, 64 + 16g + 16) of the column's 128-byte step. Blocks run over the
+// steps of a group, then over the groups, so a column group's weights stay one contiguous run and
+// the packed array has the size of the codes. Byte offset of the block (G, s):
+__device__ __forceinline__ size_t ops_block(int G, int s, int KS, bool fp4) {
+    return ((size_t)G * KS + s) * (fp4 ? 1024 : 2048);
+}
 
 // ---- activation quantization --------------------------------------------------------------------
 
@@ -73,25 +83,9 @@ __global__ __launch_bounds__(256) void k_act_quant_e4m3(const uint16_t *__restri
     if ((threadIdx.x & (lanes - 1)) == 0) scales[(size_t)i * 8 / block] = (uint8_t)((__float_as_uint(s) >> 23) & 0xffu);
 }
 
-// The same quantization written in MFMA operand order (stbl_amd_gemm's one-launch plans, whose
-// operand loads then each read one contiguous kilobyte): per group of 16 rows and 128-K step, 2 KB,
-// in which the 16 bytes lane l = r + 16 g of an operand load takes (row r, bytes [16 g, 16 g + 16) of
-// the step's first 64, then of its second 64) sit at l * 16 of the first, then of the second
-// kilobyte. One wave per group and step: lane l reads row r's 16 values at [16 g, 16 g + 16) of each
-// half of the step and stores their codes as that piece, so each store instruction writes a
-// contiguous kilobyte (measured against 8-byte stores scattered into the same layout by
-// k_act_quant_e4m3's lanes: full FP4 GEMM at 2048x7168 10.14 -> 9.75 us, FP8 12.83 -> 12.43). A block's amax
-// comes from the lanes of the same row: all four for a 128-block (xor 16, 32), the pair g, g ^ 1 of
-// one half for a 32-block (block 2 h + g / 2 of the step). Rows past m (up to the group's 16) store
-// zero codes and no scales. The codes and scales of rows < m are k_act_quant_e4m3's, byte for byte.
-__global__ __launch_bounds__(64) void k_act_quant_e4m3_ops(const uint16_t *__restrict__ x, int m, int k, int block,
-                                                          uint8_t *__restrict__ codes, uint8_t *__restrict__ scales) {
-    const int ks = k >> 7;
-    const int w = blockIdx.x, mg = w / ks, s = w % ks;  // grid: ceil(m / 16) * ks waves
-    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
-    const int row = mg * 16 + r;
-    const bool ok = row < m;
-    const uint16_t *src = x + (size_t)(ok ? row : 0) * k + (size_t)s * 128 + 16 * g;
+// The quantization of one operand lane: src points at its row's 16 values of the step's first half, 16 g
+// on; q gets the codes of both halves, sb their scale bytes.
+__device__ __forceinline__ void quant_ops(const uint16_t *src, int block, u32x4 (&out)[2], uint32_t (&sb)[2]) {
     float f[2][16];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -119,7 +113,6 @@ __global__ __launch_bounds__(64) void k_act_quant_e4m3_ops(const uint16_t *__res
         // 1/sc, exact, or 0 for sc = +Inf, as in k_act_quant_e4m3
         const float inv =
             __builtin_isinf(sc) ? 0.f : __uint_as_float((uint32_t)(254 - ((__float_as_uint(sc) >> 23) & 0xffu)) << 23);
-        u32x4 out;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             // x / sc is exact (sc is a power of two); the clamp is ref/kernel.py:41's
@@ -128,26 +121,42 @@ __global__ __launch_bounds__(64) void k_act_quant_e4m3_ops(const uint16_t *__res
             for (int e = 0; e < 4; e++) q[e] = fminf(fmaxf(f[h][4 * j + e] * inv, -448.f), 448.f);
             int p = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
             p = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], p, true);
-            out[j] = ok ? (uint32_t)p : 0u;
+            out[h][j] = (uint32_t)p;
         }
-        *(u32x4 *)(codes + (((size_t)mg * ks + s) * 2 + h) * 1024 + lane * 16) = out;
-        const uint8_t sbyte = (uint8_t)((__float_as_uint(sc) >> 23) & 0xffu);
-        if (ok && block == 128 && h == 0 && g == 0) scales[(size_t)row * ks + s] = sbyte;
-        if (ok && block == 32 && (g & 1) == 0) scales[(size_t)row * (k >> 5) + 4 * s + 2 * h + (g >> 1)] = sbyte;
+        sb[h] = (__float_as_uint(sc) >> 23) & 0xffu;
+    }
+}
+
+// The same quantization written in MFMA operand order (stbl_amd_gemm's one-launch plans, whose
+// operand loads then each read one contiguous kilobyte): per group of 16 rows and 128-K step, 2 KB,
+// in which the 16 bytes lane l = r + 16 g of an operand load takes (row r, bytes [16 g, 16 g + 16) of
+// the step's first 64, then of its second 64) sit at l * 16 of the first, then of the second
+// kilobyte. One wave per group and step: lane l reads row r's 16 values at [16 g, 16 g + 16) of each
+// half of the step and stores their codes as that piece, so each store instruction writes a
+// contiguous kilobyte (measured against 8-byte stores scattered into the same layout by
+// k_act_quant_e4m3's lanes: full FP4 GEMM at 2048x7168 10.14 -> 9.75 us, FP8 12.83 -> 12.43). A block's amax
+// comes from the lanes of the same row: all four for a 128-block (xor 16, 32), the pair g, g ^ 1 of
+// one half for a 32-block (block 2 h + g / 2 of the step). Rows past m (up to the group's 16) store
+// zero codes and no scales. The codes and scales of rows < m are k_act_quant_e4m3's, byte for byte.
+__global__ __launch_bounds__(64) void k_act_quant_e4m3_ops(const uint16_t *__restrict__ x, int m, int k, int block,
+                                                          uint8_t *__restrict__ codes, uint8_t *__restrict__ scales) {
+    const int ks = k >> 7;
+    const int w = blockIdx.x, mg = w / ks, s = w % ks;  // grid: ceil(m / 16) * ks waves
+    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
+    const int row = mg * 16 + r;
+    const bool ok = row < m;
+    u32x4 q[2];
+    uint32_t sb[2];
+    quant_ops(x + (size_t)(ok ? row : 0) * k + (size_t)s * 128 + 16 * g, block, q, sb);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        *(u32x4 *)(codes + ops_block(mg, s, ks, false) + 1024 * h + lane * 16) = ok ? q[h] : u32x4{0, 0, 0, 0};
+        if (ok && block == 128 && h == 0 && g == 0) scales[(size_t)row * ks + s] = (uint8_t)sb[0];
+        if (ok && block == 32 && (g & 1) == 0) scales[(size_t)row * (k >> 5) + 4 * s + 2 * h + (g >> 1)] = (uint8_t)sb[h];
     }
 }
 
 // ---- GEMM ---------------------------------------------------------------------------------------
-
-// WOPS: weights in MFMA operand order. Per group G of 16 columns and 128-K step s, the 64 lanes'
-// 16-byte operand pieces lie in lane order: FP4 one kilobyte, lane r + 16 g holding bytes [16g,
-// 16g + 16) of column 16 G + r's 64-byte step; FP8 two kilobytes, the first holding bytes [16g, 16g
-// + 16) and the second [64 + 16g, 64 + 16g + 16) of the column's 128-byte step. Blocks run over the
-// steps of a group, then over the groups, so a column group's weights stay one contiguous run and
-// the packed array has the size of the codes. Byte offset of the block (G, s):
-__device__ __forceinline__ size_t ops_block(int G, int s, int KS, bool fp4) {
-    return ((size_t)G * KS + s) * (fp4 ? 1024 : 2048);
-}
 
 // codes [n][k / 2] (FP4) or [n][k] (FP8), n % 16 == 0, k % 128 == 0 -> the same codes in operand
 // order. Thread t moves the 16-byte piece t of the packed array.
@@ -169,34 +178,30 @@ __global__ __launch_bounds__(256) void k_gemm_pack(const uint8_t *__restrict__ c
     *(u32x4 *)(packed + 16 * t) = *(const u32x4 *)(codes + src);
 }
 
-// One workgroup owns a 16 MT x 16 NT output tile (MT m-tiles x NT n-tiles of 16 x 16, rows m0 ..) and
-// a slice of up to NW * SW 128-K steps; wave w takes SW consecutive steps of the slice and accumulates
-// its MT * NT tiles in registers, loading its activations and weights straight from global memory
-// (no operand is shared between waves, so nothing is staged through LDS). All loads of a wave are
-// issued before its first MFMA, from addresses clamped into the buffers; a step past the slice gets
-// zero operands instead of a branch. The waves' tiles are summed through LDS in wave order. With one
-// slice the workgroup writes Y; otherwise it writes its slice's partial tile and k_gemm_reduce adds
-// the slices in order. (Summing the slices in the last workgroup to finish needs an agent-scope
-// release/acquire per workgroup, which writes back and invalidates the XCD's L2 each time: measured
-// at about 4x the whole GEMM, so the kernel boundary is the synchronization point.) The workgroup
-// order is gemm_plan's. A rows are lda bytes apart. Partial tiles and the LDS sum hold f32x4
-// q = t * 64 + lane with t = m-tile * NT + n-tile.
-template <bool FP4W, int MT, int NT, int NW, int SW, bool WOPS>
+// One workgroup owns a 16 MT x 16 NT output tile (MT m-tiles x NT n-tiles of 16 x 16) and a slice of up
+// to NW 128-K steps; wave w takes step w of the slice for all MT * NT tiles, loading its activations and
+// weights straight from global memory (no operand is shared between waves, so nothing is staged
+// through LDS), from addresses clamped into the buffers; a step past the slice gets zero operands
+// instead of a branch. The waves' tiles are summed through LDS in wave order, the workgroup writes its
+// slice's partial tile, and k_gemm_reduce adds the slices in order. (Summing the slices in the last
+// workgroup to finish needs an agent-scope release/acquire per workgroup, which writes back and
+// invalidates the XCD's L2 each time: measured at about 4x the whole GEMM, so the kernel boundary is
+// the synchronization point.) A rows are K bytes apart. Partial tiles and the LDS sum hold f32x4 q = t *
+// 64 + lane with t = m-tile * NT + n-tile.
+template <bool FP4W, int MT, int NT, int NW, bool WOPS>
 __global__ __launch_bounds__(NW * 64) void k_gemm(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
                                                   const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,
-                                                  f32x4 *__restrict__ part, void *__restrict__ y, int y_f32, int M,
-                                                  int N, int K, int lda, int act_shift, int ntiles, int mgroups,
-                                                  int slices, int steps_wg) {
+                                                  f32x4 *__restrict__ part, int M, int N, int K, int act_shift,
+                                                  int ntiles, int slices, int steps_wg) {
+    constexpr int SW = 1;
     constexpr int kTileVecs = MT * NT * 64;
     constexpr int kThreads = NW * 64;
     __shared__ f32x4 red[NW * kTileVecs];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
-    const int u = blockIdx.x % (ntiles * mgroups), slice = blockIdx.x / (ntiles * mgroups);
-    const int tile = u % ntiles, m0 = (u / ntiles) * 16 * MT;
+    const int tile = blockIdx.x % ntiles, slice = blockIdx.x / ntiles;
     const int n0 = tile * 16 * NT, KS = K >> 7;
-    const int wsteps = (steps_wg + NW - 1) / NW;
-    const int s0 = slice * steps_wg + wave * wsteps;
-    const int nst = max(0, min(wsteps, min(KS, (slice + 1) * steps_wg) - s0));  // wave-uniform
+    const int s0 = slice * steps_wg + wave;
+    const int nst = max(0, min(1, min(KS, (slice + 1) * steps_wg) - s0));  // wave-uniform
 
     // 1. loads: lane (r, g) holds, per step, rows 16 mt + r of A and columns n0 + 16 nt + r of W
     u32x4 av[SW][MT][2];
@@ -209,8 +214,8 @@ __global__ __launch_bounds__(NW * 64) void k_gemm(const uint8_t *__restrict__ wc
         const size_t kb = (size_t)(s < nst ? s0 + s : 0) * 128;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-            const int m = min(m0 + 16 * mt + r, M - 1);
-            const uint8_t *row = aq + (size_t)m * lda + kb;
+            const int m = min(16 * mt + r, M - 1);
+            const uint8_t *row = aq + (size_t)m * K + kb;
             av[s][mt][0] = *(const u32x4 *)(row + 16 * g);
             av[s][mt][1] = *(const u32x4 *)(row + 64 + 16 * g);
             asc[s][mt] = as_[(size_t)m * (K >> act_shift) + ((kb + 32 * g) >> act_shift)];
@@ -286,21 +291,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm(const uint8_t *__restrict__ wc
         f32x4 v = red[q];
 #pragma unroll
         for (int w = 1; w < NW; w++) v += red[w * kTileVecs + q];
-        if (slices > 1) {  // (split K only with mgroups == 1: u is the tile)
-            part[((size_t)u * slices + slice) * kTileVecs + q] = v;
-            continue;
-        }
-        // Y: element e of v is row 16 mt + 4 g' + e, column n0 + 16 nt + r' of the lane q % 64
-        const int t = q >> 6, ql = q & 63, mt = t / NT, nt = t % NT;
-        const int n = n0 + 16 * nt + (ql & 15);
-        if (n >= N) continue;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int m = m0 + 16 * mt + 4 * (ql >> 4) + e;
-            if (m >= M) continue;
-            if (y_f32) ((float *)y)[(size_t)m * N + n] = v[e];
-            else ((uint16_t *)y)[(size_t)m * N + n] = f32_to_bf16_bits(v[e]);
-        }
+        part[((size_t)tile * slices + slice) * kTileVecs + q] = v;
     }
 }
 
@@ -527,165 +518,724 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_one(const uint8_t *__restrict_
     }
 }
 
-// Tile shape and split of K, chosen per shape (each choice measured fastest for its shape):
-//   variant 4, k_gemm_one with 32 x 64 tiles on 4 waves of 4 steps, when K % 512 == 0, K <= 2048, m > 32
-//     and the tiles give >= 192 workgroups (7168 x 2048: 9.0 -> 6.6 us against variant 2);
-//   variant 3, k_gemm_one with 16 x 32 tiles on up to 8 waves of 8 steps (FP4 weights: 8.2 -> 7.9 us
+// GEMM of many rows: a workgroup of WR x WC waves owns a BM x BN output tile over all of K, each wave a
+// BM / WR x BN / WC part. A 128-K step's A rows, W columns and scale dwords go to LDS once for the
+// workgroup, by loads that write LDS directly (they hold no registers), S - 1 steps ahead of their use,
+// and a wave reads the next step's operands from LDS while its products of this one run. A and packed W
+// lie in LDS in operand order, row-major W with its 16-byte pieces permuted by the column, so that operand
+// reads hit every bank once.
+// The sum runs as a call of up to 64 rows at the same n and k sums (gemm_sum): steps in groups of `group`;
+// within a group CHAIN keeps one running sum (FP4: in the MFMA's accumulator, FP8: an FMA per element and
+// step), otherwise each step's product is rounded and added; then the groups' sums are added in order.
+// Measured (FP4 / FP8, with k_gemm_prep, us) against 64 rows a launch: 1024 x 7168 x 2048 84.6 / 107.2 -> 31.1 /
+// 33.9, 300 x 2048 x 7168 38.5 / 48.0 -> 22.6 / 26.8. What bounds it: of 23.6 us at 1024 x 7168 x 2048 FP4, 17.5
+// are the products alone (7.5 at the matrix cores' rate; a 64 x 128 tile's 16 steps are short against its
+// start and end), 9.5 the loads and LDS reads alone.
+// 64 lanes x 16 (4) bytes at base + off -> LDS at lds + 16 (4) x lane. The LDS address goes through M0,
+// which is left as it was. Counted by vmcnt (wait_vmem): the compiler's builtin for this load makes it
+// wait for every such load before any LDS read that could alias, which is each step's.
+__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t *base, uint32_t off) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "memory");
+}
+__device__ __forceinline__ void lds_dma4(uint32_t lds, const uint8_t *base, uint32_t off) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_lds_vmem() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+template <bool FP4W, int BM, int BN, int WR, int WC, int S, bool CHAIN, bool WOPS>
+__global__ __launch_bounds__(WR *WC * 64, BM / WR * BN / WC >= 4096 ? 1 : 2) void k_gemm_tile(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
+                                                      const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as4,
+                                                      const uint8_t *__restrict__ ws4, void *__restrict__ y, int y_f32,
+                                                      int M, int N, int K, int group, int mtiles, int ntiles) {
+    constexpr int W = WR * WC, WM = BM / WR, WN = BN / WC, MT = WM / 16, NT = WN / 16;
+    constexpr int kStepB = FP4W ? 64 : 128;                     // bytes of a W column per step
+    constexpr int kA = BM * 128, kB = BN * kStepB;              // LDS bytes per step
+    constexpr int kSA = BM * 4, kSB = FP4W ? BN * 4 : 0, kStage = kA + kB + kSA + kSB;
+    constexpr int kPieces = (kA + kB) / 1024, PV = (kPieces + W - 1) / W;  // kilobyte loads, and per wave
+    constexpr int SV = (BM + (FP4W ? BN : 0)) / 64;             // scale loads per workgroup (64 dwords each)
+    constexpr int SW = (SV + W - 1) / W;                        // ... per wave (the last waves repeat one)
+    constexpr int kLoads = PV + SW;  // the last waves repeat a load where they do not divide
+    static_assert(BM % 64 == 0 && BN % 64 == 0 && (S - 1) * kLoads < 64, "tile");
+    extern __shared__ __align__(1024) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WC, wn = wave % WC;
+    const int KS = K >> 7;
+    // workgroup b runs on XCD b % 8: each XCD gets a contiguous run of tiles, row tiles innermost, so
+    // its L2 holds its columns' weights while every row tile passes over them
+    const int total = mtiles * ntiles, xcd = blockIdx.x & 7, per = total >> 3, rem = total & 7;
+    const int t0 = xcd * per + min(xcd, rem) + (int)(blockIdx.x >> 3);
+    const int m0 = (t0 % mtiles) * BM, n0 = (t0 / mtiles) * BN;
+
+    // this lane's 32-bit offsets from the tile's uniform bases; rows past the edge reload the last
+    const int mg = (M + 15) >> 4;
+    const uint8_t *pa = aq + ops_block(m0 >> 4, 0, KS, false);
+    const uint8_t *pb = wc + (WOPS ? ops_block(n0 >> 4, 0, KS, FP4W) : (size_t)n0 * (FP4W ? K >> 1 : K));
+    uint32_t off[PV], os[SW];
+#pragma unroll
+    for (int i = 0; i < PV; i++) {
+        const int q = min(i * W + wave, kPieces - 1), u = (q - kA / 1024) * 64 + lane;
+        if (q < kA / 1024) {
+            off[i] = (uint32_t)ops_block(min(q >> 1, mg - 1 - (m0 >> 4)), 0, KS, false) + (uint32_t)((q & 1) * 1024 + lane * 16);
+        } else if constexpr (WOPS) {
+            const int blk = FP4W ? u >> 6 : u >> 7;
+            off[i] = (uint32_t)ops_block(min(blk, (N >> 4) - 1 - (n0 >> 4)), 0, KS, FP4W) + (uint32_t)(FP4W ? u & 63 : u & 127) * 16;
+        } else if constexpr (FP4W) {
+            const int col = u >> 2;
+            off[i] = (uint32_t)min(col, N - 1 - n0) * (uint32_t)(K >> 1) + (uint32_t)(((u & 3) ^ ((col >> 1) & 3)) * 16);
+        } else {
+            const int col = u >> 3;
+            off[i] = (uint32_t)min(col, N - 1 - n0) * (uint32_t)K + (uint32_t)(((u & 7) ^ (col & 7)) * 16);
+        }
+    }
+    constexpr uint32_t kAdvB = WOPS ? (FP4W ? 1024 : 2048) : kStepB;
+#pragma unroll
+    for (int i = 0; i < SW; i++) {
+        const int q = min(wave * SW + i, SV - 1);  // 64 rows of A, then of W
+        const bool a = q < BM / 64;
+        const int row = a ? m0 + q * 64 + lane : n0 + (q - BM / 64) * 64 + lane;
+        os[i] = 4u * (uint32_t)min(row, (a ? M : N) - 1);
+    }
+    const int spa = 4 * M, spw = 4 * N;  // bytes per step of the scales
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    auto issue = [&](int s, int st) {
+        const uint32_t base = lds0 + st * kStage;
+#pragma unroll
+        for (int i = 0; i < PV; i++) {
+            const int q = min(i * W + wave, kPieces - 1);
+            lds_dma16(base + q * 1024, q < kA / 1024 ? pa + (size_t)s * 2048 : pb + (size_t)s * kAdvB, off[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < SW; i++) {
+            const int q = min(wave * SW + i, SV - 1);
+            lds_dma4(base + kA + kB + q * 256, q < BM / 64 ? as4 + (size_t)s * spa : ws4 + (size_t)s * spw, os[i]);
+        }
+    };
+    const int a0 = wm * MT * 2048 + lane * 16, a1 = a0 + 1024;
+    int b0, b1 = 0;
+    if constexpr (WOPS) {
+        b0 = kA + wn * NT * (FP4W ? 1024 : 2048) + lane * 16, b1 = b0 + 1024;
+    } else if constexpr (FP4W) {
+        b0 = kA + (wn * WN + r) * 64 + ((g ^ ((r >> 1) & 3)) << 4);
+    } else {
+        const int lb = kA + (wn * WN + r) * 128;
+        b0 = lb + ((g ^ (r & 7)) << 4), b1 = lb + (((g + 4) ^ (r & 7)) << 4);
+    }
+    const int sa0 = kA + kB + (wm * WM + r) * 4 + g, sb0 = kA + kB + kSA + (wn * WN + r) * 4 + g;
+    const float *wsc = (const float *)ws + (size_t)(n0 >> 7) * KS;
+
+    f32x4 acc[MT][NT], tot[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT * NT; i++) acc[i / NT][i % NT] = tot[i / NT][i % NT] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Frag {  // a wave's operands of one step
+        i32x8 a[MT], b[NT];
+        int sa[MT], sb[NT];
+    };
+    auto read = [&](Frag &F, int st) {
+        const uint8_t *T = smem + st * kStage;
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const u32x4 x0 = *(const u32x4 *)(T + b0 + nt * (FP4W ? 1024 : 2048));
+            u32x4 x1 = {0, 0, 0, 0};
+            if constexpr (!FP4W) x1 = *(const u32x4 *)(T + b1 + nt * 2048);
+            F.b[nt] = i32x8{(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
+            F.sb[nt] = FP4W ? T[sb0 + nt * 64] : 127;
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const u32x4 x0 = *(const u32x4 *)(T + a0 + mt * 2048), x1 = *(const u32x4 *)(T + a1 + mt * 2048);
+            F.a[mt] = i32x8{(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
+            F.sa[mt] = T[sa0 + mt * 64];
+        }
+    };
+    float sw = FP4W ? 0.f : wsc[0];
+    int left = group, st = 0;
+    // Step s, its operands in F; reads step s + 1's into G. This wave's loads of step s + 1 are in LDS once at
+    // most those of the S - 2 later steps are outstanding; after the barrier everybody's are, and everybody
+    // has step s in registers, so the loads of step s + S (past the last step: of it again, unread) may
+    // fill its stage.
+    auto step = [&](Frag &F, Frag &G, int s) {
+        wait_lds_vmem<(S - 2) * kLoads>();
+        __builtin_amdgcn_s_barrier();
+        const int nx = st + 1 == S ? 0 : st + 1;
+        read(G, nx);
+        issue(min(s + S, KS - 1), st);
+        st = nx;
+        const float sw_next = FP4W ? 0.f : wsc[min(s + 1, KS - 1)];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                constexpr int bf = FP4W ? 4 : 0;
+                const f32x4 c = CHAIN && FP4W ? acc[mt][nt] : f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(F.a[mt], F.b[nt], c, 0, bf, 0, F.sa[mt], 0, F.sb[nt]);
+                if constexpr (CHAIN && FP4W) {
+                    acc[mt][nt] = d;
+                } else if constexpr (CHAIN) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[mt][nt][e] = fmaf(sw, d[e], acc[mt][nt][e]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[mt][nt][e] += FP4W ? d[e] : fmaf(sw, d[e], 0.f);
+                }
+            }
+        if (--left == 0 || s == KS - 1) {
+            left = group;
+#pragma unroll
+            for (int i = 0; i < MT * NT; i++) {
+                tot[i / NT][i % NT] += acc[i / NT][i % NT];
+                acc[i / NT][i % NT] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+        sw = sw_next;
+    };
+#pragma unroll
+    for (int s = 0; s < S; s++) issue(min(s, KS - 1), s);
+    Frag F, G;
+    wait_lds_vmem<(S - 1) * kLoads>();
+    __builtin_amdgcn_s_barrier();
+    read(F, 0);
+    for (int s = 0; s < KS; s += 2) {
+        step(F, G, s);
+        if (s + 1 < KS) step(G, F, s + 1);
+    }
+    // no load may still be writing LDS when the workgroup reuses it, or ends
+    wait_lds_vmem<0>();
+    __builtin_amdgcn_s_barrier();
+    // 16 rows at a time through the wave's own LDS, so that stores write whole row segments
+    const int mw = m0 + wm * WM, nw = n0 + wn * WN;
+    const bool wide = (N & 7) == 0 && ((uintptr_t)y & 15) == 0;
+    float *buf = (float *)smem + wave * (16 * (WN + 4));
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        if (!wide) {
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const int n = nw + 16 * nt + r;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int m = mw + 16 * mt + 4 * g + e;
+                    if (m >= M || n >= N) continue;
+                    if (y_f32) ((float *)y)[(size_t)m * N + n] = tot[mt][nt][e];
+                    else ((uint16_t *)y)[(size_t)m * N + n] = f32_to_bf16_bits(tot[mt][nt][e]);
+                }
+            }
+            continue;
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) buf[(4 * g + e) * (WN + 4) + 16 * nt + r] = tot[mt][nt][e];
+        __builtin_amdgcn_wave_barrier();
+        constexpr int kLanes = WN / 8;  // lanes per row segment, 8 values each
+#pragma unroll
+        for (int i = 0; i < 16 * kLanes / 64; i++) {
+            const int row = (i * 64 + lane) / kLanes, col = (lane % kLanes) * 8;
+            const int m = mw + 16 * mt + row, n = nw + col;
+            const f32x4 v0 = *(const f32x4 *)(buf + row * (WN + 4) + col), v1 = *(const f32x4 *)(buf + row * (WN + 4) + col + 4);
+            if (m >= M || n >= N) continue;
+            if (y_f32) {
+                *(f32x4 *)((float *)y + (size_t)m * N + n) = v0;
+                *(f32x4 *)((float *)y + (size_t)m * N + n + 4) = v1;
+            } else {
+                u32x4 o;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float x = j < 2 ? v0[2 * j] : v1[2 * j - 4], z = j < 2 ? v0[2 * j + 1] : v1[2 * j - 3];
+                    o[j] = (uint32_t)f32_to_bf16_bits(x) | (uint32_t)f32_to_bf16_bits(z) << 16;
+                }
+                *(u32x4 *)((uint16_t *)y + (size_t)m * N + n) = o;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// What k_gemm_tile reads besides the weight codes, one wave per piece: waves [0, na) take 16 rows x
+// 128 K of the activations (QUANT: of bf16 x, quantized as k_act_quant_e4m3 does; else of codes and scale
+// bytes already quantized) into operand order (k_act_quant_e4m3_ops) and their scales into as4 [step][m]
+// dwords, byte g of which is K block 32 g's of the step; the others take the FP4 weights' scale bytes
+// ws [n][K / 32], 64 columns x 16 steps each, into ws4 [step][n] the same way. A tile's operands are then
+// contiguous kilobytes and its scales of a step contiguous dwords: reads of 16 rows x 64 or 8 rows x 128
+// bytes run at half the L2 rate of contiguous ones (measured 23-33 against 44-53 bytes per clock and CU).
+template <bool QUANT>
+__global__ __launch_bounds__(256) void k_gemm_prep(const void *__restrict__ x, const uint8_t *__restrict__ as_, int m,
+                                                   int k, int block, const uint8_t *__restrict__ ws, int n,
+                                                   uint8_t *__restrict__ aq, uint32_t *__restrict__ as4,
+                                                   uint32_t *__restrict__ ws4, int na, int nw) {
+    const int ks = k >> 7, lane = threadIdx.x & 63;
+    const int w = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w >= na) {
+        const int u = w - na, cols = (n + 63) >> 6;
+        if (u >= nw) return;
+        const int c = (u % cols) * 64 + lane, s0 = (u / cols) * 16;
+        if (c >= n) return;
+        const uint8_t *p = ws + (size_t)c * (k >> 5) + 4 * s0;
+        const bool al = ((uintptr_t)p & 3) == 0;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            if (s0 + i >= ks) break;
+            const uint8_t *q = p + 4 * i;
+            ws4[(size_t)(s0 + i) * n + c] = al ? *(const uint32_t *)q : q[0] | q[1] << 8 | q[2] << 16 | (uint32_t)q[3] << 24;
+        }
+        return;
+    }
+    const int mg = w / ks, s = w % ks, r = lane & 15, g = lane >> 4, row = mg * 16 + r;
+    const bool ok = row < m;
+    uint8_t *dst = aq + ops_block(mg, s, ks, false) + lane * 16;
+    if constexpr (!QUANT) {
+        const uint8_t *src = (const uint8_t *)x + (size_t)(ok ? row : 0) * k + (size_t)s * 128 + 16 * g;
+#pragma unroll
+        for (int h = 0; h < 2; h++) *(u32x4 *)(dst + 1024 * h) = *(const u32x4 *)(src + 64 * h);
+        if (ok && block == 128 && g == 0) as4[(size_t)s * m + row] = as_[(size_t)row * ks + s] * 0x01010101u;
+        if (ok && block == 32) ((uint8_t *)as4)[((size_t)s * m + row) * 4 + g] = as_[(size_t)row * (k >> 5) + 4 * s + g];
+        return;
+    } else {
+        u32x4 q[2];
+        uint32_t sb[2];
+        quant_ops((const uint16_t *)x + (size_t)(ok ? row : 0) * k + (size_t)s * 128 + 16 * g, block, q, sb);
+#pragma unroll
+        for (int h = 0; h < 2; h++) *(u32x4 *)(dst + 1024 * h) = q[h];
+        // lane pair (g, g ^ 1) of half h holds the scale of the step's block 2 h + g / 2
+        if (ok && block == 128 && g == 0) as4[(size_t)s * m + row] = sb[0] * 0x01010101u;
+        if (ok && block == 32 && (g & 1) == 0) {
+            uint8_t *d = (uint8_t *)(as4 + (size_t)s * m + row) + (g >> 1);
+            d[0] = (uint8_t)sb[0], d[2] = (uint8_t)sb[1];
+        }
+    }
+}
+
+// GEMM of any number of rows in one launch, for calls whose tiles do not fill the GPU twice: a workgroup
+// owns a 16 MT x 16 NT output tile over all of K; wave w takes the groups w, w + NW, ... of `group` steps
+// each, loads its operands straight from global memory one step ahead of their products, and the groups'
+// sums are added in order through LDS, NW groups at a time. The waves of a tile need no barrier but the
+// sum's and no partial tiles in memory. The order of the sum is gemm_sum's, as in k_gemm_tile; chained
+// groups (a multiple of 4 steps, 4- and 16-byte aligned scales) load their scales four steps at once.
+// q form, FP4, against 64 rows a launch, us: 100 x 2048 x 7168 15.9 -> 11.3, 200 x 512 x 7168 38.6 -> 14.8,
+// 700 x 512 x 4096 100.9 -> 19.3 (2 x 4 tiles); against split K and its second launch: 64 x 4096 x 2176
+// 10.4 -> 5.7, 16 x 256 x 512 7.3 -> 3.6, 8 x 7168 x 2048 (64 x 32 tiles over 16 waves) 11.5 -> 6.5.
+template <bool FP4W, int MT, int NT, int NW, bool CHAIN, bool AARR, bool WOPS>
+__global__ __launch_bounds__(NW * 64) void k_gemm_waves(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
+                                                        const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,
+                                                        void *__restrict__ y, int y_f32, int M, int N, int K, int act32,
+                                                        int group, int mtiles, int ntiles) {
+    constexpr int kTileVecs = MT * NT * 64, kThreads = NW * 64, kPer = (kTileVecs + kThreads - 1) / kThreads;
+    
+    __shared__ f32x4 red[NW * kTileVecs];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int KS = K >> 7;
+    const bool odd = r & 1;
+    const int h0 = odd ? 64 : 0, h1 = 64 - h0;
+    const int total = mtiles * ntiles, xcd = blockIdx.x & 7, per = total >> 3, rem = total & 7;
+    const int t0 = xcd * per + min(xcd, rem) + (int)(blockIdx.x >> 3);
+    const int m0 = (t0 % mtiles) * 16 * MT, n0 = (t0 / mtiles) * 16 * NT;
+    const uint8_t *pa = aq + (AARR ? ((size_t)(m0 >> 4) * KS * 2) * 1024 : (size_t)m0 * K);
+    const uint8_t *pb = wc + (WOPS ? ops_block(n0 >> 4, 0, KS, FP4W) : (size_t)n0 * (FP4W ? K >> 1 : K));
+    uint32_t oa[MT], ob[NT], osa[MT], osb[NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        const int row = min(m0 + 16 * mt + r, M - 1) - m0;
+        if (AARR) oa[mt] = (uint32_t)(min((m0 >> 4) + mt, (M - 1) >> 4) - (m0 >> 4)) * (uint32_t)KS * 2048u + lane * 16;
+        else oa[mt] = (uint32_t)row * (uint32_t)K + 16 * g;
+        osa[mt] = (uint32_t)row * (uint32_t)(act32 ? K >> 5 : KS);
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        const int col = min(n0 + 16 * nt + r, N - 1) - n0;
+        if (WOPS) ob[nt] = (uint32_t)ops_block(min((n0 >> 4) + nt, (N >> 4) - 1) - (n0 >> 4), 0, KS, FP4W) + lane * 16;
+        else ob[nt] = (uint32_t)col * (uint32_t)(FP4W ? K >> 1 : K) + 16 * g;
+        osb[nt] = (uint32_t)col * (uint32_t)(K >> 5);
+    }
+    const uint8_t *psa = as_ + (size_t)m0 * (act32 ? K >> 5 : KS);
+    const uint8_t *psb = (const uint8_t *)ws + (FP4W ? (size_t)n0 * (K >> 5) : 0);
+    const float *wsc = (const float *)ws + (size_t)(n0 >> 7) * KS;
+
+    struct Step {
+        u32x4 a[MT][2], b[NT][FP4W ? 1 : 2];
+        uint32_t sa[MT], sb[NT];
+        float sw;
+    };
+    auto load = [&](Step &S, int s) {
+        const size_t ka = AARR ? (size_t)s * 2048 : (size_t)s * 128;
+        const size_t kb = WOPS ? (size_t)s * (FP4W ? 1024 : 2048) : (size_t)s * (FP4W ? 64 : 128);
+        if constexpr (!CHAIN) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) S.sa[mt] = psa[osa[mt] + (act32 ? 4 * s + g : s)];
+            if constexpr (FP4W) {
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) S.sb[nt] = psb[osb[nt] + 4 * s + g];
+            }
+        }
+        if constexpr (!FP4W) S.sw = wsc[s];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const uint8_t *p = pb + ob[nt] + kb;
+            if constexpr (FP4W) {
+                S.b[nt][0] = *(const u32x4 *)p;
+            } else if constexpr (WOPS) {
+                S.b[nt][0] = *(const u32x4 *)p;
+                S.b[nt][1] = *(const u32x4 *)(p + 1024);
+            } else {
+                S.b[nt][0] = *(const u32x4 *)(p + h0);
+                S.b[nt][1] = *(const u32x4 *)(p + h1);
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const uint8_t *p = pa + oa[mt] + ka;
+            S.a[mt][0] = *(const u32x4 *)(p + (AARR ? 0 : h0));
+            S.a[mt][1] = *(const u32x4 *)(p + (AARR ? 1024 : h1));
+        }
+    };
+    f32x4 acc[MT][NT], tot[kPer];
+    auto compute = [&](const Step &S, const uint32_t (&sa)[MT], const uint32_t (&sb)[NT]) {
+        i32x8 b[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const u32x4 y0 = S.b[nt][0];
+            if constexpr (FP4W) {
+                b[nt] = i32x8{(int)y0[0], (int)y0[1], (int)y0[2], (int)y0[3], 0, 0, 0, 0};
+            } else {
+                const u32x4 y1 = S.b[nt][1];
+                const bool swp = odd && !WOPS;
+                const u32x4 x0 = swp ? y1 : y0, x1 = swp ? y0 : y1;
+                b[nt] = i32x8{(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const bool swp = odd && !AARR;
+            const u32x4 x0 = swp ? S.a[mt][1] : S.a[mt][0], x1 = swp ? S.a[mt][0] : S.a[mt][1];
+            const i32x8 a = {(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                constexpr int bf = FP4W ? 4 : 0;
+                const f32x4 c = CHAIN && FP4W ? acc[mt][nt] : f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[nt], c, 0, bf, 0, (int)sa[mt], 0,
+                                                                                 FP4W ? (int)sb[nt] : 127);
+                if constexpr (CHAIN && FP4W) {
+                    acc[mt][nt] = d;
+                } else if constexpr (CHAIN) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[mt][nt][e] = fmaf(S.sw, d[e], acc[mt][nt][e]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[mt][nt][e] += FP4W ? d[e] : fmaf(S.sw, d[e], 0.f);
+                }
+            }
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < kPer; j++) tot[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int groups = (KS + group - 1) / group;
+    for (int base = 0; base < groups; base += NW) {
+        const int gi = base + wave;
+        if (gi < groups) {
+            const int s0 = gi * group, n = min(group, KS - s0);
+#pragma unroll
+            for (int i = 0; i < MT * NT; i++) acc[i / NT][i % NT] = f32x4{0.f, 0.f, 0.f, 0.f};
+            Step S[2];
+            if constexpr (CHAIN) {  // n is a multiple of 4, and scale words of 4 steps are aligned
+                const int gsh = 8 * g;
+                load(S[0], s0);
+                for (int u = 0; u < n; u += 4) {
+                    u32x4 asw[MT], bsw[NT];
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        if (act32) asw[mt] = *(const u32x4 *)(psa + osa[mt] + 4 * (s0 + u));
+                        else asw[mt][0] = *(const uint32_t *)(psa + osa[mt] + s0 + u);
+                    }
+                    if constexpr (FP4W) {
+#pragma unroll
+                        for (int nt = 0; nt < NT; nt++) bsw[nt] = *(const u32x4 *)(psb + osb[nt] + 4 * (s0 + u));
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        load(S[(q + 1) & 1], min(s0 + u + q + 1, s0 + n - 1));
+                        __builtin_amdgcn_sched_barrier(0);
+                        uint32_t sa[MT], sb[NT];
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++) sa[mt] = act32 ? asw[mt][q] >> gsh : asw[mt][0] >> (8 * q);
+#pragma unroll
+                        for (int nt = 0; nt < NT; nt++) sb[nt] = FP4W ? bsw[nt][q] >> gsh : 0;
+                        compute(S[q & 1], sa, sb);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            } else {
+                load(S[0], s0);
+                for (int u = 0; u < n; u += 2) {
+                    load(S[1], min(s0 + u + 1, s0 + n - 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                    compute(S[0], S[0].sa, S[0].sb);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (u + 1 < n) {
+                        load(S[0], min(s0 + u + 2, s0 + n - 1));
+                        __builtin_amdgcn_sched_barrier(0);
+                        compute(S[1], S[1].sa, S[1].sb);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
+        if (base > 0) __syncthreads();
+        if (gi < groups) {
+#pragma unroll
+            for (int t = 0; t < MT * NT; t++) red[(wave * MT * NT + t) * 64 + lane] = acc[t / NT][t % NT];
+        }
+        __syncthreads();
+        const int live = min(NW, groups - base);
+#pragma unroll
+        for (int j = 0; j < kPer; j++)
+            if (kTileVecs % kThreads == 0 || tid + kThreads * j < kTileVecs)
+                for (int w = 0; w < live; w++) tot[j] += red[w * kTileVecs + tid + kThreads * j];
+    }
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+        const int q = tid + kThreads * j, t = q >> 6, ql = q & 63, mt = t / NT, nt = t % NT;
+        const int n = n0 + 16 * nt + (ql & 15);
+        if (n >= N || q >= kTileVecs) continue;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int m = m0 + 16 * mt + 4 * (ql >> 4) + e;
+            if (m >= M) continue;
+            if (y_f32) ((float *)y)[(size_t)m * N + n] = tot[j][e];
+            else ((uint16_t *)y)[(size_t)m * N + n] = f32_to_bf16_bits(tot[j][e]);
+        }
+    }
+}
+
+// Kernel, tile shape and split of K, chosen per shape (each choice measured fastest for its shape). Calls of
+// up to 64 rows:
+//   kOne64, k_gemm_one with 32 x 64 tiles on 4 waves of 4 steps, when K % 512 == 0, K <= 2048, m > 32
+//     and the tiles give >= 192 workgroups (7168 x 2048: 6.6 us);
+//   kOne32, k_gemm_one with 16 x 32 tiles on up to 8 waves of 8 steps (FP4 weights: 8.2 -> 7.9 us
 //     against 16 waves of 4, 8.9 with 4 waves of 16) or 16 waves of 4 steps (FP8), when K % 512 == 0,
 //     K <= 8192, m > 32 and the tiles give >= 192 workgroups (2048 x 7168: 11.7 -> 8.3 us against
-//     variant 0, and no partial tiles or second launch);
-//   variant 2, 32 x 64 tiles (two workgroups per 64 columns when m > 32) and 16 waves of one step
-//     each, when one slice covers K (<= 16 steps) and the tiles give >= 192 workgroups: per
-//     workgroup 32 rows of activations and 64 columns of weights instead of 64 and 32 (7168 x 2048);
-//   variant 1, 64 x 32 tiles and 16 waves of one step each, when one slice covers K and the tiles
-//     alone give >= 192 workgroups (m <= 32 at 7168 x 2048: no partials and no second launch,
-//     11.6 -> 9.3 us against variant 0);
-//   variant 0 otherwise, 64 x 64 tiles and 8 waves of one step each, K split into slices of <= 8
-//     steps, as many as it takes to give >= 200 workgroups (2048 x 7168: 7 slices, 224 workgroups;
-//     against the earlier 4 waves of 2 steps, FP4 11.9 -> 11.6 us, FP8 12.7 -> 11.8 us).
-// Workgroup b takes column tile u % ntiles and row group u / ntiles, u = b % (ntiles * mgroups), and
-// slice b / (ntiles * mgroups): with ntiles % 8 == 0 the row groups and slices of a column tile run
-// on one XCD.
+//     kSplit);
+//   kWaves24, k_gemm_waves with 32 x 64 tiles, when K <= 2048, m > 32 and these give >= 192 workgroups
+//     (unaligned scales or K % 512 != 0; 64 x 7168 x 1920: 7.6 us FP4, 8.3 FP8; with 16 waves of one
+//     step 7.6 and 9.6);
+//   kWaves22, k_gemm_waves with 32 x 32 tiles, for other K of up to kSplitSteps steps;
+//   kSplit otherwise, k_gemm with 64 x 64 tiles and 8 waves of one step each, K split into slices of <= 8
+//     steps, as many as it takes to give >= 200 workgroups (2048 x 7168: 7 slices, 224 workgroups),
+//     and k_gemm_reduce: with few tiles and many steps the waves of one workgroup are too few
+//     (20 x 512 x 7168: 10.4 us, 13.7 with k_gemm_waves; at 32 steps and less that is the faster one).
+// Calls of more rows: kWaves22 while its 32 x 32 tiles give at most one workgroup per CU, kWaves24 up to
+// twice that (700 x 512 x 4096 FP8: 15.1 us, 19.2 with 32 x 32 and 20.8 with k_gemm_tile), then k_gemm_tile
+// with 64 x 64 tiles (kTile64) or, from one of those per CU on, 64 x 128 tiles on twice the waves (kTile128:
+// 600 x 2048 x 7168 31.4 -> 29.5 us, 1024 x 7168 x 2048 33.2 -> 31.1; 300 x 2048 x 7168 23.9 -> 27.6).
+enum GemmKernel { kSplit, kWaves22, kWaves24, kOne32, kOne64, kTile64, kTile128 };
+
+constexpr int kSplitSteps = 32;
+constexpr int kCUs = 256;
+
 struct GemmPlan {
-    int variant, mt, nt, ntiles, mgroups, slices, steps;
+    GemmKernel kernel;
+    bool chain;  // how the call sums K (k_gemm_tile): steps in groups of `group`, chained or not
+    int group;
+    int slices;  // kSplit: of `group` steps
 };
 
-// one_launch: variants 3 and 4 allowed (their scale loads need 16-byte aligned scale arrays).
-static GemmPlan gemm_plan(int m, int n, int k, bool one_launch = true) {
-    GemmPlan p;
-    const int ks = k / 128;
-    p.mgroups = 1;
-    if (one_launch && ks % 4 == 0 && ks <= 16 && m > 32 && ((n + 63) / 64) * ((m + 31) / 32) >= 192) {
-        p.variant = 4, p.mt = 2, p.nt = 4, p.ntiles = (n + 63) / 64, p.mgroups = (m + 31) / 32, p.slices = 1, p.steps = ks;
-        return p;
+static int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// aligned: the scale arrays are 16-byte aligned (k_gemm_one and chained sums load 4 steps' scales at once).
+// Rows of a call of more than 64 are summed as those of a call of 64, whatever the kernel.
+static GemmPlan gemm_plan(int fmt, int m, int n, int k, bool aligned) {
+    const int ks = k / 128, mc = std::min(m, kGemmMaxM);
+    GemmPlan p = {};
+    if (aligned && ks % 4 == 0 && ks <= 16 && mc > 32 && ceil_div(n, 64) * ceil_div(mc, 32) >= 192) {
+        p = {kOne64, true, 4, 1};
+    } else if (aligned && ks % 4 == 0 && ks <= 64 && mc > 32 && ceil_div(n, 32) * ceil_div(mc, 16) >= 192) {
+        p = {kOne32, true, fmt == 0 ? 8 : 4, 1};
+    } else if (ks <= 16 && mc > 32 && 2 * ceil_div(n, 64) >= 192) {
+        p = {kWaves24, false, 1, 1};
+    } else if (ks <= 16 && ceil_div(n, 32) >= 192) {
+        p = {kWaves22, false, 1, 1};
+    } else {
+        const int tiles = ceil_div(n, 64);
+        const int want = std::max(ceil_div(ks, 8), std::min(ks, ceil_div(200, tiles)));
+        p.group = ceil_div(ks, want), p.slices = ceil_div(ks, p.group);
+        p.kernel = ks > kSplitSteps ? kSplit : kWaves22;
+        if (p.slices == 1) p.group = 1;  // one running sum over the steps
     }
-    if (one_launch && ks % 4 == 0 && ks <= 64 && m > 32 && ((n + 31) / 32) * ((m + 15) / 16) >= 192) {
-        p.variant = 3, p.mt = 1, p.nt = 2, p.ntiles = (n + 31) / 32, p.mgroups = (m + 15) / 16, p.slices = 1, p.steps = ks;
-        return p;
-    }
-    if (ks <= 16 && m > 32 && 2 * ((n + 63) / 64) >= 192) {
-        p.variant = 2, p.mt = 2, p.nt = 4, p.ntiles = (n + 63) / 64, p.mgroups = 2, p.slices = 1, p.steps = ks;
-        return p;
-    }
-    if (ks <= 16 && (n + 31) / 32 >= 192) {
-        p.variant = 1, p.mt = 4, p.nt = 2, p.ntiles = (n + 31) / 32, p.slices = 1, p.steps = ks;
-        return p;
-    }
-    p.variant = 0, p.mt = 4, p.nt = 4, p.ntiles = (n + 63) / 64;
-    const int slices = std::max((ks + 7) / 8, std::min(ks, (200 + p.ntiles - 1) / p.ntiles));
-    p.steps = (ks + slices - 1) / slices;
-    p.slices = (ks + p.steps - 1) / p.steps;
+    if (m <= kGemmMaxM) return p;
+    const int64_t t32 = (int64_t)ceil_div(m, 32) * ceil_div(n, 32), t64 = (int64_t)ceil_div(m, 64) * ceil_div(n, 64);
+    p.kernel = t32 <= kCUs ? kWaves22 : t32 <= 2 * kCUs ? kWaves24 : t64 < kCUs ? kTile64 : kTile128;
     return p;
 }
 
+static bool is_tile(const GemmPlan &p) { return p.kernel == kTile64 || p.kernel == kTile128; }
+
 static uint64_t a256(uint64_t v) { return (v + 255) & ~(uint64_t)255; }
 
-static uint64_t part_bytes(const GemmPlan &p) {
-    return p.slices > 1 ? (uint64_t)p.ntiles * p.slices * (p.mt * p.nt * 64) * 16 : 0;
-}
-
-// Bytes the partial tiles take at the front of `work`: the larger of the plans for m and for m <= 32
-// (the only way m changes the plan), so a workspace sized for m also serves every smaller m. Both
-// are the plans without variants 3 and 4, which need no partials: a call whose scale arrays are not
-// 16-byte aligned falls back to those plans.
-static uint64_t part_reserve(int m, int n, int k) {
-    return a256(std::max(part_bytes(gemm_plan(m, n, k, false)), part_bytes(gemm_plan(1, n, k, false))));
-}
-
-template <int MT, int NT, int NW, bool WOPS>
-static hipError_t launch_gemm_t(const GemmPlan &p, int fmt, void *y, const void *codes, const void *scales,
-                                const uint8_t *aq, int lda, const uint8_t *as_, int m, int n, int k, int shift,
-                                int y_f32, f32x4 *part, hipStream_t st) {
-    static_assert(MT == 4 || NW == 16, "split K (the reduce kernel) takes 64-row tiles only");
-    const dim3 grid(p.ntiles * p.mgroups * p.slices);
-    if (fmt == 0)
-        hipLaunchKernelGGL((k_gemm<true, MT, NT, NW, 1, WOPS>), grid, dim3(NW * 64), 0, st, (const uint8_t *)codes, scales, aq,
-                           as_, part, y, y_f32, m, n, k, lda, shift, p.ntiles, p.mgroups, p.slices, p.steps);
-    else
-        hipLaunchKernelGGL((k_gemm<false, MT, NT, NW, 1, WOPS>), grid, dim3(NW * 64), 0, st, (const uint8_t *)codes, scales, aq,
-                           as_, part, y, y_f32, m, n, k, lda, shift, p.ntiles, p.mgroups, p.slices, p.steps);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && p.slices > 1) {
-        hipLaunchKernelGGL(k_gemm_reduce<NT>, dim3(p.ntiles * (4 * NT * 64) / 256), dim3(256), 0, st, part, p.slices,
-                           p.ntiles, y, y_f32, m, n);
-        e = hipGetLastError();
-    }
-    return e;
-}
-
-// Requires p.steps <= the variant's steps per workgroup and p.slices * p.steps covering k / 128, and
-// split K (slices > 1) only in variant 0; A rows lda bytes apart.
-// arr: the activations are in operand order (k_act_quant_e4m3_ops; variants 3 and 4 only).
-template <bool ARR, bool WOPS>
-static hipError_t launch_gemm_one(const GemmPlan &p, int fmt, void *y, const void *codes, const void *scales,
-                                  const uint8_t *aq, int lda, const uint8_t *as_, int m, int n, int k, int act_block,
-                                  int y_f32, hipStream_t st) {
-    const dim3 grid(p.ntiles * p.mgroups);
-    const int a32 = act_block == 32;
-    if (p.variant == 3 && fmt == 0)
-        hipLaunchKernelGGL((k_gemm_one<true, 1, 2, 8, 2, ARR, WOPS>), grid, dim3(512), 0, st, (const uint8_t *)codes, scales, aq,
-                           as_, y, y_f32, m, n, k, lda, a32, p.ntiles);
-    else if (p.variant == 3)
-        hipLaunchKernelGGL((k_gemm_one<false, 1, 2, 16, 1, ARR, WOPS>), grid, dim3(1024), 0, st, (const uint8_t *)codes, scales,
-                           aq, as_, y, y_f32, m, n, k, lda, a32, p.ntiles);
-    else if (fmt == 0)
-        hipLaunchKernelGGL((k_gemm_one<true, 2, 4, 4, 1, ARR, WOPS>), grid, dim3(256), 0, st, (const uint8_t *)codes, scales, aq,
-                           as_, y, y_f32, m, n, k, lda, a32, p.ntiles);
-    else
-        hipLaunchKernelGGL((k_gemm_one<false, 2, 4, 4, 1, ARR, WOPS>), grid, dim3(256), 0, st, (const uint8_t *)codes, scales,
-                           aq, as_, y, y_f32, m, n, k, lda, a32, p.ntiles);
-    return hipGetLastError();
-}
-
-template <bool WOPS>
-static hipError_t launch_gemm_plan_w(const GemmPlan &p, int fmt, void *y, const void *codes, const void *scales,
-                                     const uint8_t *aq, int lda, const uint8_t *as_, int m, int n, int k, int act_block,
-                                     int y_f32, void *work, hipStream_t st, bool arr) {
-    f32x4 *part = (f32x4 *)work;
-    const int shift = act_block == 32 ? 5 : 7;
-    if (p.variant >= 3)
-        return arr ? launch_gemm_one<true, WOPS>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, act_block, y_f32, st)
-                   : launch_gemm_one<false, WOPS>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, act_block, y_f32, st);
-    if (p.variant == 0)
-        return launch_gemm_t<4, 4, 8, WOPS>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, shift, y_f32, part, st);
-    if (p.variant == 1)
-        return launch_gemm_t<4, 2, 16, WOPS>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, shift, y_f32, part, st);
-    return launch_gemm_t<2, 4, 16, WOPS>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, shift, y_f32, part, st);
-}
-
-// wops: the weight codes are in operand order (k_gemm_pack)
-static hipError_t launch_gemm_plan(const GemmPlan &p, int fmt, void *y, const void *codes, const void *scales,
-                                   const uint8_t *aq, int lda, const uint8_t *as_, int m, int n, int k, int act_block,
-                                   int y_f32, void *work, hipStream_t st, bool arr = false, bool wops = false) {
-    return wops ? launch_gemm_plan_w<true>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, act_block, y_f32, work, st, arr)
-                : launch_gemm_plan_w<false>(p, fmt, y, codes, scales, aq, lda, as_, m, n, k, act_block, y_f32, work, st, arr);
-}
-
-// variants 3 and 4 load scale words 16 bytes at a time; unaligned scale arrays take the other plans
-static GemmPlan plan_for(int fmt, const void *scales, const uint8_t *as_, int m, int n, int k) {
-    return gemm_plan(m, n, k, aligned16(as_) && (fmt != 0 || aligned16(scales)));
-}
-
-static hipError_t launch_gemm(int fmt, void *y, const void *codes, const void *scales, const uint8_t *aq,
-                              const uint8_t *as_, int m, int n, int k, int act_block, int y_f32, void *work,
-                              hipStream_t st, bool wops = false) {
-    return launch_gemm_plan(plan_for(fmt, scales, as_, m, n, k), fmt, y, codes, scales, aq, k, as_, m, n, k, act_block,
-                            y_f32, work, st, false, wops);
+// Bytes the partial tiles of a call of up to 64 rows take at the front of `work`. The split of K does not
+// depend on m, and a call whose scale arrays are not 16-byte aligned may split where an aligned one does
+// not, so the size is that of the plan without alignment.
+static uint64_t part_reserve(int n, int k) {
+    const GemmPlan p = gemm_plan(0, 1, n, k, false);
+    return p.kernel == kSplit ? a256((uint64_t)ceil_div(n, 64) * p.slices * (4 * 4 * 64) * 16) : 0;
 }
 
 // Rows of the activation codes in the workspace: a whole number of 16-row groups (operand order).
-static uint64_t aq_bytes(int m, int k) { return a256((uint64_t)(m + 15) / 16 * 16 * k); }
+static uint64_t aq_bytes(int m, int k) { return a256((uint64_t)ceil_div(m, 16) * 16 * k); }
 
-static int check_gemm(const char *name, int fmt, const void *y, const void *codes, const void *scales, int m, int n,
-                      int k, int act_block, const void *work) {
+// One GEMM call on quantized activations; arr: aq is in operand order (not for kSplit).
+struct GemmArgs {
+    int fmt;
+    bool wops, arr;  // weights / activations in operand order
+    void *y;
+    const uint8_t *codes;
+    const void *scales;
+    const uint8_t *aq, *as_;
+    int m, n, k, act_block, y_f32;
+    hipStream_t st;
+};
+
+template <bool FP4W, bool WOPS>
+static hipError_t launch_split(const GemmPlan &p, const GemmArgs &c, void *work) {
+    const int tiles = ceil_div(c.n, 64);
+    f32x4 *part = (f32x4 *)work;
+    hipLaunchKernelGGL((k_gemm<FP4W, 4, 4, 8, WOPS>), dim3(tiles * p.slices), dim3(512), 0, c.st, c.codes, c.scales, c.aq,
+                       c.as_, part, c.m, c.n, c.k, c.act_block == 32 ? 5 : 7, tiles, p.slices, p.group);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_gemm_reduce<4>, dim3(tiles * (4 * 4 * 64) / 256), dim3(256), 0, c.st, part, p.slices, tiles, c.y,
+                       c.y_f32, c.m, c.n);
+    return hipGetLastError();
+}
+
+template <bool FP4W, int MT, int NT, int NW, int QW, bool ARR, bool WOPS>
+static hipError_t launch_one(const GemmArgs &c) {
+    const int tiles = ceil_div(c.n, 16 * NT);
+    hipLaunchKernelGGL((k_gemm_one<FP4W, MT, NT, NW, QW, ARR, WOPS>), dim3(tiles * ceil_div(c.m, 16 * MT)), dim3(NW * 64), 0,
+                       c.st, c.codes, c.scales, c.aq, c.as_, c.y, c.y_f32, c.m, c.n, c.k, c.k, c.act_block == 32, tiles);
+    return hipGetLastError();
+}
+
+template <bool FP4W, int MT, int NT, bool ARR, bool WOPS>
+static hipError_t launch_waves(const GemmPlan &p, const GemmArgs &c) {
+    const int mt = ceil_div(c.m, 16 * MT), nt = ceil_div(c.n, 16 * NT);
+#define STBL_WAVES(CHAIN)                                                                                             \
+    hipLaunchKernelGGL((k_gemm_waves<FP4W, MT, NT, 8, CHAIN, ARR, WOPS>), dim3((unsigned)mt * nt), dim3(512), 0, c.st,    \
+                       c.codes, c.scales, c.aq, c.as_, c.y, c.y_f32, c.m, c.n, c.k, c.act_block == 32, p.group, mt, nt)
+    if (p.chain) STBL_WAVES(true);
+    else STBL_WAVES(false);
+#undef STBL_WAVES
+    return hipGetLastError();
+}
+
+template <bool FP4W, bool ARR, bool WOPS>
+static hipError_t launch_direct(const GemmPlan &p, const GemmArgs &c) {
+    if (p.kernel == kOne64) return launch_one<FP4W, 2, 4, 4, 1, ARR, WOPS>(c);
+    if (p.kernel == kOne32) return launch_one<FP4W, 1, 2, FP4W ? 8 : 16, FP4W ? 2 : 1, ARR, WOPS>(c);
+    if (p.kernel == kWaves24) return launch_waves<FP4W, 2, 4, ARR, WOPS>(p, c);
+    return launch_waves<FP4W, 2, 2, ARR, WOPS>(p, c);
+}
+
+template <bool FP4W, int BN, int WC, int S, bool WOPS>
+static hipError_t launch_tile(const GemmPlan &p, const GemmArgs &c, const uint8_t *as4, const uint8_t *ws4) {
+    constexpr int BM = 64, lds = S * (BM * 128 + BN * (FP4W ? 64 : 128) + BM * 4 + (FP4W ? BN * 4 : 0));
+    const int mt = ceil_div(c.m, BM), nt = ceil_div(c.n, BN);
+#define STBL_TILE(CHAIN)                                                                                              \
+    hipLaunchKernelGGL((k_gemm_tile<FP4W, BM, BN, 2, WC, S, CHAIN, WOPS>), dim3((unsigned)mt * nt), dim3(2 * WC * 64),   \
+                       lds, c.st, c.codes, c.scales, c.aq, as4, ws4, c.y, c.y_f32, c.m, c.n, c.k, p.group, mt, nt)
+    if (p.chain) STBL_TILE(true);
+    else STBL_TILE(false);
+#undef STBL_TILE
+    return hipGetLastError();
+}
+
+template <bool FP4W, bool WOPS>
+static hipError_t launch_fmt(const GemmPlan &p, const GemmArgs &c, void *work, const uint8_t *as4, const uint8_t *ws4) {
+    if (p.kernel == kTile64) return launch_tile<FP4W, 64, 2, 4, WOPS>(p, c, as4, ws4);
+    if (p.kernel == kTile128) return launch_tile<FP4W, 128, 4, 3, WOPS>(p, c, as4, ws4);
+    if (p.kernel == kSplit) return launch_split<FP4W, WOPS>(p, c, work);
+    return c.arr ? launch_direct<FP4W, true, WOPS>(p, c) : launch_direct<FP4W, false, WOPS>(p, c);
+}
+
+static hipError_t launch_gemm(const GemmPlan &p, const GemmArgs &c, void *work, const uint8_t *as4 = nullptr,
+                              const uint8_t *ws4 = nullptr) {
+    if (c.fmt == 0) return c.wops ? launch_fmt<true, true>(p, c, work, as4, ws4) : launch_fmt<true, false>(p, c, work, as4, ws4);
+    return c.wops ? launch_fmt<false, true>(p, c, work, as4, ws4) : launch_fmt<false, false>(p, c, work, as4, ws4);
+}
+
+static int check_gemm(const char *name, int fmt, const void *y, const void *codes, const void *scales, int m, int max_m,
+                      int n, int k, int act_block, const void *work, bool wops) {
     if (fmt != 0 && fmt != 1) return abi_fail(hipErrorInvalidValue, "%s: unknown format %d", name, fmt);
     if (!y || !codes || !scales || !work) return abi_fail(hipErrorInvalidValue, "%s: null pointer", name);
-    if (m < 1 || m > kGemmMaxM || n < 1 || n > kGemmMaxN || k < 128 || k % 128 || (act_block != 32 && act_block != 128))
+    if (m < 1 || m > max_m || n < 1 || n > kGemmMaxN || k < 128 || k % 128 || (act_block != 32 && act_block != 128))
         return abi_fail(hipErrorInvalidValue,
-                        "%s: need 1 <= m <= 64, n <= %d, k %% 128 == 0, act_block 32 or 128 (m=%d n=%d k=%d)", name,
-                        kGemmMaxN, m, n, k);
+                        "%s: need 1 <= m <= %d, n <= %d, k %% 128 == 0, act_block 32 or 128 (m=%d n=%d k=%d)", name,
+                        max_m, kGemmMaxN, m, n, k);
     if (!aligned16(codes) || !aligned16(work)) return abi_fail(hipErrorInvalidValue, "%s: codes and work must be 16-byte aligned", name);
+    if (wops && n % 16) return abi_fail(hipErrorInvalidValue, "%s: packed weights need n %% 16 == 0 (n=%d)", name, n);
     return 0;
+}
+
+// The workspace of a call of more than 64 rows: activation codes in operand order, then their scales (bytes
+// [m][k / block] for the kernels that read those, dwords [k / 128][m] for k_gemm_tile), then the FP4
+// weights' scale dwords.
+static uint64_t rows_work_bytes(int m, int n, int k) {
+    return aq_bytes(m, k) + a256((uint64_t)m * (k / 32)) + a256((uint64_t)n * (k / 32));
+}
+
+// Activations prepared into `work` as the plan's kernel reads them, then the GEMM. x: bf16, or (quantized) e4m3
+// codes with their scale bytes as_.
+static hipError_t gemm_prepared(GemmPlan p, GemmArgs c, const void *x, bool quantized, uint8_t *aq, uint8_t *as, uint8_t *ws4,
+                                void *work) {
+    const int ks = c.k / 128, na = ceil_div(c.m, 16) * ks;
+    if (is_tile(p)) {
+        const int nw = c.fmt == 0 ? ceil_div(c.n, 64) * ceil_div(ks, 16) : 0;
+        const dim3 grid(ceil_div(na + nw, 4));
+        if (quantized)
+            hipLaunchKernelGGL(k_gemm_prep<false>, grid, dim3(256), 0, c.st, x, c.as_, c.m, c.k, c.act_block,
+                               (const uint8_t *)c.scales, c.n, aq, (uint32_t *)as, (uint32_t *)ws4, na, nw);
+        else
+            hipLaunchKernelGGL(k_gemm_prep<true>, grid, dim3(256), 0, c.st, x, (const uint8_t *)nullptr, c.m, c.k,
+                               c.act_block, (const uint8_t *)c.scales, c.n, aq, (uint32_t *)as, (uint32_t *)ws4, na, nw);
+        c.arr = true;
+    } else if (quantized) {
+        return launch_gemm(p, c, work);  // read in place
+    } else if (p.kernel == kSplit) {
+        const int n8 = c.m * c.k / 8;
+        hipLaunchKernelGGL(k_act_quant_e4m3, dim3(ceil_div(n8, 256)), dim3(256), 0, c.st, (const uint16_t *)x, n8, c.act_block,
+                           aq, as);
+    } else {
+        // operand order: one contiguous kilobyte per load instead of 16 rows x 64 bytes
+        hipLaunchKernelGGL(k_act_quant_e4m3_ops, dim3(na), dim3(64), 0, c.st, (const uint16_t *)x, c.m, c.k, c.act_block, aq, as);
+        c.arr = true;
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    c.aq = aq, c.as_ = as;
+    return launch_gemm(p, c, work, as, ws4);
+}
+
+static int gemm_any(const char *name, int max_m, bool wops, int fmt, void *y, const void *codes, const void *scales,
+                    const void *x, const void *as, bool quantized, int m, int n, int k, int act_block, int y_f32, void *work,
+                    hipStream_t st) {
+    if (int e = check_gemm(name, fmt, y, codes, scales, m, max_m, n, k, act_block, work, wops)) return e;
+    if (quantized && (!x || !as || !aligned16(x))) return abi_fail(hipErrorInvalidValue, "%s: aq (16-byte aligned) and as needed", name);
+    if (!quantized && (!x || !aligned16(x))) return abi_fail(hipErrorInvalidValue, "%s: x must be 16-byte aligned", name);
+    const bool aligned = (!quantized || aligned16(as)) && (fmt != 0 || aligned16(scales));
+    const GemmPlan p = gemm_plan(fmt, m, n, k, aligned);
+    uint8_t *aq = (uint8_t *)work + (m <= kGemmMaxM ? part_reserve(n, k) : 0), *as_ = aq + aq_bytes(m, k);
+    uint8_t *ws4 = as_ + a256((uint64_t)m * (k / 32));
+    const GemmArgs c = {fmt, wops, false, y, (const uint8_t *)codes, scales, (const uint8_t *)x, (const uint8_t *)as,
+                        m, n, k, act_block, y_f32, st};
+    return abi_status(gemm_prepared(p, c, x, quantized, aq, as_, ws4, work), name);
 }
 
 }  // namespace stbl
@@ -696,61 +1246,18 @@ extern "C" {
 
 uint64_t stbl_amd_gemm_work_bytes(int m, int n, int k) {
     if (m < 1 || n < 1 || k < 128) return 256;
-    return part_reserve(m, n, k) + aq_bytes(m, k) + a256((uint64_t)m * (k / 32)) + 256;
+    const uint64_t few = part_reserve(n, k) + aq_bytes(std::min(m, kGemmMaxM), k) + a256((uint64_t)std::min(m, kGemmMaxM) * (k / 32)) + 256;
+    return m > kGemmMaxM ? std::max(few, rows_work_bytes(m, n, k)) : few;
 }
-
-}  // extern "C"
-
-namespace stbl {
-
-static int gemm_q_any(const char *name, bool wops, int fmt, void *y, const void *codes, const void *scales,
-                      const void *aq, const void *as, int m, int n, int k, int act_block, int y_f32, void *work,
-                      hipStream_t st) {
-    if (int e = check_gemm(name, fmt, y, codes, scales, m, n, k, act_block, work)) return e;
-    if (wops && n % 16) return abi_fail(hipErrorInvalidValue, "%s: packed weights need n %% 16 == 0 (n=%d)", name, n);
-    if (!aq || !as || !aligned16(aq)) return abi_fail(hipErrorInvalidValue, "%s: aq (16-byte aligned) and as needed", name);
-    return abi_status(launch_gemm(fmt, y, codes, scales, (const uint8_t *)aq, (const uint8_t *)as, m, n, k, act_block,
-                                  y_f32, work, st, wops),
-                      name);
-}
-
-static int gemm_any(const char *name, bool wops, int fmt, void *y, const void *codes, const void *scales,
-                    const void *x, int m, int n, int k, int act_block, int y_f32, void *work, hipStream_t st) {
-    if (int e = check_gemm(name, fmt, y, codes, scales, m, n, k, act_block, work)) return e;
-    if (wops && n % 16) return abi_fail(hipErrorInvalidValue, "%s: packed weights need n %% 16 == 0 (n=%d)", name, n);
-    if (!x || !aligned16(x)) return abi_fail(hipErrorInvalidValue, "%s: x must be 16-byte aligned", name);
-    uint8_t *aq = (uint8_t *)work + part_reserve(m, n, k);
-    uint8_t *as_ = aq + aq_bytes(m, k);
-    // the one-launch plans read activations this call quantizes in operand order (one contiguous
-    // kilobyte per load instead of 16 rows x 64 bytes)
-    const GemmPlan p = plan_for(fmt, scales, as_, m, n, k);
-    const bool arr = p.variant >= 3;
-    if (arr) {
-        hipLaunchKernelGGL(k_act_quant_e4m3_ops, dim3((m + 15) / 16 * (k / 128)), dim3(64), 0, st, (const uint16_t *)x, m,
-                           k, act_block, aq, as_);
-    } else {
-        const int n8 = m * k / 8;
-        hipLaunchKernelGGL(k_act_quant_e4m3, dim3((n8 + 255) / 256), dim3(256), 0, st, (const uint16_t *)x, n8, act_block,
-                           aq, as_);
-    }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = launch_gemm_plan(p, fmt, y, codes, scales, aq, k, as_, m, n, k, act_block, y_f32, work, st, arr, wops);
-    return abi_status(e, name);
-}
-
-}  // namespace stbl
-
-extern "C" {
 
 int stbl_amd_gemm_q(int fmt, void *y, const void *codes, const void *scales, const void *aq, const void *as, int m,
                     int n, int k, int act_block, int y_f32, void *work, hipStream_t st) {
-    return gemm_q_any("gemm_q", false, fmt, y, codes, scales, aq, as, m, n, k, act_block, y_f32, work, st);
+    return gemm_any("gemm_q", kGemmMaxM, false, fmt, y, codes, scales, aq, as, true, m, n, k, act_block, y_f32, work, st);
 }
 
 int stbl_amd_gemm(int fmt, void *y, const void *codes, const void *scales, const void *x, int m, int n, int k,
                   int act_block, int y_f32, void *work, hipStream_t st) {
-    return gemm_any("gemm", false, fmt, y, codes, scales, x, m, n, k, act_block, y_f32, work, st);
+    return gemm_any("gemm", kGemmMaxM, false, fmt, y, codes, scales, x, nullptr, false, m, n, k, act_block, y_f32, work, st);
 }
 
 int stbl_amd_gemm_pack(int fmt, void *packed, const void *codes, int n, int k, hipStream_t st) {
@@ -767,12 +1274,25 @@ int stbl_amd_gemm_pack(int fmt, void *packed, const void *codes, int n, int k, h
 
 int stbl_amd_gemm_q_packed(int fmt, void *y, const void *packed, const void *scales, const void *aq, const void *as,
                            int m, int n, int k, int act_block, int y_f32, void *work, hipStream_t st) {
-    return gemm_q_any("gemm_q_packed", true, fmt, y, packed, scales, aq, as, m, n, k, act_block, y_f32, work, st);
+    return gemm_any("gemm_q_packed", kGemmMaxM, true, fmt, y, packed, scales, aq, as, true, m, n, k, act_block, y_f32, work, st);
 }
 
 int stbl_amd_gemm_packed(int fmt, void *y, const void *packed, const void *scales, const void *x, int m, int n, int k,
                          int act_block, int y_f32, void *work, hipStream_t st) {
-    return gemm_any("gemm_packed", true, fmt, y, packed, scales, x, m, n, k, act_block, y_f32, work, st);
+    return gemm_any("gemm_packed", kGemmMaxM, true, fmt, y, packed, scales, x, nullptr, false, m, n, k, act_block, y_f32, work,
+                    st);
+}
+
+int stbl_amd_gemm_rows(int fmt, int packed, void *y, const void *codes, const void *scales, const void *x, int m, int n,
+                       int k, int act_block, int y_f32, void *work, hipStream_t st) {
+    return gemm_any("gemm_rows", kGemmMaxRows, packed != 0, fmt, y, codes, scales, x, nullptr, false, m, n, k, act_block, y_f32,
+                    work, st);
+}
+
+int stbl_amd_gemm_q_rows(int fmt, int packed, void *y, const void *codes, const void *scales, const void *aq, const void *as,
+                         int m, int n, int k, int act_block, int y_f32, void *work, hipStream_t st) {
+    return gemm_any("gemm_q_rows", kGemmMaxRows, packed != 0, fmt, y, codes, scales, aq, as, true, m, n, k, act_block, y_f32,
+                    work, st);
 }
 
 // act_quant(x, block, "ue8m0") of ref/kernel.py:35-45 with the codes and E8M0 scale bytes it feeds

@@ -501,46 +501,59 @@ def _work_for(work, m, n, k, device):
 
 
 GEMM_MAX_M = 64  # rows per stbl_amd_gemm / stbl_amd_gemm_q launch
+GEMM_MAX_ROWS = 8192  # rows per stbl_amd_gemm_rows / stbl_amd_gemm_q_rows call
+
+
+def _gemm_rows(packed, codes, scales, x, fmt, act_block, out_f32, work):
+    """gemm / gemm_packed on checked shapes: any number of rows, at most GEMM_MAX_ROWS per call."""
+    m, k = x.shape
+    n = _gemm_shapes(codes, scales, fmt, k)
+    work = _work_for(work, min(m, GEMM_MAX_ROWS), n, k, x.device)
+    y = torch.empty((m, n), dtype=torch.float32 if out_f32 else torch.bfloat16, device=x.device)
+    for r0 in range(0, m, GEMM_MAX_ROWS):
+        r1 = min(m, r0 + GEMM_MAX_ROWS)
+        _lib.check(_lib.load().stbl_amd_gemm_rows(fmt, packed, _ptr(y[r0:r1]), _ptr(codes), _ptr(scales), _ptr(x[r0:r1]),
+                                                  r1 - r0, n, k, act_block, int(out_f32), _ptr(work), _stream()),
+                   "gemm_packed" if packed else "gemm")
+    return y
+
+
+def _gemm_q_rows(packed, codes, scales, aq, a_s, fmt, act_block, out_f32, work):
+    """gemm_q / gemm_q_packed likewise."""
+    name = "gemm_q_packed" if packed else "gemm_q"
+    _need(aq, torch.uint8, "aq", 2)
+    _need(a_s, torch.uint8, "a_s", 2)
+    m, k = aq.shape
+    if m < 1:
+        raise ValueError(f"{name}: aq has no rows")
+    if tuple(a_s.shape) != (m, k // act_block):
+        raise ValueError(f"a_s {tuple(a_s.shape)} does not match aq {tuple(aq.shape)} at block {act_block}")
+    n = _gemm_shapes(codes, scales, fmt, k)
+    work = _work_for(work, min(m, GEMM_MAX_ROWS), n, k, aq.device)
+    y = torch.empty((m, n), dtype=torch.float32 if out_f32 else torch.bfloat16, device=aq.device)
+    for r0 in range(0, m, GEMM_MAX_ROWS):
+        r1 = min(m, r0 + GEMM_MAX_ROWS)
+        _lib.check(_lib.load().stbl_amd_gemm_q_rows(fmt, packed, _ptr(y[r0:r1]), _ptr(codes), _ptr(scales), _ptr(aq[r0:r1]),
+                                                    _ptr(a_s[r0:r1]), r1 - r0, n, k, act_block, int(out_f32), _ptr(work),
+                                                    _stream()), name)
+    return y
 
 
 def gemm(codes, scales, x, fmt, act_block=128, out_f32=False, work=None):
-    """Y [M, N] = act_quant(X, act_block) . Wdeq^T (fp4_gemm / fp8_gemm of ref/kernel.py), any M: one
-    launch per 64 rows (each output row depends only on its own activation row). `work` (from
-    gemm_work) may be passed to reuse the scratch across calls on one stream."""
+    """Y [M, N] = act_quant(X, act_block) . Wdeq^T (fp4_gemm / fp8_gemm of ref/kernel.py), any M (each
+    output row depends only on its own activation row). `work` (from gemm_work) may be passed to reuse
+    the scratch across calls on one stream."""
     _need(x, torch.bfloat16, "x", 2)
-    m, k = x.shape
-    if m < 1:
+    if x.shape[0] < 1:
         raise ValueError("gemm: x has no rows")
-    n = _gemm_shapes(codes, scales, fmt, k)
-    work = _work_for(work, min(m, GEMM_MAX_M), n, k, x.device)
-    y = torch.empty((m, n), dtype=torch.float32 if out_f32 else torch.bfloat16, device=x.device)
-    for r0 in range(0, m, GEMM_MAX_M):
-        mc = min(GEMM_MAX_M, m - r0)
-        _lib.check(_lib.load().stbl_amd_gemm(fmt, _ptr(y[r0:r0 + mc]), _ptr(codes), _ptr(scales), _ptr(x[r0:r0 + mc]),
-                                             mc, n, k, act_block, int(out_f32), _ptr(work), _stream()), "gemm")
-    return y
+    return _gemm_rows(0, codes, scales, x, fmt, act_block, out_f32, work)
 
 
 def gemm_q(codes, scales, aq, a_s, fmt, act_block=128, out_f32=False, work=None):
     """Y [M, N] = (Aq * a_s) . Wdeq^T with the activations already quantized: aq e4m3 codes uint8 [M, K],
     a_s E8M0 scale bytes uint8 [M, K / act_block] (act_quant_e4m3's output), as ref/kernel.py's
-    fp8_gemm(a, a_s, b, b_s) takes them; any M, one launch per 64 rows."""
-    _need(aq, torch.uint8, "aq", 2)
-    _need(a_s, torch.uint8, "a_s", 2)
-    m, k = aq.shape
-    if m < 1:
-        raise ValueError("gemm_q: aq has no rows")
-    if tuple(a_s.shape) != (m, k // act_block):
-        raise ValueError(f"a_s {tuple(a_s.shape)} does not match aq {tuple(aq.shape)} at block {act_block}")
-    n = _gemm_shapes(codes, scales, fmt, k)
-    work = _work_for(work, min(m, GEMM_MAX_M), n, k, aq.device)
-    y = torch.empty((m, n), dtype=torch.float32 if out_f32 else torch.bfloat16, device=aq.device)
-    for r0 in range(0, m, GEMM_MAX_M):
-        mc = min(GEMM_MAX_M, m - r0)
-        _lib.check(_lib.load().stbl_amd_gemm_q(fmt, _ptr(y[r0:r0 + mc]), _ptr(codes), _ptr(scales), _ptr(aq[r0:r0 + mc]),
-                                               _ptr(a_s[r0:r0 + mc]), mc, n, k, act_block, int(out_f32), _ptr(work),
-                                               _stream()), "gemm_q")
-    return y
+    fp8_gemm(a, a_s, b, b_s) takes them; any M."""
+    return _gemm_q_rows(0, codes, scales, aq, a_s, fmt, act_block, out_f32, work)
 
 
 def gemm_pack(codes, fmt):
@@ -557,38 +570,14 @@ def gemm_pack(codes, fmt):
 def gemm_packed(packed, scales, x, fmt, act_block=128, out_f32=False, work=None):
     """gemm() with the weight codes from gemm_pack; the same result bit for bit."""
     _need(x, torch.bfloat16, "x", 2)
-    m, k = x.shape
-    if m < 1:
+    if x.shape[0] < 1:
         raise ValueError("gemm_packed: x has no rows")
-    n = _gemm_shapes(packed, scales, fmt, k)
-    work = _work_for(work, min(m, GEMM_MAX_M), n, k, x.device)
-    y = torch.empty((m, n), dtype=torch.float32 if out_f32 else torch.bfloat16, device=x.device)
-    for r0 in range(0, m, GEMM_MAX_M):
-        mc = min(GEMM_MAX_M, m - r0)
-        _lib.check(_lib.load().stbl_amd_gemm_packed(fmt, _ptr(y[r0:r0 + mc]), _ptr(packed), _ptr(scales),
-                                                    _ptr(x[r0:r0 + mc]), mc, n, k, act_block, int(out_f32), _ptr(work),
-                                                    _stream()), "gemm_packed")
-    return y
+    return _gemm_rows(1, packed, scales, x, fmt, act_block, out_f32, work)
 
 
 def gemm_q_packed(packed, scales, aq, a_s, fmt, act_block=128, out_f32=False, work=None):
     """gemm_q() with the weight codes from gemm_pack; the same result bit for bit."""
-    _need(aq, torch.uint8, "aq", 2)
-    _need(a_s, torch.uint8, "a_s", 2)
-    m, k = aq.shape
-    if m < 1:
-        raise ValueError("gemm_q_packed: aq has no rows")
-    if tuple(a_s.shape) != (m, k // act_block):
-        raise ValueError(f"a_s {tuple(a_s.shape)} does not match aq {tuple(aq.shape)} at block {act_block}")
-    n = _gemm_shapes(packed, scales, fmt, k)
-    work = _work_for(work, min(m, GEMM_MAX_M), n, k, aq.device)
-    y = torch.empty((m, n), dtype=torch.float32 if out_f32 else torch.bfloat16, device=aq.device)
-    for r0 in range(0, m, GEMM_MAX_M):
-        mc = min(GEMM_MAX_M, m - r0)
-        _lib.check(_lib.load().stbl_amd_gemm_q_packed(fmt, _ptr(y[r0:r0 + mc]), _ptr(packed), _ptr(scales),
-                                                      _ptr(aq[r0:r0 + mc]), _ptr(a_s[r0:r0 + mc]), mc, n, k, act_block,
-                                                      int(out_f32), _ptr(work), _stream()), "gemm_q_packed")
-    return y
+    return _gemm_q_rows(1, packed, scales, aq, a_s, fmt, act_block, out_f32, work)
 
 
 def act_quant_e4m3(x, block=128):

@@ -268,3 +268,50 @@ def test_gemm_pack_refuses_bad_shapes(gpu):
     a_s = torch.zeros((64, 2), dtype=torch.uint8, device=gpu)
     with pytest.raises(RuntimeError):
         ops.gemm_q_packed(w, s, aq, a_s, 0)
+
+
+@pytest.mark.parametrize("fmt,block", [(0, 32), (0, 128), (1, 128)])
+@pytest.mark.parametrize("m,n,k,shift", [(65, 16, 128, 0), (70, 2048, 7168, 0), (129, 208, 384, 0), (257, 515, 640, 0),
+                                         (300, 2048, 1024, 0), (200, 2050, 2176, 0), (640, 512, 4096, 0),
+                                         (1000, 1040, 512, 0), (321, 6160, 1536, 0), (260, 1664, 2048, 1),
+                                         (8200, 64, 256, 0)])
+def test_gemm_many_rows_equal_64_row_calls(gpu, fmt, block, m, n, k, shift):
+    # one call on many rows against calls on 64 of them, bit for bit on every whole 64 rows: 32 x 32 and
+    # 32 x 64 tiles of waves, 64 x 64 and 64 x 128 tiles through LDS (their counts cross one and two per
+    # CU), partial tiles in both directions, groups of 1 to 8 steps, chained or not, scales that are not
+    # 16-byte aligned, N that is no multiple of 8 (element stores), and more rows than a call takes; the
+    # first, last and some middle rows against the oracle
+    w = data.weight(n, k, seed=n + k + m)
+    q, deq = (oracle.quant_fp4, oracle.dequant_fp4) if fmt == 0 else (oracle.quant_fp8_b128, oracle.dequant_fp8_b128)
+    codes, scales = q(w.numpy())
+    x = data.activation(m, k, seed=m + 11)
+    dc, ds, xg = torch.from_numpy(codes).to(gpu), torch.from_numpy(scales).to(gpu), x.to(gpu)
+    aq, a_s = ops.act_quant_e4m3(xg, block)
+    if shift:
+        buf = torch.zeros(a_s.numel() + 16, dtype=a_s.dtype, device=gpu)
+        a_s = buf[shift:shift + a_s.numel()].view(a_s.shape).copy_(a_s)
+    y32 = ops.gemm_q(dc, ds, aq, a_s, fmt, block, out_f32=True)
+    whole = min(m, 640) // 64 * 64
+    want = torch.cat([ops.gemm_q(dc, ds, aq[r:r + 64], a_s[r:r + 64], fmt, block, out_f32=True) for r in range(0, whole, 64)])
+    assert torch.equal(y32[:whole], want)
+    rows = sorted({0, 63, m // 2, m - 2, m - 1})
+    _check(np_(y32)[rows], np_(ops.gemm_q(dc, ds, aq, a_s, fmt, block))[rows], _oracle_gemm(x[rows], deq(codes, scales), block))
+    if not shift:
+        assert torch.equal(ops.gemm(dc, ds, xg, fmt, block, out_f32=True), y32)
+    if n % 16 == 0:
+        assert torch.equal(ops.gemm_q_packed(ops.gemm_pack(dc, fmt), ds, aq, a_s, fmt, block, out_f32=True), y32)
+
+
+@pytest.mark.parametrize("fmt,block", [(0, 32), (0, 128), (1, 128)])
+@pytest.mark.parametrize("m,n,k", [(1, 48, 128), (64, 520, 2176), (33, 6160, 1664), (20, 6150, 1152), (64, 300, 4096), (64, 300, 4224)])
+def test_gemm_few_rows_one_launch(gpu, fmt, block, m, n, k):
+    # up to 64 rows in tiles of waves: one group and several, K at and past the most steps such a call takes
+    w = data.weight(n, k, seed=n + k + m)
+    q, deq = (oracle.quant_fp4, oracle.dequant_fp4) if fmt == 0 else (oracle.quant_fp8_b128, oracle.dequant_fp8_b128)
+    codes, scales = q(w.numpy())
+    x = data.activation(m, k, seed=m + 13)
+    dc, ds = torch.from_numpy(codes).to(gpu), torch.from_numpy(scales).to(gpu)
+    y32 = np_(ops.gemm(dc, ds, x.to(gpu), fmt, block, out_f32=True))
+    _check(y32, np_(ops.gemm(dc, ds, x.to(gpu), fmt, block)), _oracle_gemm(x, deq(codes, scales), block))
+    aq, a_s = ops.act_quant_e4m3(x.to(gpu), block)
+    assert bits_equal(np_(ops.gemm_q(dc, ds, aq, a_s, fmt, block, out_f32=True)), y32)
