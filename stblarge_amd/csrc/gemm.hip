@@ -1031,14 +1031,14 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_waves(const uint8_t *__restric
 //   kSplit otherwise, k_gemm with 64 x 64 tiles and 8 waves of one step each, K split into slices of <= 8
 //     steps, as many as it takes to give >= 200 workgroups (2048 x 7168: 7 slices, 224 workgroups),
 //     and k_gemm_reduce: with few tiles and many steps the waves of one workgroup are too few
-//     (20 x 512 x 7168: 10.4 us, 13.7 with k_gemm_waves; at 32 steps and less that is the faster one).
+//     (64 x 512 x 4096: 9.7 us, 13.3 with k_gemm_waves; x 3072: 10.0 and 8.5; 10 x 2048 x 3584: 9.0 and 7.5).
 // Calls of more rows: kWaves22 while its 32 x 32 tiles give at most one workgroup per CU, kWaves24 up to
 // twice that (700 x 512 x 4096 FP8: 15.1 us, 19.2 with 32 x 32 and 20.8 with k_gemm_tile), then k_gemm_tile
 // with 64 x 64 tiles (kTile64) or, from one of those per CU on, 64 x 128 tiles on twice the waves (kTile128:
 // 600 x 2048 x 7168 31.4 -> 29.5 us, 1024 x 7168 x 2048 33.2 -> 31.1; 300 x 2048 x 7168 23.9 -> 27.6).
 enum GemmKernel { kSplit, kWaves22, kWaves24, kOne32, kOne64, kTile64, kTile128 };
 
-constexpr int kSplitSteps = 32;
+constexpr int kSplitSteps = 26;
 constexpr int kCUs = 256;
 
 struct GemmPlan {
