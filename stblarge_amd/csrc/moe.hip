@@ -451,66 +451,80 @@ __global__ __launch_bounds__(256) void k_sqrt_softplus(float *__restrict__ s, in
     if (i < n) s[i] = sqrt_softplus(s[i]);
 }
 
-// One workgroup of 256 threads per token. score = 1 / (1 + exp(-logit)) (score_fn 0, the
-// configuration's router) or sqrt(softplus(logit)) with softplus(l) = l above 20, else
-// log1p(exp(l)) (score_fn 1, stbl/kernels.cu:436-442); the top-k of score + bias (ties to the lower
-// expert id) by k rounds of a workgroup argmax; weight_i = score_i / (sum of the top-k scores in
-// top-k order + 1e-20) * route_scale. A NaN key ranks below every number (so a token with fewer than
-// k numeric keys takes the lowest unused ids next), and its weight comes out NaN.
-__global__ __launch_bounds__(256) void k_route(const float *__restrict__ logits, const float *__restrict__ bias,
+// A float's bits as an unsigned integer of the same order (-0 as +0); 0 is below every float's.
+__device__ __forceinline__ uint32_t float_order(float v) {
+    const uint32_t u = __float_as_uint(v == 0.f ? 0.f : v);
+    return u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u);
+}
+
+// The maximum of a u32 (the minimum: MIN) over the wave, in every lane: rows of 16 by DPP, then the four rows'.
+template <bool MIN>
+__device__ __forceinline__ uint32_t wave_extreme(uint32_t v) {
+    auto pick = [](uint32_t a, uint32_t b) { return MIN ? min(a, b) : max(a, b); };
+#define STBL_EXT(ctrl) v = pick(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, ctrl, 0xF, 0xF, false))
+    STBL_EXT(0xB1);   // quad_perm [1,0,3,2]
+    STBL_EXT(0x4E);   // quad_perm [2,3,0,1]
+    STBL_EXT(0x141);  // row_half_mirror
+    STBL_EXT(0x140);  // row_mirror
+#undef STBL_EXT
+    auto lane = [&](int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); };
+    return pick(pick(lane(0), lane(16)), pick(lane(32), lane(48)));
+}
+
+// One wave per token; lane l holds experts l, l + 64, ... (NI of them) in registers. score = 1 / (1 +
+// exp(-logit)) (score_fn 0, the configuration's router) or sqrt(softplus(logit)) with softplus(l) = l
+// above 20, else log1p(exp(l)) (score_fn 1, stbl/kernels.cu:436-442); the top-k of score + bias (ties to the
+// lower expert id) by k rounds of a wave maximum over the lanes' best keys, where only a tie takes a
+// second reduction, over the ids; weight_i = score_i / (sum of the top-k scores in top-k order + 1e-20) *
+// route_scale. A NaN key ranks with -Inf (so a token with fewer than k numeric keys takes the lowest unused
+// ids next), and its weight comes out NaN. Bound by its chain of rounds: one token,
+// 32 experts, top-8 12.4 us with a workgroup argmax and two barriers a round, 3.0 so; 256 experts 12.0 -> 3.5, 4096 tokens of
+// them 37.1 -> 7.2.
+template <int NI>
+__global__ __launch_bounds__(256) void k_route(const float *__restrict__ logits, const float *__restrict__ bias, int t,
                                                int n_exp, int topk, float route_scale, int score_fn,
                                                int *__restrict__ ids, float *__restrict__ weights,
                                                float *__restrict__ scores) {
-    __shared__ float sc[1024];
-    __shared__ float bv[4];
-    __shared__ int bi[4];
-    __shared__ int chosen[32];
-    const int t = blockIdx.x, tid = threadIdx.x;
-    for (int e = tid; e < n_exp; e += 256) {
-        const float l = logits[(size_t)t * n_exp + e];
-        const float s = score_fn == 1 ? sqrt_softplus(l) : __fdiv_rn(1.f, 1.f + expf(-l));
-        sc[e] = s;
-        if (scores) scores[(size_t)t * n_exp + e] = s;
-    }
-    __syncthreads();
-    for (int p = 0; p < topk; p++) {
-        float best = -INFINITY;
-        int besti = 0x7fffffff;
-        for (int e = tid; e < n_exp; e += 256) {
-            bool used = false;
-            for (int q = 0; q < p; q++) used |= chosen[q] == e;
-            if (used) continue;
-            float v = sc[e] + (bias ? bias[e] : 0.f);
-            v = v != v ? -INFINITY : v;  // a NaN key ranks last; among equal keys the lower id wins
-            if (v > best || (v == best && e < besti)) best = v, besti = e;
-        }
+    const int tok = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (tok >= t) return;  // the whole wave
+    float l[NI], sc[NI];
+    uint32_t key[NI];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(best, off, kWave);
-            const int oi = __shfl_xor(besti, off, kWave);
-            if (ov > best || (ov == best && oi < besti)) best = ov, besti = oi;
-        }
-        if ((tid & 63) == 0) bv[tid >> 6] = best, bi[tid >> 6] = besti;
-        __syncthreads();
-        if (tid == 0) {
-            float b = bv[0];
-            int i = bi[0];
-            for (int w = 1; w < 4; w++)
-                if (bv[w] > b || (bv[w] == b && bi[w] < i)) b = bv[w], i = bi[w];
-            chosen[p] = i;
-        }
-        __syncthreads();
+    for (int i = 0; i < NI; i++) l[i] = logits[(size_t)tok * n_exp + min(lane + 64 * i, n_exp - 1)];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int e = lane + 64 * i;
+        sc[i] = score_fn == 1 ? sqrt_softplus(l[i]) : __fdiv_rn(1.f, 1.f + expf(-l[i]));
+        const float v = sc[i] + (bias ? bias[min(e, n_exp - 1)] : 0.f);
+        key[i] = e < n_exp ? float_order(v != v ? -INFINITY : v) : 0;
+        if (scores && e < n_exp) scores[(size_t)tok * n_exp + e] = sc[i];
     }
-    if (tid == 0) {
-        float sum = 0.f;
-        for (int p = 0; p < topk; p++) sum += sc[chosen[p]];
-        for (int p = 0; p < topk; p++) {
-            float wt = sc[chosen[p]];
-            wt = __fdiv_rn(wt, sum + 1e-20f);
-            wt *= route_scale;
-            ids[(size_t)t * topk + p] = chosen[p];
-            weights[(size_t)t * topk + p] = wt;
+    float sum = 0.f, mine = 0.f;
+    int mine_id = 0;
+    for (int p = 0; p < topk; p++) {
+        uint32_t bk = 0;
+        int bi = lane;
+        float bs = 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; i++)  // ascending ids: the first of equal keys stays
+            if (key[i] > bk) bk = key[i], bi = lane + 64 * i, bs = sc[i];
+        const uint32_t m = wave_extreme<false>(bk);
+        const uint64_t at = __ballot(bk == m);
+        int win = __builtin_ctzll(at), id = __builtin_amdgcn_readlane(bi, win);
+        if (at & (at - 1)) {
+            id = (int)wave_extreme<true>(bk == m ? (uint32_t)bi : 0xffffffffu);
+            win = id & 63;
         }
+        const float s = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(bs), win));
+        sum += s;
+        if (lane == p) mine = s, mine_id = id;
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+            if (lane + 64 * i == id) key[i] = 0;
+    }
+    if (lane < topk) {
+        ids[(size_t)tok * topk + lane] = mine_id;
+        weights[(size_t)tok * topk + lane] = __fdiv_rn(mine, sum + 1e-20f) * route_scale;
     }
 }
 
@@ -1032,8 +1046,13 @@ int stbl_amd_route(const float *logits, const float *bias, int t, int n_exp, int
     if (!logits || !ids || !weights || t < 1 || n_exp < 1 || n_exp > 1024 || topk < 1 || topk > 32 || topk > n_exp)
         return abi_fail(hipErrorInvalidValue, "route: need 1 <= topk <= min(32, n_exp), n_exp <= 1024");
     if (score_fn != 0 && score_fn != 1) return abi_fail(hipErrorInvalidValue, "route: score_fn must be 0 (sigmoid) or 1 (sqrt-softplus)");
-    hipLaunchKernelGGL(k_route, dim3(t), dim3(256), 0, st, logits, bias, n_exp, topk, route_scale, score_fn, ids,
-                       weights, scores);
+#define STBL_ROUTE(NI)                                                                                             \
+    hipLaunchKernelGGL(k_route<NI>, dim3(ceil_div(t, 4)), dim3(256), 0, st, logits, bias, t, n_exp, topk, route_scale, \
+                       score_fn, ids, weights, scores)
+    if (n_exp <= 64) STBL_ROUTE(1);
+    else if (n_exp <= 256) STBL_ROUTE(4);
+    else STBL_ROUTE(16);
+#undef STBL_ROUTE
     return abi_status(hipGetLastError(), "route launch");
 }
 
