@@ -95,6 +95,7 @@ SIGNATURES = {
 }
 
 _lib = None
+native = None  # the compiled call path of stblarge_amd.ops (csrc/bind.cpp), set by load()
 
 
 class StblError(RuntimeError):
@@ -102,8 +103,8 @@ class StblError(RuntimeError):
 
 
 def load():
-    """The bound library (loaded once). Raises if it was not built."""
-    global _lib
+    """The bound library (loaded once). Raises if it, or the compiled call path, was not built."""
+    global _lib, native
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise StblError(f"{LIB_PATH} is missing: build it with `python -m stblarge_amd.build`")
@@ -116,6 +117,12 @@ def load():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        try:
+            from . import _bind
+        except ImportError as e:
+            raise StblError(f"stblarge_amd/_bind.so cannot be loaded ({e}): build it with `python -m stblarge_amd.build`") from e
+        _bind.bind([ctypes.cast(getattr(lib, n), P).value for n in _bind.names()], StblError)
+        native = _bind
         _lib = lib
     return _lib
 

@@ -1,4 +1,5 @@
-"""Builds libstbl_amd.so in-tree with hipcc for gfx950 (no JIT cache: the .so travels with the tree).
+"""Builds libstbl_amd.so in-tree with hipcc for gfx950, and _bind.so, the torch-facing call path of
+stblarge_amd.ops, with g++ (no JIT cache: the .so files travel with the tree).
 
 Run: python -m stblarge_amd.build   (or __graft_entry__.build()).
 """
@@ -10,6 +11,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libstbl_amd.so")
+BIND = os.path.join(HERE, "_bind.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["abi.hip", "quant.hip", "gemv.hip", "moe.hip", "gemm.hip", "expert_cache.hip", "gguf.hip", "calib.hip"]
@@ -37,14 +39,35 @@ def sources():
     return [os.path.join(CSRC, s) for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
 
 
+def bind_command(out):
+    """The g++ command for csrc/bind.cpp, against the torch and Python that run this. The HIP headers that
+    torch's stream header includes ask the host compiler for their platform."""
+    import sysconfig
+
+    import torch
+
+    t = os.path.join(os.path.dirname(torch.__file__))
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DUSE_ROCM=1",
+            "-D__HIP_PLATFORM_AMD__=1", "-isystem", os.path.join(t, "include"), "-isystem",
+            sysconfig.get_paths()["include"], "-isystem", os.path.join(rocm, "include"),
+            os.path.join(CSRC, "bind.cpp"), "-o", out, "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_python"]
+
+
 def build(verbose=False):
-    """Compile every HIP source into one shared library. Always recompiles."""
-    tmp = LIB + ".tmp"
-    cmd = [HIPCC, *FLAGS, "-I", CSRC, "-I", os.path.join(os.path.dirname(HERE), "include"), *sources(), "-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
-    os.replace(tmp, LIB)
+    """Compile every HIP source into one shared library, and the binding. Always recompiles."""
+    lib = [HIPCC, *FLAGS, "-I", CSRC, "-I", os.path.join(os.path.dirname(HERE), "include"), *sources(), "-o", LIB + ".tmp"]
+    jobs = []
+    for cmd, out in ((lib, LIB), (bind_command(BIND + ".tmp"), BIND)):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        jobs.append((subprocess.Popen(cmd), cmd, out))
+    for job, cmd, out in jobs:
+        if job.wait():
+            raise subprocess.CalledProcessError(job.returncode, cmd)
+        os.replace(out + ".tmp", out)
     return LIB
 
 

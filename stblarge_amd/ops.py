@@ -30,6 +30,14 @@ def _stream(stream=None):
     return P(s.cuda_stream)
 
 
+def _native():
+    """The compiled call path (csrc/bind.cpp). Its functions do a whole wrapper's work for plain tensors, and
+    return NotImplemented, having done nothing, where the wrapper has to look closer."""
+    if _lib.native is None:
+        _lib.load()
+    return _lib.native
+
+
 def _need(t, dtype, name, dims=None):
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
@@ -125,6 +133,9 @@ def dequant_fp8(codes, scales, e8m0=False):
 def act_quant(x, block_size=128, pow2=True, want_deq=False):
     """ref/kernel.py:35-45 on bf16 x [..., n]: (codes uint8 [..., n], fp32 scales [..., n/block]);
     with want_deq also the in-place form bf16(e4m3 * s)."""
+    y = _native().act_quant(x, block_size, pow2, want_deq)
+    if y is not NotImplemented:
+        return y
     _need(x, torch.bfloat16, "x")
     n = x.shape[-1]
     rows = x.numel() // n
@@ -140,6 +151,9 @@ def act_quant(x, block_size=128, pow2=True, want_deq=False):
 
 def gemv_fp4(codes, scales, x, out_f32=False, out=None):
     """y [M, N] = x [M, K] . (e2m1(codes) * 2^(scales-127))^T, M <= 4; bf16 (or fp32) output."""
+    y = _native().gemv(FP4, codes, scales, x, out_f32, out)
+    if y is not NotImplemented:
+        return y
     _need(codes, torch.uint8, "codes", 2)
     _need(scales, torch.uint8, "scales", 2)
     _need(x, torch.bfloat16, "x")
@@ -157,6 +171,9 @@ def gemv_fp4(codes, scales, x, out_f32=False, out=None):
 
 def gemv_fp8(codes, scales, x, out_f32=False, out=None):
     """y [M, N] = x [M, K] . (e4m3(codes) * scales[r/128][k/128])^T, M <= 4; bf16 (or fp32) output."""
+    y = _native().gemv(FP8, codes, scales, x, out_f32, out)
+    if y is not NotImplemented:
+        return y
     _need(codes, torch.uint8, "codes", 2)
     _need(scales, torch.float32, "scales", 2)
     _need(x, torch.bfloat16, "x")
@@ -174,6 +191,9 @@ def gemv_fp8(codes, scales, x, out_f32=False, out=None):
 
 def gemv_batch(codes, scales, xs, fmt, out_f32=False, outs=None):
     """len(codes) <= 64 same-shape GEMVs in one launch: ys[j] = gemv(codes[j], scales[j], xs[j])."""
+    y = _native().gemv_batch(codes, scales, xs, fmt, out_f32, outs)
+    if y is not NotImplemented:
+        return y
     n = len(codes)
     if not (len(scales) == n == len(xs)) or n == 0 or n > 64:
         raise ValueError("gemv_batch: need 1..64 matching codes/scales/x")
@@ -230,6 +250,9 @@ def stbl_gemv_mxfp4(y, w, x, rows, k):
 
 
 def stbl_gemv_mxfp4_batch(ys, ws, xs, rows, k):
+    y = _native().mxfp4_batch(ys, ws, xs, rows, k)
+    if y is not NotImplemented:
+        return y
     n = len(ys)
     if not (len(ws) == n == len(xs)) or n == 0 or n > 16:
         raise ValueError("stbl_gemv_mxfp4_batch: need 1..16 matching y/w/x tensors")
@@ -401,6 +424,9 @@ def quant_expert(w_gate, w_up, w_down, fmt, out=None):
 
 def expert_ffn(slot, x, fmt, dim, inter, weight=1.0, limit=0.0, official=False, out_f32=False):
     """y [m, dim] = down(swiglu(gate x, up x)) for one expert slot, m <= 4 tokens."""
+    y = _native().expert_ffn(slot, x, fmt, dim, inter, weight, limit, official, out_f32)
+    if y is not NotImplemented:
+        return y
     _need(slot, torch.uint8, "slot")
     _need(x, torch.bfloat16, "x")
     x2 = _rows2(x)
@@ -428,6 +454,11 @@ def moe_experts(x, slots, pick, weights, fmt, dim, inter, shared=-1, limit=0.0, 
     the always-on expert or -1; shared_fmt: its format when it differs from the routed experts'.
     phase 1 / 2 with slot_ready (one flag per slot): the experts of ready slots, then the others and
     the combine (stbl_amd_moe_experts_phase); both calls need the same out and work."""
+    if phase == 0 and stream is None:
+        y = _native().moe_experts(x, slots, pick, weights, fmt, dim, inter, shared, limit, official, out_f32, work, out,
+                                  shared_fmt)
+        if y is not NotImplemented:
+            return y
     _need(x, torch.bfloat16, "x")
     x2 = _rows2(x)
     t = x2.shape[0]
@@ -462,6 +493,10 @@ SCORE_SIGMOID, SCORE_SQRT_SOFTPLUS = 0, 1
 def route(logits, topk, bias=None, route_scale=1.0, want_scores=False, score_fn=SCORE_SIGMOID, stream=None):
     """Device router: (ids int32 [t, topk], weights fp32 [t, topk][, scores fp32 [t, E]]). score_fn:
     SCORE_SIGMOID (the configuration's) or SCORE_SQRT_SOFTPLUS (the reference engine's)."""
+    if stream is None and not want_scores:
+        y = _native().route(logits, topk, bias, route_scale, score_fn)
+        if y is not NotImplemented:
+            return y
     _need(logits, torch.float32, "logits", 2)
     t, e = logits.shape
     ids = torch.empty((t, topk), dtype=torch.int32, device=logits.device)
@@ -506,6 +541,9 @@ GEMM_MAX_ROWS = 8192  # rows per stbl_amd_gemm_rows / stbl_amd_gemm_q_rows call
 
 def _gemm_rows(packed, codes, scales, x, fmt, act_block, out_f32, work):
     """gemm / gemm_packed on checked shapes: any number of rows, at most GEMM_MAX_ROWS per call."""
+    y = _native().gemm(packed, codes, scales, x, None, fmt, act_block, out_f32, work)
+    if y is not NotImplemented:
+        return y
     m, k = x.shape
     n = _gemm_shapes(codes, scales, fmt, k)
     work = _work_for(work, min(m, GEMM_MAX_ROWS), n, k, x.device)
@@ -520,6 +558,9 @@ def _gemm_rows(packed, codes, scales, x, fmt, act_block, out_f32, work):
 
 def _gemm_q_rows(packed, codes, scales, aq, a_s, fmt, act_block, out_f32, work):
     """gemm_q / gemm_q_packed likewise."""
+    y = _native().gemm(packed, codes, scales, aq, a_s, fmt, act_block, out_f32, work)
+    if y is not NotImplemented:
+        return y
     name = "gemm_q_packed" if packed else "gemm_q"
     _need(aq, torch.uint8, "aq", 2)
     _need(a_s, torch.uint8, "a_s", 2)
@@ -582,6 +623,9 @@ def gemm_q_packed(packed, scales, aq, a_s, fmt, act_block=128, out_f32=False, wo
 
 def act_quant_e4m3(x, block=128):
     """(e4m3 codes uint8 [rows, k], E8M0 scale bytes uint8 [rows, k/block]) of bf16 x."""
+    y = _native().act_quant_e4m3(x, block)
+    if y is not NotImplemented:
+        return y
     _need(x, torch.bfloat16, "x", 2)
     rows, k = x.shape
     codes = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
