@@ -25,13 +25,13 @@ namespace stbl {
 
 // DW: OCP FP4 scales fetched as dwords and handed to the lanes by ds_bpermute (tiles of 4 rows and
 // 2-4 tokens whose scale rows are dword-aligned: k % 128 == 0 and 4-byte aligned scales).
-template <WFmt F, bool XF32, int M, int R, bool DW>
-__global__ __launch_bounds__(512) void k_gemv(GemvJobs jobs, int rows, int k, int out_mode) {
+template <WFmt F, bool XF32, int M, int R, bool DW, int NJ>
+__global__ __launch_bounds__(512) void k_gemv(GemvTable<NJ> jobs, int rows, int k, int out_mode) {
     using T = WTraits<F>;
     constexpr int CH = T::CH;
     static_assert(F == WFmt::FP4_GGUF || 32 % R == 0, "a row tile must sit inside one scale block");
     static_assert(F != WFmt::FP4_GGUF || (XF32 && M == 1), "GGUF rows: the reference ABI's one fp32 token");
-    const GemvJob J = jobs.j[blockIdx.y];
+    const GemvJob J = jobs.j[NJ == 1 ? 0 : blockIdx.y];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int nch = k / CH, c = wave * 64 + lane;
     const bool active = c < nch;
@@ -403,20 +403,27 @@ static hipError_t launch_longk(const GemvJobs &jobs, int njobs, int rows, int k,
     return hipGetLastError();
 }
 
+// The launch with the shortest table that holds its matrices (the reference ABI's batches stop at kMxBatch).
+template <WFmt F, bool XF32, int M, int R, bool DW>
+static hipError_t launch_table(const GemvJobs &jobs, int njobs, int rows, int k, int out_mode, hipStream_t st) {
+    const dim3 grid(ceil_div(rows, R), njobs), block(64 * ceil_div(k / WTraits<F>::CH, 64));
+    if (njobs == 1)
+        hipLaunchKernelGGL((k_gemv<F, XF32, M, R, DW, 1>), grid, block, 0, st, first_jobs<1>(jobs), rows, k, out_mode);
+    else if (XF32 || njobs <= kMxBatch)
+        hipLaunchKernelGGL((k_gemv<F, XF32, M, R, DW, kMxBatch>), grid, block, 0, st, first_jobs<kMxBatch>(jobs), rows, k, out_mode);
+    else if constexpr (!XF32)
+        hipLaunchKernelGGL((k_gemv<F, XF32, M, R, DW, kMaxJobs>), grid, block, 0, st, jobs, rows, k, out_mode);
+    return hipGetLastError();
+}
+
 template <WFmt F, bool XF32, int M, int R>
 static hipError_t launch_r(const GemvJobs &jobs, int njobs, int rows, int k, int out_mode, hipStream_t st) {
-    const int nch = k / WTraits<F>::CH, waves = ceil_div(nch, 64);
-    const dim3 grid(ceil_div(rows, R), njobs), block(64 * waves);
     if constexpr (F == WFmt::FP4_OCP && R == 4 && M >= 2) {
-        bool dw = nch % 4 == 0;
+        bool dw = k / WTraits<F>::CH % 4 == 0;
         for (int j = 0; j < njobs; j++) dw = dw && ((uintptr_t)jobs.j[j].s & 3) == 0;
-        if (dw) {
-            hipLaunchKernelGGL((k_gemv<F, XF32, M, R, true>), grid, block, 0, st, jobs, rows, k, out_mode);
-            return hipGetLastError();
-        }
+        if (dw) return launch_table<F, XF32, M, R, true>(jobs, njobs, rows, k, out_mode, st);
     }
-    hipLaunchKernelGGL((k_gemv<F, XF32, M, R, false>), grid, block, 0, st, jobs, rows, k, out_mode);
-    return hipGetLastError();
+    return launch_table<F, XF32, M, R, false>(jobs, njobs, rows, k, out_mode, st);
 }
 
 // Compute units of the current device (256 on MI355X), read once per device.

@@ -24,6 +24,7 @@
 // renormalized in top-k order (stbl/model.cu:444-451, :528-530 with sigmoid for sqrt-softplus).
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "abi_util.hpp"
 #include "expert_layout.hpp"
@@ -44,9 +45,27 @@ struct MoeJob {
     int pair[kMoeMaxTok];      // rows of the intermediate / output buffers
     float w[kMoeMaxTok];       // route weight of each token
 };
-struct MoeJobs {
-    MoeJob j[kMoeMaxJobs];
+// A launch's jobs, passed by value in a table no longer than the launch needs (as GemvTable).
+constexpr int kMoeFewJobs = 16;
+template <int N>
+struct MoeTable {
+    MoeJob j[N];
 };
+using MoeJobs = MoeTable<kMoeMaxJobs>;
+
+// f(table) with the first n of `jobs`; ONE: launches of one job have a table of their own.
+template <bool ONE, typename F>
+static void with_table(const MoeJobs &jobs, int n, const F &f) {
+    if (ONE && n == 1) {
+        f(MoeTable<1>{{jobs.j[0]}});
+    } else if (n <= kMoeFewJobs) {
+        MoeTable<kMoeFewJobs> t;
+        std::copy(jobs.j, jobs.j + kMoeFewJobs, t.j);
+        f(t);
+    } else {
+        f(jobs);
+    }
+}
 
 // Weights of matrix `mat` (0 gate, 1 up, 2 down) of a slot.
 template <WFmt F>
@@ -256,11 +275,11 @@ __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &
     h[(size_t)pair_out * inter + row0 + r] = f32_to_bf16_bits(__fdiv_rn(gv, 1.f + expf(-gv)) * uv * w_out);
 }
 
-template <WFmt F, int M, int R, bool DW>
-__global__ __launch_bounds__(512) void k_moe_gateup(MoeJobs jobs, ExpertLayout L, const uint16_t *__restrict__ x,
+template <WFmt F, int M, int R, bool DW, int NJ>
+__global__ __launch_bounds__(512) void k_moe_gateup(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x,
                                                     uint16_t *__restrict__ h, int dim, int inter, float limit,
                                                     int official) {
-    gateup_job<F, M, R, DW>(jobs.j[blockIdx.y], L, x, h, dim, inter, limit, official);
+    gateup_job<F, M, R, DW>(jobs.j[NJ == 1 ? 0 : blockIdx.y], L, x, h, dim, inter, limit, official);
 }
 
 // Jobs of two formats in one launch (the reference's FP4 routed experts next to its FP8 E8M0 shared
@@ -272,8 +291,8 @@ constexpr int mix_cpl() {
     return WTraits<FB>::fp4 ? 1 : WTraits<FA>::CH / WTraits<FB>::CH;
 }
 
-template <WFmt FA, WFmt FB, int M, int R, bool DWA, bool DWB>
-__global__ __launch_bounds__(512) void k_moe_gateup_mix(MoeJobs jobs, ExpertLayout LA, ExpertLayout LB,
+template <WFmt FA, WFmt FB, int M, int R, bool DWA, bool DWB, int NJ>
+__global__ __launch_bounds__(512) void k_moe_gateup_mix(MoeTable<NJ> jobs, ExpertLayout LA, ExpertLayout LB,
                                                         const uint16_t *__restrict__ x, uint16_t *__restrict__ h,
                                                         int dim, int inter, float limit, int official, int fmt_a) {
     const MoeJob &J = jobs.j[blockIdx.y];
@@ -353,15 +372,15 @@ __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L,
     else ((uint16_t *)o)[at] = f32_to_bf16_bits(v);
 }
 
-template <WFmt F, int M, int R, bool DW>
-__global__ __launch_bounds__(512) void k_moe_down(MoeJobs jobs, ExpertLayout L, const uint16_t *__restrict__ h,
+template <WFmt F, int M, int R, bool DW, int NJ>
+__global__ __launch_bounds__(512) void k_moe_down(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
                                                   void *__restrict__ o, int dim, int inter, int official, int out_f32) {
-    down_job<F, M, R, DW>(jobs.j[blockIdx.y], L, h, o, dim, inter, official, out_f32);
+    down_job<F, M, R, DW>(jobs.j[NJ == 1 ? 0 : blockIdx.y], L, h, o, dim, inter, official, out_f32);
 }
 
 // Down rows of jobs of two formats in one launch, as k_moe_gateup_mix.
-template <WFmt FA, WFmt FB, int M, int R, bool DWA, bool DWB>
-__global__ __launch_bounds__(512) void k_moe_down_mix(MoeJobs jobs, ExpertLayout LA, ExpertLayout LB,
+template <WFmt FA, WFmt FB, int M, int R, bool DWA, bool DWB, int NJ>
+__global__ __launch_bounds__(512) void k_moe_down_mix(MoeTable<NJ> jobs, ExpertLayout LA, ExpertLayout LB,
                                                       const uint16_t *__restrict__ h, void *__restrict__ o, int dim,
                                                       int inter, int official, int out_f32, int fmt_a) {
     const MoeJob &J = jobs.j[blockIdx.y];
@@ -377,8 +396,8 @@ __global__ __launch_bounds__(512) void k_moe_down_mix(MoeJobs jobs, ExpertLayout
 // stream, instead of running in launches of their own at a fraction of the bandwidth. The kernel
 // needs more registers than the one-token body alone, so a launch of one-token jobs only keeps
 // k_moe_gateup / k_moe_down.
-template <WFmt F, int R, bool DW>
-__global__ __launch_bounds__(512) void k_moe_gateup_any(MoeJobs jobs, ExpertLayout L, const uint16_t *__restrict__ x,
+template <WFmt F, int R, bool DW, int NJ>
+__global__ __launch_bounds__(512) void k_moe_gateup_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x,
                                                         uint16_t *__restrict__ h, int dim, int inter, float limit,
                                                         int official) {
     const MoeJob &J = jobs.j[blockIdx.y];
@@ -397,8 +416,8 @@ __global__ __launch_bounds__(512) void k_moe_gateup_any(MoeJobs jobs, ExpertLayo
     }
 }
 
-template <WFmt F, int R, bool DW>
-__global__ __launch_bounds__(512) void k_moe_down_any(MoeJobs jobs, ExpertLayout L, const uint16_t *__restrict__ h,
+template <WFmt F, int R, bool DW, int NJ>
+__global__ __launch_bounds__(512) void k_moe_down_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
                                                       void *__restrict__ o, int dim, int inter, int official,
                                                       int out_f32) {
     const MoeJob &J = jobs.j[blockIdx.y];
@@ -417,15 +436,18 @@ __global__ __launch_bounds__(512) void k_moe_down_any(MoeJobs jobs, ExpertLayout
 
 // ---- combine ------------------------------------------------------------------------------------
 
+template <int T>
 struct PickTable {
-    int pair[kMoeMaxT][kMoeMaxPick];  // per token: output rows in top-k order, then the shared one
+    uint16_t pair[T][kMoeMaxPick];  // per token: output rows in top-k order, then the shared one
 };
+static_assert(kMoeMaxT * kMoeMaxPick <= 65536, "output rows are 16-bit");
 
 // y[t][r] = bf16(sum over token t's picks in order of o[pair][r]) with the fp32 sum starting at 0
 // (stbl/model.cu:579-592: memset, axpy per expert in top-k order, axpy shared, round_bf16).
 // Every pick's load is issued before the sum (a fixed trip count; unused picks read pick 0's row),
 // so the thread waits for one memory latency, not one per pick.
-__global__ void k_moe_combine(PickTable picks, int npick, const uint16_t *__restrict__ o, void *__restrict__ y,
+template <int T>
+__global__ void k_moe_combine(PickTable<T> picks, int npick, const uint16_t *__restrict__ o, void *__restrict__ y,
                               int dim, int y_f32) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
     if (r >= dim) return;
@@ -546,12 +568,13 @@ static hipError_t launch_gateup_r(const MoeJobs &jobs, int n, const ExpertLayout
     // scales as dwords (slot parts are 256-byte aligned): the MoE steps' 4-row gate/up tiles issue 2
     // dword loads instead of 8 byte loads per lane (measured T=1 41.6 -> 40.1 us, T=4 134.9 -> 126.0
     // us); one expert's 2-row tiles keep byte loads (dwords there: 9.24 -> 9.33 us)
-    if (WTraits<F>::fp4 && R >= 4 && (dim / 32) % 4 == 0)
-        hipLaunchKernelGGL((k_moe_gateup<F, M, R, WTraits<F>::fp4 && R >= 4>), dim3(ceil_div(inter, R), n), dim3(64 * waves), 0,
-                           st, jobs, L, x, h, dim, inter, limit, official);
-    else
-        hipLaunchKernelGGL((k_moe_gateup<F, M, R, false>), dim3(ceil_div(inter, R), n), dim3(64 * waves), 0, st, jobs,
-                           L, x, h, dim, inter, limit, official);
+    const bool dw = WTraits<F>::fp4 && R >= 4 && (dim / 32) % 4 == 0;
+    with_table<true>(jobs, n, [&](const auto &table) {
+        constexpr int NJ = sizeof table / sizeof(MoeJob);
+        const dim3 grid(ceil_div(inter, R), n), block(64 * waves);
+        if (dw) hipLaunchKernelGGL((k_moe_gateup<F, M, R, WTraits<F>::fp4 && R >= 4, NJ>), grid, block, 0, st, table, L, x, h, dim, inter, limit, official);
+        else hipLaunchKernelGGL((k_moe_gateup<F, M, R, false, NJ>), grid, block, 0, st, table, L, x, h, dim, inter, limit, official);
+    });
     return hipGetLastError();
 }
 
@@ -566,12 +589,13 @@ template <WFmt F, int M, int R>
 static hipError_t launch_down_r(const MoeJobs &jobs, int n, const ExpertLayout &L, const uint16_t *h, void *o, int dim,
                                 int inter, int official, int out_f32, hipStream_t st) {
     const int waves = ceil_div(inter / WTraits<F>::CH, 64);
-    if (WTraits<F>::fp4 && R >= 4 && (inter / 32) % 4 == 0)
-        hipLaunchKernelGGL((k_moe_down<F, M, R, WTraits<F>::fp4 && R >= 4>), dim3(ceil_div(dim, R), n), dim3(64 * waves), 0, st,
-                           jobs, L, h, o, dim, inter, official, out_f32);
-    else
-        hipLaunchKernelGGL((k_moe_down<F, M, R, false>), dim3(ceil_div(dim, R), n), dim3(64 * waves), 0, st, jobs, L,
-                           h, o, dim, inter, official, out_f32);
+    const bool dw = WTraits<F>::fp4 && R >= 4 && (inter / 32) % 4 == 0;
+    with_table<true>(jobs, n, [&](const auto &table) {
+        constexpr int NJ = sizeof table / sizeof(MoeJob);
+        const dim3 grid(ceil_div(dim, R), n), block(64 * waves);
+        if (dw) hipLaunchKernelGGL((k_moe_down<F, M, R, WTraits<F>::fp4 && R >= 4, NJ>), grid, block, 0, st, table, L, h, o, dim, inter, official, out_f32);
+        else hipLaunchKernelGGL((k_moe_down<F, M, R, false, NJ>), grid, block, 0, st, table, L, h, o, dim, inter, official, out_f32);
+    });
     return hipGetLastError();
 }
 
@@ -601,23 +625,18 @@ static hipError_t launch_any(bool gateup, const MoeJobs &jobs, int n, const Expe
     const dim3 block(64 * ceil_div(k / WTraits<F>::CH, 64));
     // FP4 tiles whose scale rows are a multiple of 4 bytes fetch their scales as dwords
     const bool dw = WTraits<F>::fp4 && (k / 32) % 4 == 0;
-    if (gateup) {
-        const dim3 grid(ceil_div(inter, 4), n);
-        if (dw)
-            hipLaunchKernelGGL((k_moe_gateup_any<F, 4, WTraits<F>::fp4>), grid, block, 0, st, jobs, L, x, h, dim, inter,
-                               limit, official);
+    with_table<false>(jobs, n, [&](const auto &table) {
+        constexpr int NJ = sizeof table / sizeof(MoeJob);
+        const dim3 grid(gateup ? ceil_div(inter, 4) : ceil_div(dim, 8), n);
+        if (gateup && dw)
+            hipLaunchKernelGGL((k_moe_gateup_any<F, 4, WTraits<F>::fp4, NJ>), grid, block, 0, st, table, L, x, h, dim, inter, limit, official);
+        else if (gateup)
+            hipLaunchKernelGGL((k_moe_gateup_any<F, 4, false, NJ>), grid, block, 0, st, table, L, x, h, dim, inter, limit, official);
+        else if (dw)
+            hipLaunchKernelGGL((k_moe_down_any<F, 8, WTraits<F>::fp4, NJ>), grid, block, 0, st, table, L, h, o, dim, inter, official, out_f32);
         else
-            hipLaunchKernelGGL((k_moe_gateup_any<F, 4, false>), grid, block, 0, st, jobs, L, x, h, dim, inter, limit,
-                               official);
-    } else {
-        const dim3 grid(ceil_div(dim, 8), n);
-        if (dw)
-            hipLaunchKernelGGL((k_moe_down_any<F, 8, WTraits<F>::fp4>), grid, block, 0, st, jobs, L, h, o, dim, inter,
-                               official, out_f32);
-        else
-            hipLaunchKernelGGL((k_moe_down_any<F, 8, false>), grid, block, 0, st, jobs, L, h, o, dim, inter, official,
-                               out_f32);
-    }
+            hipLaunchKernelGGL((k_moe_down_any<F, 8, false, NJ>), grid, block, 0, st, table, L, h, o, dim, inter, official, out_f32);
+    });
     return hipGetLastError();
 }
 
@@ -703,29 +722,24 @@ static hipError_t launch_mix(bool gateup, const MoeJobs &jobs, int n, int fmt_a,
     const int waves = std::max(ceil_div(k / WTraits<FA>::CH, 64), ceil_div(k / (WTraits<FB>::CH * mix_cpl<FA, FB>()), 64));
     // FP4 tiles of 4+ rows whose scale rows are a multiple of 4 bytes fetch their scales as dwords
     const bool dwa = WTraits<FA>::fp4 && (k / 32) % 4 == 0, dwb = WTraits<FB>::fp4 && (k / 32) % 4 == 0;
-    if (gateup) {
-        constexpr int R = 4;
-        const dim3 grid(ceil_div(inter, R), n), block(64 * waves);
-#define STBL_GU(DA, DB)                                                                                          \
-    hipLaunchKernelGGL((k_moe_gateup_mix<FA, FB, M, R, DA, DB>), grid, block, 0, st, jobs, LA, LB, x, h, dim, inter, \
-                       limit, official, fmt_a)
-        if (dwa && dwb) STBL_GU(WTraits<FA>::fp4, WTraits<FB>::fp4);
-        else if (dwa) STBL_GU(WTraits<FA>::fp4, false);
-        else if (dwb) STBL_GU(false, WTraits<FB>::fp4);
-        else STBL_GU(false, false);
-#undef STBL_GU
-    } else {
-        constexpr int R = M == 4 ? 4 : 8;
-        const dim3 grid(ceil_div(dim, R), n), block(64 * waves);
-#define STBL_DN(DA, DB)                                                                                             \
-    hipLaunchKernelGGL((k_moe_down_mix<FA, FB, M, R, DA, DB>), grid, block, 0, st, jobs, LA, LB, h, o, dim, inter, \
-                       official, out_f32, fmt_a)
-        if (dwa && dwb) STBL_DN(WTraits<FA>::fp4, WTraits<FB>::fp4);
-        else if (dwa) STBL_DN(WTraits<FA>::fp4, false);
-        else if (dwb) STBL_DN(false, WTraits<FB>::fp4);
-        else STBL_DN(false, false);
-#undef STBL_DN
-    }
+    with_table<false>(jobs, n, [&](const auto &table) {
+        constexpr int NJ = sizeof table / sizeof(MoeJob), RG = 4, RD = M == 4 ? 4 : 8;
+        const dim3 grid(gateup ? ceil_div(inter, RG) : ceil_div(dim, RD), n), block(64 * waves);
+        auto go = [&](auto da, auto db) {
+            if (gateup)
+                hipLaunchKernelGGL((k_moe_gateup_mix<FA, FB, M, RG, da(), db(), NJ>), grid, block, 0, st, table, LA, LB, x, h,
+                                   dim, inter, limit, official, fmt_a);
+            else
+                hipLaunchKernelGGL((k_moe_down_mix<FA, FB, M, RD, da(), db(), NJ>), grid, block, 0, st, table, LA, LB, h, o,
+                                   dim, inter, official, out_f32, fmt_a);
+        };
+        using A = std::integral_constant<bool, WTraits<FA>::fp4>;
+        using B = std::integral_constant<bool, WTraits<FB>::fp4>;
+        if (dwa && dwb) go(A(), B());
+        else if (dwa) go(A(), std::false_type());
+        else if (dwb) go(std::false_type(), B());
+        else go(std::false_type(), std::false_type());
+    });
     return hipGetLastError();
 }
 
@@ -906,7 +920,7 @@ static int moe_experts_impl(int fmt, void *y, const void *x, int t, int dim, int
     // so both phases number them alike. A shared expert of another format runs in launches of its
     // own (sjobs). Each array holds every (token, pick) pair, duplicates included.
     static thread_local MoeJob jobs[kMoeMaxT * kMoeMaxPick], sjobs[kMoeMaxT * kMoeMaxPick];
-    PickTable table = {};
+    PickTable<kMoeMaxT> table = {};
     int njobs = 0, nsjobs = 0, npairs = 0;
     for (int s = 0; s < n_slots; s++) {
         const bool run = phase == 0 || (phase == 1) == (slot_ready[s] != 0);
@@ -915,7 +929,7 @@ static int moe_experts_impl(int fmt, void *y, const void *x, int t, int dim, int
             for (int p = 0; p < npick; p++) {
                 const int sl = p < topk ? pick[tt * topk + p] : shared;
                 if (sl != s) continue;
-                table.pair[tt][p] = npairs;
+                table.pair[tt][p] = (uint16_t)npairs;
                 if (run) {
                     if (!J || J->m == kMoeMaxTok) {
                         const bool other = s == shared && shared_fmt != fmt;
@@ -946,7 +960,14 @@ static int moe_experts_impl(int fmt, void *y, const void *x, int t, int dim, int
             e = run_fmt(shared_fmt, sjobs, nsjobs, dim, inter, (const uint16_t *)x, h, o, limit, official, 0, st);
     }
     if (e == hipSuccess && phase != 1) {
-        hipLaunchKernelGGL(k_moe_combine, dim3(ceil_div(dim, 256), t), dim3(256), 0, st, table, npick, o, y, dim, y_f32);
+        const dim3 grid(ceil_div(dim, 256), t);
+        if (t == 1) {
+            PickTable<1> one;
+            std::copy(table.pair[0], table.pair[0] + kMoeMaxPick, one.pair[0]);
+            hipLaunchKernelGGL(k_moe_combine<1>, grid, dim3(256), 0, st, one, npick, o, y, dim, y_f32);
+        } else {
+            hipLaunchKernelGGL(k_moe_combine<kMoeMaxT>, grid, dim3(256), 0, st, table, npick, o, y, dim, y_f32);
+        }
         e = hipGetLastError();
     }
     return abi_status(e, "moe_experts launch");
