@@ -179,8 +179,7 @@ class MoELayer:
         self.last_lookup = None  # (distinct expert ids in lookup order, hit flags) of the last step
 
     def route(self, logits):
-        ids, w = ops.route(logits, self.topk, self.bias, self.route_scale, score_fn=self.score_fn)
-        return ids.cpu().tolist(), w.cpu().tolist()  # host sync, as the reference's to_host
+        return ops.route_to_host(logits, self.topk, self.bias, self.route_scale, self.score_fn)  # the reference's to_host
 
     def forward(self, x, logits, route=None, stream=None, after_reads=None):
         """y = the layer's output for x. Every device call goes on `stream` (default: the current

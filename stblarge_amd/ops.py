@@ -509,6 +509,23 @@ def route(logits, topk, bias=None, route_scale=1.0, want_scores=False, score_fn=
     return (ids, w, sc) if want_scores else (ids, w)
 
 
+def route_to_host(logits, topk, bias=None, route_scale=1.0, score_fn=SCORE_SIGMOID):
+    """route() as lists on the host: (ids [t][topk], weights [t][topk]). The kernel writes them into pinned
+    host memory, so the host waits for it once, and no copies follow (a resident one-token layer at 7168 x 2048: 88.6 us
+    with two copies, 70.7 so)."""
+    _need(logits, torch.float32, "logits", 2)
+    t, e = logits.shape
+    ids = torch.empty((t, topk), dtype=torch.int32, pin_memory=True)
+    w = torch.empty((t, topk), dtype=torch.float32, pin_memory=True)
+    if bias is not None:
+        _need(bias, torch.float32, "bias", 1)
+    stream = torch.cuda.current_stream()
+    _lib.check(_lib.load().stbl_amd_route(_ptr(logits), _ptr(bias), t, e, topk, float(route_scale), int(score_fn),
+                                          _ptr(ids), _ptr(w), None, P(stream.cuda_stream)), "route")
+    stream.synchronize()
+    return ids.tolist(), w.tolist()
+
+
 # ---- multi-token GEMM (scaled MFMA) ------------------------------------------------------------------
 
 def _gemm_shapes(codes, scales, fmt, k):
