@@ -36,6 +36,7 @@ constexpr int kMoeMaxTok = 4;    // tokens per job
 constexpr int kMoeMaxJobs = 40;  // jobs per launch
 constexpr int kMoeMaxT = 16;     // tokens per MoE call
 constexpr int kMoeMaxPick = 17;  // top-k + shared
+constexpr int kQuantOnceTokens = 2;  // official numerics: tokens from which activations are quantized once
 
 struct MoeJob {
     const uint8_t *slot;
@@ -434,6 +435,38 @@ __global__ __launch_bounds__(512) void k_moe_down_any(MoeTable<NJ> jobs, ExpertL
     }
 }
 
+// ---- official numerics of several tokens --------------------------------------------------------------
+
+// out = the values that the gate/up and down kernels make of x in registers in official numerics
+// (act_quant_packed), 16 per thread; in place or not. With several tokens every workgroup of a job quantizes
+// its tokens' chunks again, which costs as much as a quarter of its products; quantized once, x and the
+// SwiGLU outputs cost two small launches instead (5120 x 2304, top-6 and an FP8 shared expert, us: 4 tokens 120.5
+// -> 92.3, 3 tokens 98.4 -> 79.0, 2 tokens 58.9 -> 55.6; one token, whose launches take 33.2 without any
+// quantization, keeps its 36.0).
+__global__ __launch_bounds__(256) void k_moe_act_quant(const uint16_t *x, uint16_t *out, int n16) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const bool ok = i < n16;  // n16 is even: a block's two lanes are both in or both out
+    const u32x4 *src = (const u32x4 *)(x + (size_t)(ok ? i : 0) * 16);
+    uint32_t w[1][8];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const u32x4 v = src[q];
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[0][4 * q + j] = v[j];
+    }
+    act_quant_packed<1, 16>(w);
+    if (!ok) return;
+    u32x4 *dst = (u32x4 *)(out + (size_t)i * 16);
+    dst[0] = u32x4{w[0][0], w[0][1], w[0][2], w[0][3]};
+    dst[1] = u32x4{w[0][4], w[0][5], w[0][6], w[0][7]};
+}
+
+static hipError_t launch_act_quant(const uint16_t *x, uint16_t *out, size_t n, hipStream_t st) {
+    const int n16 = (int)(n / 16);
+    hipLaunchKernelGGL(k_moe_act_quant, dim3((n16 + 255) / 256), dim3(256), 0, st, x, out, n16);
+    return hipGetLastError();
+}
+
 // ---- combine ------------------------------------------------------------------------------------
 
 template <int T>
@@ -640,13 +673,17 @@ static hipError_t launch_any(bool gateup, const MoeJobs &jobs, int n, const Expe
     return hipGetLastError();
 }
 
+// The launches that a run_ function issues: gate/up, down, or both.
+constexpr int kGateUp = 1, kDown = 2, kBothParts = 3;
+
 // Runs jobs of one format and several token classes through one gate/up and one down launch (per
 // kMoeMaxJobs jobs), in order of falling token class: the workgroups with the most arithmetic per
 // byte are dispatched first, so it overlaps the one-token jobs' streaming.
 template <WFmt F>
 static hipError_t run_jobs_any(const MoeJob *all, int njobs, const ExpertLayout &L, const uint16_t *x, uint16_t *h,
-                               void *o, int dim, int inter, float limit, int official, int out_f32, hipStream_t st) {
+                               void *o, int dim, int inter, float limit, int official, int out_f32, hipStream_t st, int parts = kBothParts) {
     for (int phase = 0; phase < 2; phase++) {
+        if (!(parts >> phase & 1)) continue;
         MoeJobs batch;
         int n = 0;
         auto flush = [&]() -> hipError_t {
@@ -674,8 +711,9 @@ static hipError_t run_jobs_any(const MoeJob *all, int njobs, const ExpertLayout 
 template <WFmt F>
 static hipError_t run_jobs_by_class(const MoeJob *all, int njobs, const ExpertLayout &L, const uint16_t *x,
                                     uint16_t *h, void *o, int dim, int inter, float limit, int official, int out_f32,
-                                    hipStream_t st) {
+                                    hipStream_t st, int parts = kBothParts) {
     for (int phase = 0; phase < 2; phase++) {
+        if (!(parts >> phase & 1)) continue;
         for (int mclass = 1; mclass <= 3; mclass++) {  // M = 1, 2, 4 templates
             MoeJobs batch;
             int n = 0;
@@ -750,9 +788,10 @@ static hipError_t launch_mix(bool gateup, const MoeJobs &jobs, int n, int fmt_a,
 template <WFmt FA, WFmt FB>
 static hipError_t run_jobs_mix_by_class(const MoeJob *all, int njobs, int fmt_a, int fmt_b, const uint16_t *x,
                                         uint16_t *h, void *o, int dim, int inter, float limit, int official,
-                                        int out_f32, hipStream_t st) {
+                                        int out_f32, hipStream_t st, int parts = kBothParts) {
     const ExpertLayout LA = expert_layout(fmt_a, dim, inter), LB = expert_layout(fmt_b, dim, inter);
     for (int phase = 0; phase < 2; phase++) {
+        if (!(parts >> phase & 1)) continue;
         for (int mclass = 1; mclass <= 3; mclass++) {
             MoeJobs batch;
             int n = 0, na = 0, nb = 0;
@@ -808,7 +847,7 @@ static hipError_t run_jobs_mix_by_class(const MoeJob *all, int njobs, int fmt_a,
 // (measured with FP8 E8M0 jobs of two chunks per lane: C4 T=4 122 -> 137 us, V4.1 T=4 108 -> 115 us).
 template <WFmt FA, WFmt FB>
 static hipError_t run_jobs_split(const MoeJob *all, int njobs, int fmt_a, int fmt_b, const uint16_t *x, uint16_t *h,
-                                 void *o, int dim, int inter, float limit, int official, int out_f32, hipStream_t st) {
+                                 void *o, int dim, int inter, float limit, int official, int out_f32, hipStream_t st, int parts = kBothParts) {
     const ExpertLayout LA = expert_layout(fmt_a, dim, inter);
     static thread_local MoeJob lo[kMoeMaxT * kMoeMaxPick], hi[kMoeMaxT * kMoeMaxPick];
     int nlo = 0, nhi = 0;
@@ -817,29 +856,29 @@ static hipError_t run_jobs_split(const MoeJob *all, int njobs, int fmt_a, int fm
         else hi[nhi++] = all[j];
     }
     if (!several_classes(lo, nlo)) {
-        if constexpr (FA == FB) return run_jobs_by_class<FA>(all, njobs, LA, x, h, o, dim, inter, limit, official, out_f32, st);
-        else return run_jobs_mix_by_class<FA, FB>(all, njobs, fmt_a, fmt_b, x, h, o, dim, inter, limit, official, out_f32, st);
+        if constexpr (FA == FB) return run_jobs_by_class<FA>(all, njobs, LA, x, h, o, dim, inter, limit, official, out_f32, st, parts);
+        else return run_jobs_mix_by_class<FA, FB>(all, njobs, fmt_a, fmt_b, x, h, o, dim, inter, limit, official, out_f32, st, parts);
     }
-    hipError_t e = run_jobs_any<FA>(lo, nlo, LA, x, h, o, dim, inter, limit, official, out_f32, st);
+    hipError_t e = run_jobs_any<FA>(lo, nlo, LA, x, h, o, dim, inter, limit, official, out_f32, st, parts);
     if constexpr (FA != FB) {
         if (e == hipSuccess && nhi > 0)
             e = run_jobs_by_class<FB>(hi, nhi, expert_layout(fmt_b, dim, inter), x, h, o, dim, inter, limit, official,
-                                      out_f32, st);
+                                      out_f32, st, parts);
     }
     return e;
 }
 
 // Runs jobs whose slots hold format fmt.
 static hipError_t run_fmt(int fmt, const MoeJob *all, int njobs, int dim, int inter, const uint16_t *x, uint16_t *h,
-                          void *o, float limit, int official, int out_f32, hipStream_t st) {
+                          void *o, float limit, int official, int out_f32, hipStream_t st, int parts = kBothParts) {
     if (fmt == EXPERT_FP4)
         return run_jobs_split<WFmt::FP4_OCP, WFmt::FP4_OCP>(all, njobs, fmt, fmt, x, h, o, dim, inter, limit, official,
-                                                            out_f32, st);
+                                                            out_f32, st, parts);
     if (fmt == EXPERT_FP8)
         return run_jobs_split<WFmt::FP8_B128, WFmt::FP8_B128>(all, njobs, fmt, fmt, x, h, o, dim, inter, limit, official,
-                                                              out_f32, st);
+                                                              out_f32, st, parts);
     return run_jobs_split<WFmt::FP8_E8M0, WFmt::FP8_E8M0>(all, njobs, fmt, fmt, x, h, o, dim, inter, limit, official,
-                                                          out_f32, st);
+                                                          out_f32, st, parts);
 }
 
 static bool fmt_ok(int fmt) { return fmt == EXPERT_FP4 || fmt == EXPERT_FP8 || fmt == EXPERT_FP8_E8M0; }
@@ -948,16 +987,29 @@ static int moe_experts_impl(int fmt, void *y, const void *x, int t, int dim, int
     }
     uint16_t *h = (uint16_t *)work;
     uint16_t *o = h + (size_t)t * npick * inter;
-    hipError_t e;
-    if (nsjobs > 0 && fmt == EXPERT_FP4 && shared_fmt == EXPERT_FP8_E8M0) {
-        // the reference's pairing (FP4 routed, FP8 E8M0 shared): both formats in the same launches
-        for (int i = 0; i < nsjobs; i++) jobs[njobs + i] = sjobs[i];
-        e = run_jobs_split<WFmt::FP4_OCP, WFmt::FP8_E8M0>(jobs, njobs + nsjobs, EXPERT_FP4, EXPERT_FP8_E8M0,
-                                                          (const uint16_t *)x, h, o, dim, inter, limit, official, 0, st);
-    } else {
-        e = run_fmt(fmt, jobs, njobs, dim, inter, (const uint16_t *)x, h, o, limit, official, 0, st);
+    auto run = [&](const uint16_t *in, int act, int parts) -> hipError_t {
+        if (nsjobs > 0 && fmt == EXPERT_FP4 && shared_fmt == EXPERT_FP8_E8M0)
+            // the reference's pairing (FP4 routed, FP8 E8M0 shared): both formats in the same launches
+            return run_jobs_split<WFmt::FP4_OCP, WFmt::FP8_E8M0>(jobs, njobs + nsjobs, EXPERT_FP4, EXPERT_FP8_E8M0, in, h, o,
+                                                                 dim, inter, limit, act, 0, st, parts);
+        hipError_t e = run_fmt(fmt, jobs, njobs, dim, inter, in, h, o, limit, act, 0, st, parts);
         if (e == hipSuccess && nsjobs > 0)
-            e = run_fmt(shared_fmt, sjobs, nsjobs, dim, inter, (const uint16_t *)x, h, o, limit, official, 0, st);
+            e = run_fmt(shared_fmt, sjobs, nsjobs, dim, inter, in, h, o, limit, act, 0, st, parts);
+        return e;
+    };
+    if (nsjobs > 0 && fmt == EXPERT_FP4 && shared_fmt == EXPERT_FP8_E8M0)
+        for (int i = 0; i < nsjobs; i++) jobs[njobs + i] = sjobs[i];
+    hipError_t e;
+    if (official && phase == 0 && t >= kQuantOnceTokens) {
+        // the quantized x waits in the output rows' memory, which only the down launches write (phases 1 and
+        // 2 have outputs of each other there)
+        uint16_t *xq = o;
+        e = launch_act_quant((const uint16_t *)x, xq, (size_t)t * dim, st);
+        if (e == hipSuccess) e = run(xq, 0, kGateUp);
+        if (e == hipSuccess) e = launch_act_quant(h, h, (size_t)npairs * inter, st);
+        if (e == hipSuccess) e = run(xq, 0, kDown);
+    } else {
+        e = run((const uint16_t *)x, official, kBothParts);
     }
     if (e == hipSuccess && phase != 1) {
         const dim3 grid(ceil_div(dim, 256), t);

@@ -144,6 +144,32 @@ def test_moe_one_token_one_call_matches_two_phases(gpu, fmt, dim, inter, topk, o
         assert u.max() <= 1 and u.mean() < 0.02, (u.max(), u.mean())
 
 
+@pytest.mark.parametrize("fmt,sfmt,dim,inter", [(ops.FP4, ops.FP8_E8M0, 160, 96), (ops.FP4, ops.FP4, 1024, 544),
+                                                (ops.FP8, ops.FP8, 384, 256), (ops.FP8_E8M0, ops.FP8_E8M0, 96, 64)])
+@pytest.mark.parametrize("t", [2, 3, 16])
+def test_moe_official_activations_quantized_once(gpu, fmt, sfmt, dim, inter, t):
+    # several tokens in one call quantize x and the SwiGLU outputs once, the two-phase call quantizes them
+    # in registers in every workgroup: the same bits, with an infinity and NaNs in x (which reach whole
+    # tokens) and odd numbers of 32-blocks
+    n, topk = 6, 3
+    slots = [make_expert(fmt, dim, inter, seed=40 + i, gpu=gpu)[0] for i in range(n - 1)]
+    slots.append(make_expert(sfmt, dim, inter, seed=49, gpu=gpu)[0])
+    rng = np.random.default_rng(t + dim)
+    pick = [[int(v) for v in rng.choice(n - 1, size=topk, replace=False)] for _ in range(t)]
+    w = [list((rng.random(topk)).astype(np.float32)) for _ in range(t)]
+    x = data.activation(t, dim, seed=t) * torch.logspace(-3, 3, dim).to(torch.bfloat16)
+    x[0, 5], x[t - 1, dim - 1], x[t - 1, 40] = float("nan"), float("inf"), float("nan")
+    x = x.to(gpu)
+    kw = dict(shared=n - 1, limit=10.0, official=True, shared_fmt=sfmt)
+    y = ops.moe_experts(x, slots, pick, w, fmt, dim, inter, **kw)
+    work = torch.empty(ops.moe_work_bytes(t, topk, dim, inter), dtype=torch.uint8, device=gpu)
+    y2 = torch.full_like(y, 7.0)
+    for phase in (1, 2):
+        ops.moe_experts(x, slots, pick, w, fmt, dim, inter, work=work, out=y2, slot_ready=[i % 2 == 0 for i in range(n)],
+                        phase=phase, **kw)
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+
+
 @pytest.mark.parametrize("dim,inter", [(1024, 512), (7168, 2048)])
 def test_moe_token_classes_in_one_launch_match_one_token_calls(gpu, dim, inter):
     # four tokens whose experts take one, two and four tokens (the shared expert every token): the
