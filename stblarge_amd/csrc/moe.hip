@@ -128,23 +128,33 @@ __device__ __forceinline__ float post_scale(float lscale) {
 // the waves: the first lane holding each value's wave total writes red[wave][i]; after the barrier
 // thread i < N holds the total of value i in *out.
 template <int N>
-__device__ __forceinline__ bool wave_total(float (&vals)[N], float (*red)[N], float *out) {
-    constexpr int NV = pow2_at_least(N), kShift = 6 - log2_exact(NV);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    float p[NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++) p[i] = i < N ? vals[i] : 0.f;
-    const float mine = wave_sum_rows<NV>(p);
-    const int vi = lane >> kShift;
-    if ((lane & ((1 << kShift) - 1)) == 0 && vi < N) red[wave][vi] = mine;
+__device__ __forceinline__ bool waves_total(float (*red)[N], float *out) {
+    const int waves = blockDim.x >> 6, i = threadIdx.x;
     __syncthreads();
-    const int i = threadIdx.x;
     if (i >= N) return false;
     float acc = red[0][i];
     for (int v = 1; v < waves; v++) acc += red[v][i];
     *out = acc;
     return true;
 }
+
+template <int N>
+__device__ __forceinline__ bool wave_total(float (&vals)[N], float (*red)[N], float *out) {
+    constexpr int NV = pow2_at_least(N), kShift = 6 - log2_exact(NV);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float p[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) p[i] = i < N ? vals[i] : 0.f;
+    const float mine = wave_sum_rows<NV>(p);
+    const int vi = lane >> kShift;
+    if ((lane & ((1 << kShift) - 1)) == 0 && vi < N) red[wave][vi] = mine;
+    return waves_total<N>(red, out);
+}
+
+// Whether a job of M tokens sums each row over the wave as soon as its products are done, instead of the
+// whole tile's rows together: 4 tokens' tile would hold 32 sums next to 64 registers of x (the order of
+// a sum does not depend on how many are summed together: wave_sum_rows).
+constexpr bool row_sums(int M) { return M >= 4; }
 
 // The lane's products over its CPL chunks of 16 bytes (x words of chunk i: i * CH / 2 on), chunk by
 // chunk.
@@ -183,15 +193,14 @@ __device__ __forceinline__ void chunk_dot_lane(float (&s)[M], const u32x4 (&w)[C
 // nothing and add zeros.
 template <WFmt F, int M, int R, bool DW, int CPL = 1>
 __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &L, const uint16_t *__restrict__ x,
-                                           uint16_t *__restrict__ h, int dim, int inter, float limit, int official,
-                                           int tile0 = -1) {
+                                           uint16_t *__restrict__ h, int dim, int inter, float limit, int official) {
     static_assert(CPL == 1 || !WTraits<F>::fp4, "two chunks per lane: FP8 rows");
     constexpr int CH = WTraits<F>::CH * CPL;  // elements per lane
     const SlotMat<F> G(J.slot, L, 0, dim, inter), U(J.slot, L, 1, dim, inter);
     const int lane = threadIdx.x & 63, c = (threadIdx.x >> 6) * 64 + lane, nch = dim / CH;
     const bool active = c < nch;
     const int cc = active ? c : 0;
-    const int row0 = tile0 < 0 ? (int)blockIdx.x * R : tile0;  // the tile's first row
+    const int row0 = (int)blockIdx.x * R;  // the tile's first row
     const int m = J.m;
     // the output row and route weight of the (token, row) this thread may finish, read now: indexed
     // by thread they are memory loads, which at the end would add a round trip to every workgroup
@@ -199,9 +208,8 @@ __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &
     const int pair_out = J.pair[t_out];
     const float w_out = J.w[t_out];
     __shared__ float red[kMaxWaves][2 * M * R];
-    float tot[2 * M * R];
-#pragma unroll
-    for (int i = 0; i < 2 * M * R; i++) tot[i] = 0.f;
+    constexpr bool kRowwise = row_sums(M);
+    float tot[kRowwise ? 1 : 2 * M * R] = {};
     if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 64 < nch) {
         uint32_t xw[M][CH / 2];
 #pragma unroll
@@ -254,16 +262,30 @@ __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &
             chunk_dot_lane<F, M, CPL>(sgv, wg[r], xw, conv_scale<F>(sg[r], lg));
             chunk_dot_lane<F, M, CPL>(suv, wu[r], xw, conv_scale<F>(su[r], lu));
             const float a = post_scale<F>(lg), b = post_scale<F>(lu);
+            if constexpr (kRowwise) {
+                float row[2 * M];
 #pragma unroll
-            for (int t = 0; t < M; t++) {
-                tot[(t * R + r) * 2] = active ? sgv[t] * a : 0.f;
-                tot[(t * R + r) * 2 + 1] = active ? suv[t] * b : 0.f;
+                for (int t = 0; t < M; t++) row[2 * t] = active ? sgv[t] * a : 0.f, row[2 * t + 1] = active ? suv[t] * b : 0.f;
+                const float sum = wave_sum_rows<2 * M>(row);
+                constexpr int kShift = 6 - log2_exact(2 * M);
+                const int vi = lane >> kShift;
+                if ((lane & ((1 << kShift) - 1)) == 0) red[threadIdx.x >> 6][((vi >> 1) * R + r) * 2 + (vi & 1)] = sum;
+            } else {
+#pragma unroll
+                for (int t = 0; t < M; t++) {
+                    tot[(t * R + r) * 2] = active ? sgv[t] * a : 0.f;
+                    tot[(t * R + r) * 2 + 1] = active ? suv[t] * b : 0.f;
+                }
             }
         }
+    } else if constexpr (kRowwise) {
+        if (lane < 2 * M * R) red[threadIdx.x >> 6][lane] = 0.f;
     }
     // thread q = (t * R + r) * 2 + {0 gate, 1 up}; the even thread finishes the pair
     float v = 0.f;
-    const bool mine = wave_total<2 * M * R>(tot, red, &v);
+    bool mine;
+    if constexpr (kRowwise) mine = waves_total<2 * M * R>(red, &v);
+    else mine = wave_total<2 * M * R>(tot, red, &v);
     const float u = __shfl_down(v, 1, kWave);
     if (!mine || (threadIdx.x & 1)) return;
     const int q = threadIdx.x >> 1, t = q / R, r = q % R;
@@ -307,21 +329,20 @@ __global__ __launch_bounds__(512) void k_moe_gateup_mix(MoeTable<NJ> jobs, Exper
 // holding the unrounded sum when out_f32). DW as in k_moe_gateup.
 template <WFmt F, int M, int R, bool DW, int CPL = 1>
 __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L, const uint16_t *__restrict__ h,
-                                         void *__restrict__ o, int dim, int inter, int official, int out_f32,
-                                         int tile0 = -1) {
+                                         void *__restrict__ o, int dim, int inter, int official, int out_f32) {
     static_assert(CPL == 1 || !WTraits<F>::fp4, "two chunks per lane: FP8 rows");
     constexpr int CH = WTraits<F>::CH * CPL;  // elements per lane
     const SlotMat<F> D(J.slot, L, 2, dim, inter);
     const int lane = threadIdx.x & 63, c = (threadIdx.x >> 6) * 64 + lane, nch = inter / CH;
     const bool active = c < nch;
     const int cc = active ? c : 0;
-    const int row0 = tile0 < 0 ? (int)blockIdx.x * R : tile0;  // the tile's first row
+    const int row0 = (int)blockIdx.x * R;  // the tile's first row
     const int m = J.m;
     const int pair_out = J.pair[min((int)threadIdx.x / R, M - 1)];  // read early, as in gateup_job
     __shared__ float red[kMaxWaves][M * R];
-    float tot[M * R];
-#pragma unroll
-    for (int i = 0; i < M * R; i++) tot[i] = 0.f;
+    constexpr bool kRowwise = row_sums(M) && R % 2 == 0;
+    float tot[kRowwise ? 1 : M * R] = {};
+    float two[kRowwise ? 2 * M : 1] = {};  // two rows' values, summed together
     if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 64 < nch) {
         uint32_t xw[M][CH / 2];
 #pragma unroll
@@ -360,12 +381,29 @@ __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L,
             float s[M];
             chunk_dot_lane<F, M, CPL>(s, wd[r], xw, conv_scale<F>(sd[r], ld));
             const float a = post_scale<F>(ld);
+            if constexpr (kRowwise) {
 #pragma unroll
-            for (int t = 0; t < M; t++) tot[t * R + r] = active ? s[t] * a : 0.f;
+                for (int t = 0; t < M; t++) two[2 * t + (r & 1)] = active ? s[t] * a : 0.f;
+                if (r & 1) {
+                    const float sum = wave_sum_rows<2 * M>(two);
+                    constexpr int kShift = 6 - log2_exact(2 * M);
+                    const int vi = lane >> kShift;
+                    if ((lane & ((1 << kShift) - 1)) == 0) red[threadIdx.x >> 6][(vi >> 1) * R + r - 1 + (vi & 1)] = sum;
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < M; t++) tot[t * R + r] = active ? s[t] * a : 0.f;
+            }
         }
+    } else if constexpr (kRowwise) {
+        if (lane < M * R) red[threadIdx.x >> 6][lane] = 0.f;
     }
     float v = 0.f;
-    if (!wave_total<M * R>(tot, red, &v)) return;
+    if constexpr (kRowwise) {
+        if (!waves_total<M * R>(red, &v)) return;
+    } else {
+        if (!wave_total<M * R>(tot, red, &v)) return;
+    }
     const int t = threadIdx.x / R, r = threadIdx.x % R;
     if (t >= m || row0 + r >= dim) return;
     const size_t at = (size_t)pair_out * dim + row0 + r;
@@ -398,7 +436,7 @@ __global__ __launch_bounds__(512) void k_moe_down_mix(MoeTable<NJ> jobs, ExpertL
 // needs more registers than the one-token body alone, so a launch of one-token jobs only keeps
 // k_moe_gateup / k_moe_down.
 template <WFmt F, int R, bool DW, int NJ>
-__global__ __launch_bounds__(512) void k_moe_gateup_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_moe_gateup_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x,
                                                         uint16_t *__restrict__ h, int dim, int inter, float limit,
                                                         int official) {
     const MoeJob &J = jobs.j[blockIdx.y];
@@ -407,18 +445,12 @@ __global__ __launch_bounds__(512) void k_moe_gateup_any(MoeTable<NJ> jobs, Exper
     } else if (J.m == 2) {
         gateup_job<F, 2, R, DW>(J, L, x, h, dim, inter, limit, official);
     } else {
-        // the 4-token body in passes of one row (down: two rows), so that the kernel needs no more
-        // registers than for the 2-token body
-#pragma unroll 1
-        for (int p = 0; p < R; p++) {
-            if (p > 0) __syncthreads();  // the pass before has read its sums out of LDS
-            gateup_job<F, 4, 1, DW>(J, L, x, h, dim, inter, limit, official, (int)blockIdx.x * R + p);
-        }
+        gateup_job<F, 4, R, DW>(J, L, x, h, dim, inter, limit, official);
     }
 }
 
 template <WFmt F, int R, bool DW, int NJ>
-__global__ __launch_bounds__(512) void k_moe_down_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_moe_down_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
                                                       void *__restrict__ o, int dim, int inter, int official,
                                                       int out_f32) {
     const MoeJob &J = jobs.j[blockIdx.y];
@@ -427,11 +459,7 @@ __global__ __launch_bounds__(512) void k_moe_down_any(MoeTable<NJ> jobs, ExpertL
     } else if (J.m == 2) {
         down_job<F, 2, R, DW>(J, L, h, o, dim, inter, official, out_f32);
     } else {
-#pragma unroll 1
-        for (int p = 0; p < R / 2; p++) {
-            if (p > 0) __syncthreads();
-            down_job<F, 4, 2, DW>(J, L, h, o, dim, inter, official, out_f32, (int)blockIdx.x * R + 2 * p);
-        }
+        down_job<F, 4, R, DW>(J, L, h, o, dim, inter, official, out_f32);
     }
 }
 
