@@ -152,9 +152,9 @@ __device__ __forceinline__ bool wave_total(float (&vals)[N], float (*red)[N], fl
 }
 
 // Whether a job of M tokens sums each row over the wave as soon as its products are done, instead of the
-// whole tile's rows together: 4 tokens' tile would hold 32 sums next to 64 registers of x (the order of
-// a sum does not depend on how many are summed together: wave_sum_rows).
-constexpr bool row_sums(int M) { return M >= 4; }
+// whole tile's rows together: 4 tokens' tile would hold 32 sums next to 64 registers of x. (The order of
+// a sum does not depend on how many are summed together: wave_sum_rows.)
+constexpr bool row_sums(int M) { return M >= 3; }
 
 // The lane's products over its CPL chunks of 16 bytes (x words of chunk i: i * CH / 2 on), chunk by
 // chunk.
@@ -263,13 +263,14 @@ __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &
             chunk_dot_lane<F, M, CPL>(suv, wu[r], xw, conv_scale<F>(su[r], lu));
             const float a = post_scale<F>(lg), b = post_scale<F>(lu);
             if constexpr (kRowwise) {
-                float row[2 * M];
+                constexpr int NV = pow2_at_least(2 * M);
+                float row[NV] = {};
 #pragma unroll
                 for (int t = 0; t < M; t++) row[2 * t] = active ? sgv[t] * a : 0.f, row[2 * t + 1] = active ? suv[t] * b : 0.f;
-                const float sum = wave_sum_rows<2 * M>(row);
-                constexpr int kShift = 6 - log2_exact(2 * M);
+                const float sum = wave_sum_rows<NV>(row);
+                constexpr int kShift = 6 - log2_exact(NV);
                 const int vi = lane >> kShift;
-                if ((lane & ((1 << kShift) - 1)) == 0) red[threadIdx.x >> 6][((vi >> 1) * R + r) * 2 + (vi & 1)] = sum;
+                if ((lane & ((1 << kShift) - 1)) == 0 && vi < 2 * M) red[threadIdx.x >> 6][((vi >> 1) * R + r) * 2 + (vi & 1)] = sum;
             } else {
 #pragma unroll
                 for (int t = 0; t < M; t++) {
@@ -342,7 +343,8 @@ __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L,
     __shared__ float red[kMaxWaves][M * R];
     constexpr bool kRowwise = row_sums(M) && R % 2 == 0;
     float tot[kRowwise ? 1 : M * R] = {};
-    float two[kRowwise ? 2 * M : 1] = {};  // two rows' values, summed together
+    constexpr int NV = pow2_at_least(2 * M);
+    float two[kRowwise ? NV : 1] = {};  // two rows' values, summed together
     if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 64 < nch) {
         uint32_t xw[M][CH / 2];
 #pragma unroll
@@ -385,10 +387,13 @@ __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L,
 #pragma unroll
                 for (int t = 0; t < M; t++) two[2 * t + (r & 1)] = active ? s[t] * a : 0.f;
                 if (r & 1) {
-                    const float sum = wave_sum_rows<2 * M>(two);
-                    constexpr int kShift = 6 - log2_exact(2 * M);
+                    float sums[NV];
+#pragma unroll
+                    for (int i = 0; i < NV; i++) sums[i] = i < 2 * M ? two[i] : 0.f;
+                    const float sum = wave_sum_rows<NV>(sums);
+                    constexpr int kShift = 6 - log2_exact(NV);
                     const int vi = lane >> kShift;
-                    if ((lane & ((1 << kShift) - 1)) == 0) red[threadIdx.x >> 6][(vi >> 1) * R + r - 1 + (vi & 1)] = sum;
+                    if ((lane & ((1 << kShift) - 1)) == 0 && vi < 2 * M) red[threadIdx.x >> 6][(vi >> 1) * R + r - 1 + (vi & 1)] = sum;
                 }
             } else {
 #pragma unroll
@@ -429,35 +434,44 @@ __global__ __launch_bounds__(512) void k_moe_down_mix(MoeTable<NJ> jobs, ExpertL
 
 // ---- jobs of every token class in one launch --------------------------------------------------------
 
-// Jobs of 1, 2 and 3-4 tokens of one format in one gate/up and one down launch: each workgroup
+// Jobs of 1 to 4 tokens of one format in one gate/up and one down launch: each workgroup
 // takes its job's token class (workgroup-uniform). The few multi-token jobs of a step (the shared
 // expert, which every token takes; experts two tokens picked) then compute while the one-token jobs
 // stream, instead of running in launches of their own at a fraction of the bandwidth. The kernel
 // needs more registers than the one-token body alone, so a launch of one-token jobs only keeps
-// k_moe_gateup / k_moe_down.
-template <WFmt F, int R, bool DW, int NJ>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_moe_gateup_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x,
-                                                        uint16_t *__restrict__ h, int dim, int inter, float limit,
-                                                        int official) {
+// k_moe_gateup / k_moe_down, and one of one- and two-token jobs a kernel without the bodies of 3 and 4
+// (MANY). Those load x and all their rows once and sum row by row (row_sums): the tile in passes of one or
+// two rows, which needs 10 to 16 registers less, loads x (8 times a row's weights) again in every pass and
+// waits for each. 4 tokens, us: 7168 x 2048 top-8 126.3 -> 93.1, 5120 x 2304 top-6 86.3 -> 72.2 (3 tokens 71.1 ->
+// 58.7). Gate/up is held to 128 registers, 4 waves per SIMD; down is faster with its 138 (99.7 us against 106
+// at 7168 x 2048, before the 3-token bodies).
+template <WFmt F, int R, bool DW, bool MANY, int NJ>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_moe_gateup_any(
+    MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x, uint16_t *__restrict__ h, int dim, int inter,
+    float limit, int official) {
     const MoeJob &J = jobs.j[blockIdx.y];
     if (J.m == 1) {
         gateup_job<F, 1, R, DW>(J, L, x, h, dim, inter, limit, official);
-    } else if (J.m == 2) {
+    } else if (!MANY || J.m == 2) {
         gateup_job<F, 2, R, DW>(J, L, x, h, dim, inter, limit, official);
+    } else if (J.m == 3) {
+        gateup_job<F, 3, R, DW>(J, L, x, h, dim, inter, limit, official);
     } else {
         gateup_job<F, 4, R, DW>(J, L, x, h, dim, inter, limit, official);
     }
 }
 
-template <WFmt F, int R, bool DW, int NJ>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_moe_down_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
+template <WFmt F, int R, bool DW, bool MANY, int NJ>
+__global__ __launch_bounds__(512) void k_moe_down_any(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
                                                       void *__restrict__ o, int dim, int inter, int official,
                                                       int out_f32) {
     const MoeJob &J = jobs.j[blockIdx.y];
     if (J.m == 1) {
         down_job<F, 1, R, DW>(J, L, h, o, dim, inter, official, out_f32);
-    } else if (J.m == 2) {
+    } else if (!MANY || J.m == 2) {
         down_job<F, 2, R, DW>(J, L, h, o, dim, inter, official, out_f32);
+    } else if (J.m == 3) {
+        down_job<F, 3, R, DW>(J, L, h, o, dim, inter, official, out_f32);
     } else {
         down_job<F, 4, R, DW>(J, L, h, o, dim, inter, official, out_f32);
     }
@@ -686,17 +700,24 @@ static hipError_t launch_any(bool gateup, const MoeJobs &jobs, int n, const Expe
     const dim3 block(64 * ceil_div(k / WTraits<F>::CH, 64));
     // FP4 tiles whose scale rows are a multiple of 4 bytes fetch their scales as dwords
     const bool dw = WTraits<F>::fp4 && (k / 32) % 4 == 0;
+    bool many = false;
+    for (int j = 0; j < n; j++) many = many || jobs.j[j].m > 2;
     with_table<false>(jobs, n, [&](const auto &table) {
         constexpr int NJ = sizeof table / sizeof(MoeJob);
         const dim3 grid(gateup ? ceil_div(inter, 4) : ceil_div(dim, 8), n);
-        if (gateup && dw)
-            hipLaunchKernelGGL((k_moe_gateup_any<F, 4, WTraits<F>::fp4, NJ>), grid, block, 0, st, table, L, x, h, dim, inter, limit, official);
-        else if (gateup)
-            hipLaunchKernelGGL((k_moe_gateup_any<F, 4, false, NJ>), grid, block, 0, st, table, L, x, h, dim, inter, limit, official);
-        else if (dw)
-            hipLaunchKernelGGL((k_moe_down_any<F, 8, WTraits<F>::fp4, NJ>), grid, block, 0, st, table, L, h, o, dim, inter, official, out_f32);
-        else
-            hipLaunchKernelGGL((k_moe_down_any<F, 8, false, NJ>), grid, block, 0, st, table, L, h, o, dim, inter, official, out_f32);
+        auto go = [&](auto d, auto many) {
+            if (gateup)
+                hipLaunchKernelGGL((k_moe_gateup_any<F, 4, d(), many(), NJ>), grid, block, 0, st, table, L, x, h, dim, inter,
+                                   limit, official);
+            else
+                hipLaunchKernelGGL((k_moe_down_any<F, 8, d(), many(), NJ>), grid, block, 0, st, table, L, h, o, dim, inter,
+                                   official, out_f32);
+        };
+        using D = std::integral_constant<bool, WTraits<F>::fp4>;
+        if (dw && many) go(D(), std::true_type());
+        else if (dw) go(D(), std::false_type());
+        else if (many) go(std::false_type(), std::true_type());
+        else go(std::false_type(), std::false_type());
     });
     return hipGetLastError();
 }
