@@ -23,16 +23,11 @@
 // (column r of B); e4m3 operands hold K bytes [16g, 16g+16) and [64+16g, 64+16g+16) of the 128-K
 // step, e2m1 operands K elements [32g, 32g+32) (low nibble first); the lane's E8M0 scale covers K
 // block [32g, 32g+32); D lane l holds rows 4g..4g+3 of column r.
-#include <algorithm>
-
 #include "abi_util.hpp"
 #include "common.hpp"
+#include "gemm_plan.hpp"
 
 namespace stbl {
-
-constexpr int kGemmMaxM = 64;
-constexpr int kGemmMaxN = 1 << 20;
-constexpr int kGemmMaxRows = 8192;  // of stbl_amd_gemm_rows
 
 // ---- operand order --------------------------------------------------------------------------------
 
@@ -436,7 +431,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_one(const uint8_t *__restrict_
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
                 if constexpr (AARR) {  // operand order (k_act_quant_e4m3_ops): two contiguous kilobytes
-                    const uint8_t *blk = aq + (((size_t)((m0 >> 4) + mt) * KS + (kb >> 7)) * 2) * 1024 + lane * 16;
+                    const uint8_t *blk = aq + ops_block(operand_group(m0, mt, M), (int)(kb >> 7), KS, false) + lane * 16;
                     av[s][mt][0] = *(const u32x4 *)blk;
                     av[s][mt][1] = *(const u32x4 *)(blk + 1024);
                 } else {
@@ -846,7 +841,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_waves(const uint8_t *__restric
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const int row = min(m0 + 16 * mt + r, M - 1) - m0;
-        if (AARR) oa[mt] = (uint32_t)(min((m0 >> 4) + mt, (M - 1) >> 4) - (m0 >> 4)) * (uint32_t)KS * 2048u + lane * 16;
+        if (AARR) oa[mt] = (uint32_t)ops_block(operand_group(m0, mt, M) - (m0 >> 4), 0, KS, false) + lane * 16;
         else oa[mt] = (uint32_t)row * (uint32_t)K + 16 * g;
         osa[mt] = (uint32_t)row * (uint32_t)(act32 ? K >> 5 : KS);
     }
@@ -1016,81 +1011,6 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_waves(const uint8_t *__restric
     }
 }
 
-// Kernel, tile shape and split of K, chosen per shape (each choice measured fastest for its shape). Calls of
-// up to 64 rows:
-//   kOne64, k_gemm_one with 32 x 64 tiles on 4 waves of 4 steps, when K % 512 == 0, K <= 2048, m > 32
-//     and the tiles give >= 192 workgroups (7168 x 2048: 6.6 us);
-//   kOne32, k_gemm_one with 16 x 32 tiles on up to 8 waves of 8 steps (FP4 weights: 8.2 -> 7.9 us
-//     against 16 waves of 4, 8.9 with 4 waves of 16) or 16 waves of 4 steps (FP8), when K % 512 == 0,
-//     K <= 8192, m > 32 and the tiles give >= 192 workgroups (2048 x 7168: 11.7 -> 8.3 us against
-//     kSplit);
-//   kWaves24, k_gemm_waves with 32 x 64 tiles, when K <= 2048, m > 32 and these give >= 192 workgroups
-//     (unaligned scales or K % 512 != 0; 64 x 7168 x 1920: 7.6 us FP4, 8.3 FP8; with 16 waves of one
-//     step 7.6 and 9.6);
-//   kWaves22, k_gemm_waves with 32 x 32 tiles, for other K of up to kSplitSteps steps;
-//   kSplit otherwise, k_gemm with 64 x 64 tiles and 8 waves of one step each, K split into slices of <= 8
-//     steps, as many as it takes to give >= 200 workgroups (2048 x 7168: 7 slices, 224 workgroups),
-//     and k_gemm_reduce: with few tiles and many steps the waves of one workgroup are too few
-//     (64 x 512 x 4096: 9.7 us, 13.3 with k_gemm_waves; x 3072: 10.0 and 8.5; 10 x 2048 x 3584: 9.0 and 7.5).
-// Calls of more rows: kWaves22 while its 32 x 32 tiles give at most one workgroup per CU, kWaves24 up to
-// twice that (700 x 512 x 4096 FP8: 15.1 us, 19.2 with 32 x 32 and 20.8 with k_gemm_tile), then k_gemm_tile
-// with 64 x 64 tiles (kTile64) or, from one of those per CU on, 64 x 128 tiles on twice the waves (kTile128:
-// 600 x 2048 x 7168 31.4 -> 29.5 us, 1024 x 7168 x 2048 33.2 -> 31.1; 300 x 2048 x 7168 23.9 -> 27.6).
-enum GemmKernel { kSplit, kWaves22, kWaves24, kOne32, kOne64, kTile64, kTile128 };
-
-constexpr int kSplitSteps = 26;
-constexpr int kCUs = 256;
-
-struct GemmPlan {
-    GemmKernel kernel;
-    bool chain;  // how the call sums K (k_gemm_tile): steps in groups of `group`, chained or not
-    int group;
-    int slices;  // kSplit: of `group` steps
-};
-
-static int ceil_div(int a, int b) { return (a + b - 1) / b; }
-
-// aligned: the scale arrays are 16-byte aligned (k_gemm_one and chained sums load 4 steps' scales at once).
-// Rows of a call of more than 64 are summed as those of a call of 64, whatever the kernel.
-static GemmPlan gemm_plan(int fmt, int m, int n, int k, bool aligned) {
-    const int ks = k / 128, mc = std::min(m, kGemmMaxM);
-    GemmPlan p = {};
-    if (aligned && ks % 4 == 0 && ks <= 16 && mc > 32 && ceil_div(n, 64) * ceil_div(mc, 32) >= 192) {
-        p = {kOne64, true, 4, 1};
-    } else if (aligned && ks % 4 == 0 && ks <= 64 && mc > 32 && ceil_div(n, 32) * ceil_div(mc, 16) >= 192) {
-        p = {kOne32, true, fmt == 0 ? 8 : 4, 1};
-    } else if (ks <= 16 && mc > 32 && 2 * ceil_div(n, 64) >= 192) {
-        p = {kWaves24, false, 1, 1};
-    } else if (ks <= 16 && ceil_div(n, 32) >= 192) {
-        p = {kWaves22, false, 1, 1};
-    } else {
-        const int tiles = ceil_div(n, 64);
-        const int want = std::max(ceil_div(ks, 8), std::min(ks, ceil_div(200, tiles)));
-        p.group = ceil_div(ks, want), p.slices = ceil_div(ks, p.group);
-        p.kernel = ks > kSplitSteps ? kSplit : kWaves22;
-        if (p.slices == 1) p.group = 1;  // one running sum over the steps
-    }
-    if (m <= kGemmMaxM) return p;
-    const int64_t t32 = (int64_t)ceil_div(m, 32) * ceil_div(n, 32), t64 = (int64_t)ceil_div(m, 64) * ceil_div(n, 64);
-    p.kernel = t32 <= kCUs ? kWaves22 : t32 <= 2 * kCUs ? kWaves24 : t64 < kCUs ? kTile64 : kTile128;
-    return p;
-}
-
-static bool is_tile(const GemmPlan &p) { return p.kernel == kTile64 || p.kernel == kTile128; }
-
-static uint64_t a256(uint64_t v) { return (v + 255) & ~(uint64_t)255; }
-
-// Bytes the partial tiles of a call of up to 64 rows take at the front of `work`. The split of K does not
-// depend on m, and a call whose scale arrays are not 16-byte aligned may split where an aligned one does
-// not, so the size is that of the plan without alignment.
-static uint64_t part_reserve(int n, int k) {
-    const GemmPlan p = gemm_plan(0, 1, n, k, false);
-    return p.kernel == kSplit ? a256((uint64_t)ceil_div(n, 64) * p.slices * (4 * 4 * 64) * 16) : 0;
-}
-
-// Rows of the activation codes in the workspace: a whole number of 16-row groups (operand order).
-static uint64_t aq_bytes(int m, int k) { return a256((uint64_t)ceil_div(m, 16) * 16 * k); }
-
 // One GEMM call on quantized activations; arr: aq is in operand order (not for kSplit).
 struct GemmArgs {
     int fmt;
@@ -1138,15 +1058,15 @@ static hipError_t launch_waves(const GemmPlan &p, const GemmArgs &c) {
 
 template <bool FP4W, bool ARR, bool WOPS>
 static hipError_t launch_direct(const GemmPlan &p, const GemmArgs &c) {
-    if (p.kernel == kOne64) return launch_one<FP4W, 2, 4, 4, 1, ARR, WOPS>(c);
-    if (p.kernel == kOne32) return launch_one<FP4W, 1, 2, FP4W ? 8 : 16, FP4W ? 2 : 1, ARR, WOPS>(c);
-    if (p.kernel == kWaves24) return launch_waves<FP4W, 2, 4, ARR, WOPS>(p, c);
-    return launch_waves<FP4W, 2, 2, ARR, WOPS>(p, c);
+    if (p.kernel == kOne64) return launch_one<FP4W, tile_rows(kOne64) / 16, 4, 4, 1, ARR, WOPS>(c);
+    if (p.kernel == kOne32) return launch_one<FP4W, tile_rows(kOne32) / 16, 2, FP4W ? 8 : 16, FP4W ? 2 : 1, ARR, WOPS>(c);
+    if (p.kernel == kWaves24) return launch_waves<FP4W, tile_rows(kWaves24) / 16, 4, ARR, WOPS>(p, c);
+    return launch_waves<FP4W, tile_rows(kWaves22) / 16, 2, ARR, WOPS>(p, c);
 }
 
 template <bool FP4W, int BN, int WC, int S, bool WOPS>
 static hipError_t launch_tile(const GemmPlan &p, const GemmArgs &c, const uint8_t *as4, const uint8_t *ws4) {
-    constexpr int BM = 64, lds = S * (BM * 128 + BN * (FP4W ? 64 : 128) + BM * 4 + (FP4W ? BN * 4 : 0));
+    constexpr int BM = tile_rows(kTile64), lds = S * (BM * 128 + BN * (FP4W ? 64 : 128) + BM * 4 + (FP4W ? BN * 4 : 0));
     const int mt = ceil_div(c.m, BM), nt = ceil_div(c.n, BN);
 #define STBL_TILE(CHAIN)                                                                                              \
     hipLaunchKernelGGL((k_gemm_tile<FP4W, BM, BN, 2, WC, S, CHAIN, WOPS>), dim3((unsigned)mt * nt), dim3(2 * WC * 64),   \
@@ -1182,13 +1102,6 @@ static int check_gemm(const char *name, int fmt, const void *y, const void *code
     if (!aligned16(codes) || !aligned16(work)) return abi_fail(hipErrorInvalidValue, "%s: codes and work must be 16-byte aligned", name);
     if (wops && n % 16) return abi_fail(hipErrorInvalidValue, "%s: packed weights need n %% 16 == 0 (n=%d)", name, n);
     return 0;
-}
-
-// The workspace of a call of more than 64 rows: activation codes in operand order, then their scales (bytes
-// [m][k / block] for the kernels that read those, dwords [k / 128][m] for k_gemm_tile), then the FP4
-// weights' scale dwords.
-static uint64_t rows_work_bytes(int m, int n, int k) {
-    return aq_bytes(m, k) + a256((uint64_t)m * (k / 32)) + a256((uint64_t)n * (k / 32));
 }
 
 // Activations prepared into `work` as the plan's kernel reads them, then the GEMM. x: bf16, or (quantized) e4m3
@@ -1244,11 +1157,7 @@ using namespace stbl;
 
 extern "C" {
 
-uint64_t stbl_amd_gemm_work_bytes(int m, int n, int k) {
-    if (m < 1 || n < 1 || k < 128) return 256;
-    const uint64_t few = part_reserve(n, k) + aq_bytes(std::min(m, kGemmMaxM), k) + a256((uint64_t)std::min(m, kGemmMaxM) * (k / 32)) + 256;
-    return m > kGemmMaxM ? std::max(few, rows_work_bytes(m, n, k)) : few;
-}
+uint64_t stbl_amd_gemm_work_bytes(int m, int n, int k) { return gemm_work_bytes(m, n, k); }
 
 int stbl_amd_gemm_q(int fmt, void *y, const void *codes, const void *scales, const void *aq, const void *as, int m,
                     int n, int k, int act_block, int y_f32, void *work, hipStream_t st) {

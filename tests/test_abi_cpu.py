@@ -4,6 +4,7 @@ the ctypes table covers exactly that list, and argument checks fail before any d
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -150,3 +151,14 @@ def test_gemm_workspace_for_m_serves_every_smaller_m():
     for n, k in ((6100, 2048), (7168, 2048), (2048, 7168), (4096, 4096)):
         sizes = [lib.stbl_amd_gemm_work_bytes(m, n, k) for m in range(1, 65)]
         assert all(a <= b for a, b in zip(sizes, sizes[1:])), (n, k, sizes)
+
+
+def test_gemm_plans_read_inside_their_workspace(tmp_path):
+    # The tiles of a call read whole 16-row groups of activations from the workspace, which holds
+    # ceil(m / 16) of them: a 32-row tile whose second group is past the last one (m = 33..48, say) must
+    # not read it. The rules are host C++ (gemm_plan.hpp), and the group is the function the kernels call.
+    exe = str(tmp_path / "gemm_plan_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "stblarge_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "gemm_plan_check.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
