@@ -162,3 +162,39 @@ def test_gemm_plans_read_inside_their_workspace(tmp_path):
                     os.path.join(ROOT, "tests", "gemm_plan_check.cpp"), "-o", exe], check=True)
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+def test_route_to_host_waits_for_the_kernel_before_it_raises(monkeypatch):
+    # The router's kernel writes pinned buffers that only the call holds. An error recorded earlier on the
+    # thread makes the call raise although its kernel was launched: the buffers must not go back to the
+    # allocator before the stream is done with them.
+    import torch
+
+    from stblarge_amd import ops
+
+    events = []
+
+    class Stream:
+        cuda_stream = 0
+
+        def synchronize(self):
+            events.append("wait")
+
+    class Lib:
+        def stbl_amd_route(self, *args):
+            events.append("launch")
+            return 0
+
+    def check(status, what):
+        events.append("check")
+        raise _lib.StblError(what)
+
+    empty = torch.empty
+    monkeypatch.setattr(ops, "_need", lambda *a, **k: None)
+    monkeypatch.setattr(_lib, "load", Lib)
+    monkeypatch.setattr(_lib, "check", check)
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: empty(*a, **k))
+    with pytest.raises(_lib.StblError):
+        ops.route_to_host(torch.zeros((2, 8)), 2)
+    assert events == ["launch", "wait", "check"]
