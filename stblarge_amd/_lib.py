@@ -1,11 +1,14 @@
 """ctypes binding of libstbl_amd.so (the C ABI declared in include/stbl_amd.h).
 
 The library is loaded from the package directory, where stblarge_amd.build puts it. There is no
-fallback: if the library is missing, load() raises, and every op in stblarge_amd.ops fails loudly.
+fallback: if the library is missing, load() raises, and every op in stblarge_amd.ops fails loudly. (The
+compiled call path beside it, _bind.so, only makes calls cheaper; load() warns where it is missing.)
 """
 
 import ctypes
 import os
+import sys
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 # STBL_AMD_LIB names another build of the library (for comparing builds); default the in-tree one
@@ -95,15 +98,45 @@ SIGNATURES = {
 }
 
 _lib = None
-native = None  # the compiled call path of stblarge_amd.ops (csrc/bind.cpp), set by load()
+native = None  # the call path of stblarge_amd.ops (csrc/bind.cpp, or _PythonPath), set by load()
 
 
 class StblError(RuntimeError):
     pass
 
 
+def host_version():
+    """The Python and torch that run this, which the compiled call path has to be built for."""
+    import torch
+
+    return f"Python {sys.version_info.major}.{sys.version_info.minor} torch {torch.__version__}"
+
+
+class _PythonPath:
+    """In the place of the compiled call path: leaves every call to the wrappers of stblarge_amd.ops."""
+
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
+def _call_path(lib):
+    """The compiled call path bound to lib, or without one that fits a warning and _PythonPath."""
+    try:
+        from . import _bind
+
+        built_for = getattr(_bind, "built_for", "another version")
+        if built_for != host_version():
+            raise ImportError(f"built for {built_for}")
+    except ImportError as e:
+        warnings.warn(f"stblarge_amd/_bind.so cannot be used ({e}): calls take the slower Python path; build it "
+                      "with `python -m stblarge_amd.build`", RuntimeWarning, stacklevel=3)
+        return _PythonPath()
+    _bind.bind([ctypes.cast(getattr(lib, n), P).value for n in _bind.names()], StblError)
+    return _bind
+
+
 def load():
-    """The bound library (loaded once). Raises if it, or the compiled call path, was not built."""
+    """The bound library (loaded once). Raises if it was not built."""
     global _lib, native
     if _lib is None:
         if not os.path.exists(LIB_PATH):
@@ -117,12 +150,7 @@ def load():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        try:
-            from . import _bind
-        except ImportError as e:
-            raise StblError(f"stblarge_amd/_bind.so cannot be loaded ({e}): build it with `python -m stblarge_amd.build`") from e
-        _bind.bind([ctypes.cast(getattr(lib, n), P).value for n in _bind.names()], StblError)
-        native = _bind
+        native = _call_path(lib)
         _lib = lib
     return _lib
 

@@ -46,11 +46,13 @@ def bind_command(out):
 
     import torch
 
+    from . import _lib
+
     t = os.path.join(os.path.dirname(torch.__file__))
     rocm = os.path.dirname(os.path.dirname(HIPCC))
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DUSE_ROCM=1",
-            "-D__HIP_PLATFORM_AMD__=1", "-isystem", os.path.join(t, "include"), "-isystem",
+            "-D__HIP_PLATFORM_AMD__=1", f'-DSTBL_BUILT_FOR="{_lib.host_version()}"', "-isystem", os.path.join(t, "include"), "-isystem",
             sysconfig.get_paths()["include"], "-isystem", os.path.join(rocm, "include"),
             os.path.join(CSRC, "bind.cpp"), "-o", out, "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
             "-ltorch_python"]

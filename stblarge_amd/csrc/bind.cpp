@@ -474,4 +474,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_bind", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__bind() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__bind() {
+    PyObject *m = PyModule_Create(&module);
+    // the Python and torch of the build: both are used by their in-memory layouts, so _lib.py binds no other's
+    if (m && PyModule_AddStringConstant(m, "built_for", STBL_BUILT_FOR) < 0) Py_CLEAR(m);
+    return m;
+}

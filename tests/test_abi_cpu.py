@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -198,3 +199,32 @@ def test_route_to_host_waits_for_the_kernel_before_it_raises(monkeypatch):
     with pytest.raises(_lib.StblError):
         ops.route_to_host(torch.zeros((2, 8)), 2)
     assert events == ["launch", "wait", "check"]
+
+
+def _fresh_load(monkeypatch):
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "native", None)
+
+
+@pytest.mark.parametrize("how", ["missing", "other version"])
+def test_library_loads_without_the_compiled_call_path(monkeypatch, how):
+    # _bind.so only makes calls cheaper: without one that fits this Python and torch, load() warns and every
+    # wrapper of ops goes its own way
+    import stblarge_amd
+    from stblarge_amd import ops
+
+    _lib.load()
+    built = _lib.native
+    assert built.__name__ == "stblarge_amd._bind", "build the call path first: python -m stblarge_amd.build"
+    _fresh_load(monkeypatch)
+    if how == "missing":
+        monkeypatch.delattr(stblarge_amd, "_bind", raising=False)
+        monkeypatch.setitem(sys.modules, "stblarge_amd._bind", None)  # what an import of a missing one does
+    else:
+        monkeypatch.setattr(built, "built_for", "Python 3.0 torch 1.0", raising=False)
+    with pytest.warns(RuntimeWarning, match="_bind"):
+        lib = _lib.load()
+    assert lib.stbl_amd_version() >= 1
+    assert ops._native().gemv(ops.FP4, None, None, None, False, None) is NotImplemented
+    with pytest.raises(TypeError, match="codes must be a tensor"):
+        ops.gemv_fp4(None, None, None)
