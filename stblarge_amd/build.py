@@ -5,6 +5,7 @@ Run: python -m stblarge_amd.build   (or __graft_entry__.build()).
 """
 
 import os
+import shutil
 import subprocess
 import sys
 
@@ -39,6 +40,13 @@ def sources():
     return [os.path.join(CSRC, s) for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
 
 
+def rocm_home():
+    """The ROCm tree that HIPCC (a path or a bare name) belongs to."""
+    exe = shutil.which(HIPCC)
+    homes = [os.environ.get("ROCM_PATH"), exe and os.path.dirname(os.path.dirname(os.path.realpath(exe))), "/opt/rocm"]
+    return next((h for h in homes if h and os.path.isdir(os.path.join(h, "include", "hip"))), "/opt/rocm")
+
+
 def bind_command(out):
     """The g++ command for csrc/bind.cpp, against the torch and Python that run this. The HIP headers that
     torch's stream header includes ask the host compiler for their platform."""
@@ -48,28 +56,43 @@ def bind_command(out):
 
     from . import _lib
 
-    t = os.path.join(os.path.dirname(torch.__file__))
-    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    t = os.path.dirname(torch.__file__)
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
-    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DUSE_ROCM=1",
-            "-D__HIP_PLATFORM_AMD__=1", f'-DSTBL_BUILT_FOR="{_lib.host_version()}"', "-isystem", os.path.join(t, "include"), "-isystem",
-            sysconfig.get_paths()["include"], "-isystem", os.path.join(rocm, "include"),
-            os.path.join(CSRC, "bind.cpp"), "-o", out, "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
-            "-ltorch_python"]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-missing-field-initializers",
+            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+            f'-DSTBL_BUILT_FOR="{_lib.host_version()}"', "-isystem", os.path.join(t, "include"), "-isystem",
+            sysconfig.get_paths()["include"], "-isystem", os.path.join(rocm_home(), "include"),
+            os.path.join(CSRC, "bind.cpp"), "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_python", "-o", out]
+
+
+def build_bind(verbose=False):
+    """Compile the binding. The library works without it, so a failure (no g++, no torch headers) is only
+    reported, and an older binding, which may not fit the library, is removed."""
+    tmp = BIND + ".tmp"
+    try:
+        cmd = bind_command(tmp)
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.run(cmd, check=True)
+        os.replace(tmp, BIND)
+    except (ImportError, OSError, subprocess.CalledProcessError) as e:
+        if os.path.exists(BIND):
+            os.remove(BIND)
+        print(f"{BIND} was not built ({e}): calls will take the slower Python path", file=sys.stderr)
 
 
 def build(verbose=False):
-    """Compile every HIP source into one shared library, and the binding. Always recompiles."""
-    lib = [HIPCC, *FLAGS, "-I", CSRC, "-I", os.path.join(os.path.dirname(HERE), "include"), *sources(), "-o", LIB + ".tmp"]
-    jobs = []
-    for cmd, out in ((lib, LIB), (bind_command(BIND + ".tmp"), BIND)):
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        jobs.append((subprocess.Popen(cmd), cmd, out))
-    for job, cmd, out in jobs:
-        if job.wait():
-            raise subprocess.CalledProcessError(job.returncode, cmd)
-        os.replace(out + ".tmp", out)
+    """Compile every HIP source into one shared library, and beside it the binding. Always recompiles."""
+    tmp = LIB + ".tmp"
+    cmd = [HIPCC, *FLAGS, "-I", CSRC, "-I", os.path.join(os.path.dirname(HERE), "include"), *sources(), "-o", tmp]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    with subprocess.Popen(cmd) as job:  # leaving waits for it
+        build_bind(verbose)
+    if job.returncode:
+        raise subprocess.CalledProcessError(job.returncode, cmd)
+    os.replace(tmp, LIB)
     return LIB
 
 
