@@ -29,6 +29,7 @@
 #include "abi_util.hpp"
 #include "expert_layout.hpp"
 #include "gemv_core.hpp"
+#include "moe_plan.hpp"
 
 namespace stbl {
 
@@ -36,7 +37,6 @@ constexpr int kMoeMaxTok = 4;    // tokens per job
 constexpr int kMoeMaxJobs = 40;  // jobs per launch
 constexpr int kMoeMaxT = 16;     // tokens per MoE call
 constexpr int kMoeMaxPick = 17;  // top-k + shared
-constexpr int kQuantOnceTokens = 2;  // official numerics: tokens from which activations are quantized once
 
 struct MoeJob {
     const uint8_t *slot;
@@ -482,9 +482,7 @@ __global__ __launch_bounds__(512) void k_moe_down_any(MoeTable<NJ> jobs, ExpertL
 // out = the values that the gate/up and down kernels make of x in registers in official numerics
 // (act_quant_packed), 16 per thread; in place or not. With several tokens every workgroup of a job quantizes
 // its tokens' chunks again, which costs as much as a quarter of its products; quantized once, x and the
-// SwiGLU outputs cost two small launches instead (5120 x 2304, top-6 and an FP8 shared expert, us: 4 tokens 120.5
-// -> 92.3, 3 tokens 98.4 -> 79.0, 2 tokens 58.9 -> 55.6; one token, whose launches take 33.2 without any
-// quantization, keeps its 36.0).
+// SwiGLU outputs cost two small launches instead, which pays for large steps only (quantize_once).
 __global__ __launch_bounds__(256) void k_moe_act_quant(const uint16_t *x, uint16_t *out, int n16) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     const bool ok = i < n16;  // n16 is even: a block's two lanes are both in or both out
@@ -1049,7 +1047,10 @@ static int moe_experts_impl(int fmt, void *y, const void *x, int t, int dim, int
     if (nsjobs > 0 && fmt == EXPERT_FP4 && shared_fmt == EXPERT_FP8_E8M0)
         for (int i = 0; i < nsjobs; i++) jobs[njobs + i] = sjobs[i];
     hipError_t e;
-    if (official && phase == 0 && t >= kQuantOnceTokens) {
+    int64_t tokens = 0;  // of the jobs of several tokens
+    for (int j = 0; j < njobs; j++) tokens += jobs[j].m > 1 ? jobs[j].m : 0;
+    for (int j = 0; j < nsjobs; j++) tokens += sjobs[j].m > 1 ? sjobs[j].m : 0;
+    if (official && phase == 0 && t > 1 && quantize_once(fmt == EXPERT_FP4, tokens, dim, inter)) {
         // the quantized x waits in the output rows' memory, which only the down launches write (phases 1 and
         // 2 have outputs of each other there)
         uint16_t *xq = o;

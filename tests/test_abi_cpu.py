@@ -154,15 +154,24 @@ def test_gemm_workspace_for_m_serves_every_smaller_m():
         assert all(a <= b for a, b in zip(sizes, sizes[1:])), (n, k, sizes)
 
 
+def _run_check(name, tmp_path):
+    """Compiles tests/<name>.cpp against the headers of csrc and runs it."""
+    exe = str(tmp_path / name)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "stblarge_amd", "csrc"),
+                    os.path.join(ROOT, "tests", name + ".cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
+def test_moe_steps_quantize_where_that_is_faster(tmp_path):
+    _run_check("moe_plan_check", tmp_path)
+
+
 def test_gemm_plans_read_inside_their_workspace(tmp_path):
     # The tiles of a call read whole 16-row groups of activations from the workspace, which holds
     # ceil(m / 16) of them: a 32-row tile whose second group is past the last one (m = 33..48, say) must
     # not read it. The rules are host C++ (gemm_plan.hpp), and the group is the function the kernels call.
-    exe = str(tmp_path / "gemm_plan_check")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "stblarge_amd", "csrc"),
-                    os.path.join(ROOT, "tests", "gemm_plan_check.cpp"), "-o", exe], check=True)
-    r = subprocess.run([exe], capture_output=True, text=True)
-    assert r.returncode == 0, r.stdout
+    _run_check("gemm_plan_check", tmp_path)
 
 
 def test_route_to_host_waits_for_the_kernel_before_it_raises(monkeypatch):

@@ -144,14 +144,9 @@ def test_moe_one_token_one_call_matches_two_phases(gpu, fmt, dim, inter, topk, o
         assert u.max() <= 1 and u.mean() < 0.02, (u.max(), u.mean())
 
 
-@pytest.mark.parametrize("fmt,sfmt,dim,inter", [(ops.FP4, ops.FP8_E8M0, 160, 96), (ops.FP4, ops.FP4, 1024, 544),
-                                                (ops.FP8, ops.FP8, 384, 256), (ops.FP8_E8M0, ops.FP8_E8M0, 96, 64)])
-@pytest.mark.parametrize("t", [2, 3, 16])
-def test_moe_official_activations_quantized_once(gpu, fmt, sfmt, dim, inter, t):
-    # several tokens in one call quantize x and the SwiGLU outputs once, the two-phase call quantizes them
-    # in registers in every workgroup: the same bits, with an infinity and NaNs in x (which reach whole
-    # tokens) and odd numbers of 32-blocks
-    n, topk = 6, 3
+def _official_one_call_equals_two_phases(gpu, fmt, sfmt, dim, inter, t, n, topk):
+    # the two-phase call quantizes x and the SwiGLU outputs in registers in every workgroup: the same bits as
+    # one call's, with an infinity and NaNs in x (which reach whole tokens)
     slots = [make_expert(fmt, dim, inter, seed=40 + i, gpu=gpu)[0] for i in range(n - 1)]
     slots.append(make_expert(sfmt, dim, inter, seed=49, gpu=gpu)[0])
     rng = np.random.default_rng(t + dim)
@@ -168,6 +163,28 @@ def test_moe_official_activations_quantized_once(gpu, fmt, sfmt, dim, inter, t):
         ops.moe_experts(x, slots, pick, w, fmt, dim, inter, work=work, out=y2, slot_ready=[i % 2 == 0 for i in range(n)],
                         phase=phase, **kw)
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+
+
+@pytest.mark.parametrize("fmt,sfmt,dim,inter", [(ops.FP4, ops.FP8_E8M0, 160, 96), (ops.FP4, ops.FP4, 1024, 544),
+                                                (ops.FP8, ops.FP8, 384, 256), (ops.FP8_E8M0, ops.FP8_E8M0, 96, 64)])
+@pytest.mark.parametrize("t", [2, 3, 16])
+def test_moe_official_activations_of_small_steps(gpu, fmt, sfmt, dim, inter, t):
+    # steps below quantize_once's line, in registers in one call too; odd numbers of 32-blocks
+    _official_one_call_equals_two_phases(gpu, fmt, sfmt, dim, inter, t, 6, 3)
+
+
+@pytest.mark.parametrize("fmt,sfmt,dim,inter,t", [(ops.FP4, ops.FP8_E8M0, 2080, 544, 16), (ops.FP4, ops.FP4, 2080, 1056, 9),
+                                                  (ops.FP4, ops.FP8_E8M0, 5120, 2304, 2), (ops.FP8, ops.FP8, 2176, 1152, 16),
+                                                  (ops.FP8_E8M0, ops.FP8_E8M0, 2080, 1056, 16)])
+def test_moe_official_activations_quantized_once(gpu, fmt, sfmt, dim, inter, t):
+    # steps above the line (five of five experts a token, so every job holds several tokens), in launches of
+    # their own; odd numbers of 32-blocks, a partial last workgroup
+    n, topk = 6, 5
+    tokens, groups = t * (topk + 1), -(-dim // 2048) * -(-inter // 4) + -(-inter // 2048) * -(-dim // 8)
+    if t % 4 == 1:  # the last token of each expert is a job of its own
+        tokens -= topk + 1
+    assert tokens * groups >= (14000 if fmt == ops.FP4 else 50000)
+    _official_one_call_equals_two_phases(gpu, fmt, sfmt, dim, inter, t, n, topk)
 
 
 @pytest.mark.parametrize("dim,inter", [(1024, 512), (7168, 2048)])
