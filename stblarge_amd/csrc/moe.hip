@@ -566,33 +566,54 @@ __device__ __forceinline__ uint32_t wave_extreme(uint32_t v) {
     return pick(pick(lane(0), lane(16)), pick(lane(32), lane(48)));
 }
 
-// One wave per token; lane l holds experts l, l + 64, ... (NI of them) in registers. score = 1 / (1 +
-// exp(-logit)) (score_fn 0, the configuration's router) or sqrt(softplus(logit)) with softplus(l) = l
+// One wave per token; lane l holds experts l, l + 64, ... (NI of them) in registers. SPLIT: a workgroup per
+// token, whose waves take the experts' scores in turns and leave the top-k to the first (route_split). score = 1 /
+// (1 + exp(-logit)) (score_fn 0, the configuration's router) or sqrt(softplus(logit)) with softplus(l) = l
 // above 20, else log1p(exp(l)) (score_fn 1, stbl/kernels.cu:436-442); the top-k of score + bias (ties to the
 // lower expert id) by k rounds of a wave maximum over the lanes' best keys, where only a tie takes a
 // second reduction, over the ids; weight_i = score_i / (sum of the top-k scores in top-k order + 1e-20) *
 // route_scale. A NaN key ranks with -Inf (so a token with fewer than k numeric keys takes the lowest unused
-// ids next), and its weight comes out NaN. Bound by its chain of rounds: one token,
-// 32 experts, top-8 12.4 us with a workgroup argmax and two barriers a round, 3.0 so; 256 experts 12.0 -> 3.5, 4096 tokens of
-// them 37.1 -> 7.2.
-template <int NI>
+// ids next), and its weight comes out NaN. Bound by its chain of scores and rounds: one token, 256 experts,
+// top-8 11.4 us with a workgroup argmax and two barriers a round, 3.5 so; 8192 tokens of them 64 -> 9.1; 512
+// experts with sqrt(softplus), one token, top-8 15.0 -> 4.4, top-1 3.7 -> 3.1 (5.1 in one wave).
+template <int NI, bool SPLIT>
 __global__ __launch_bounds__(256) void k_route(const float *__restrict__ logits, const float *__restrict__ bias, int t,
                                                int n_exp, int topk, float route_scale, int score_fn,
                                                int *__restrict__ ids, float *__restrict__ weights,
                                                float *__restrict__ scores) {
-    const int tok = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int tok = SPLIT ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
     if (tok >= t) return;  // the whole wave
-    float l[NI], sc[NI];
-    uint32_t key[NI];
+    constexpr int kParts = SPLIT ? 4 : 1, kMine = NI / kParts;
+    float l[kMine], sc[NI];
 #pragma unroll
-    for (int i = 0; i < NI; i++) l[i] = logits[(size_t)tok * n_exp + min(lane + 64 * i, n_exp - 1)];
+    for (int i = 0; i < kMine; i++)
+        l[i] = logits[(size_t)tok * n_exp + min(lane + 64 * (kParts * i + (SPLIT ? wave : 0)), n_exp - 1)];
+    __shared__ float all[SPLIT ? 64 * NI : 1];
+#pragma unroll
+    for (int i = 0; i < kMine; i++) {
+        const int e = lane + 64 * (kParts * i + (SPLIT ? wave : 0));
+        if (NI > 4 && e - lane >= n_exp) {  // the wave's whole part is past the last expert
+            if constexpr (!SPLIT) sc[i] = 0.f;
+            continue;
+        }
+        const float s = score_fn == 1 ? sqrt_softplus(l[i]) : __fdiv_rn(1.f, 1.f + expf(-l[i]));
+        if (scores && e < n_exp) scores[(size_t)tok * n_exp + e] = s;
+        if constexpr (SPLIT) all[e] = s;
+        else sc[i] = s;
+    }
+    if constexpr (SPLIT) {
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int i = 0; i < NI; i++) sc[i] = all[lane + 64 * i];
+    }
+    uint32_t key[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int e = lane + 64 * i;
-        sc[i] = score_fn == 1 ? sqrt_softplus(l[i]) : __fdiv_rn(1.f, 1.f + expf(-l[i]));
         const float v = sc[i] + (bias ? bias[min(e, n_exp - 1)] : 0.f);
         key[i] = e < n_exp ? float_order(v != v ? -INFINITY : v) : 0;
-        if (scores && e < n_exp) scores[(size_t)tok * n_exp + e] = sc[i];
     }
     float sum = 0.f, mine = 0.f;
     int mine_id = 0;
@@ -1169,12 +1190,17 @@ int stbl_amd_route(const float *logits, const float *bias, int t, int n_exp, int
     if (!logits || !ids || !weights || t < 1 || n_exp < 1 || n_exp > 1024 || topk < 1 || topk > 32 || topk > n_exp)
         return abi_fail(hipErrorInvalidValue, "route: need 1 <= topk <= min(32, n_exp), n_exp <= 1024");
     if (score_fn != 0 && score_fn != 1) return abi_fail(hipErrorInvalidValue, "route: score_fn must be 0 (sigmoid) or 1 (sqrt-softplus)");
-#define STBL_ROUTE(NI)                                                                                             \
-    hipLaunchKernelGGL(k_route<NI>, dim3(ceil_div(t, 4)), dim3(256), 0, st, logits, bias, t, n_exp, topk, route_scale, \
-                       score_fn, ids, weights, scores)
-    if (n_exp <= 64) STBL_ROUTE(1);
-    else if (n_exp <= 256) STBL_ROUTE(4);
-    else STBL_ROUTE(16);
+#define STBL_ROUTE(NI, SPLIT)                                                                                       \
+    hipLaunchKernelGGL((k_route<NI, SPLIT>), dim3(SPLIT ? t : ceil_div(t, 4)), dim3(256), 0, st, logits, bias, t, n_exp, \
+                       topk, route_scale, score_fn, ids, weights, scores)
+    const bool split = route_split(n_exp, t, score_fn);
+    if (n_exp <= 64) STBL_ROUTE(1, false);
+    else if (n_exp <= 256 && split) STBL_ROUTE(4, true);
+    else if (n_exp <= 256) STBL_ROUTE(4, false);
+    else if (n_exp <= 512 && split) STBL_ROUTE(8, true);
+    else if (n_exp <= 512) STBL_ROUTE(8, false);
+    else if (split) STBL_ROUTE(16, true);
+    else STBL_ROUTE(16, false);
 #undef STBL_ROUTE
     return abi_status(hipGetLastError(), "route launch");
 }

@@ -1,5 +1,4 @@
-// How an MoE step in official numerics quantizes its activations: plain host C++, so that the rule can be
-// checked without a GPU.
+// Rules of an MoE step: plain host C++, so that they can be checked without a GPU.
 #pragma once
 
 #include <cstdint>
@@ -23,6 +22,17 @@ inline bool quantize_once(bool fp4, int64_t tokens, int dim, int inter) {
     const int64_t gate_up = (int64_t)((dim + 2047) / 2048) * ((inter + 3) / 4);
     const int64_t down = (int64_t)((inter + 2047) / 2048) * ((dim + 7) / 8);
     return tokens * (gate_up + down) >= (fp4 ? 14000 : 50000);
+}
+
+// Whether the router takes a workgroup a token, whose four waves share the scores, instead of a wave (k_route).
+// Few tokens leave the GPU idle, and a wave's scores then take longer than its top-k: from 5 a lane on, or
+// from 2 with the longer sqrt(softplus) (score_fn 1). Many tokens fill it either way, and three of
+// the four waves only wait. A wave -> a workgroup, us, top-1:
+//   1 token:      384 experts 2.9 -> 2.5, with sqrt(softplus) 4.4 -> 3.2; 1024 8.7 -> 4.5; 256 3.3 -> 2.4
+//   2048 tokens:  384 experts 3.6 -> 3.7, with sqrt(softplus) 5.8 -> 5.6; 1024 11.7 -> 10.3; 256 (1024 tokens) 4.0 -> 3.7
+//   8192 tokens:  384 experts 6.4 -> 7.7, with sqrt(softplus) 12.5 -> 13.5; 256 9.0 -> 11.9
+inline bool route_split(int n_exp, int t, int score_fn) {
+    return n_exp > 256 ? t <= 2048 : n_exp > 64 && score_fn == 1 && t <= 1024;
 }
 
 }  // namespace stbl

@@ -1,4 +1,4 @@
-// moe_plan.hpp's rule at measured steps: in registers where that was faster, in launches of their own where those were.
+// moe_plan.hpp's rules at measured sizes: the way that was faster.
 #include <cstdio>
 
 #include "moe_plan.hpp"
@@ -17,6 +17,17 @@ int main() {
     for (const auto &s : steps)
         if (stbl::quantize_once(s.fp4, s.tokens, s.dim, s.inter) != s.once) {
             printf("fp4 %d, %d tokens, %d x %d: not %d\n", s.fp4, s.tokens, s.dim, s.inter, s.once);
+            return 1;
+        }
+    const struct {
+        int n_exp, t, score_fn;
+        bool split;
+    } routers[] = {{64, 1, 1, false},   {128, 1, 0, false},   {128, 1, 1, true},    {256, 1, 1, true},    {256, 1024, 1, true},
+                   {256, 2048, 1, false}, {257, 1, 0, true},  {384, 2, 1, true},    {512, 1024, 0, true}, {1024, 2048, 1, true},
+                   {384, 8192, 0, false}, {1024, 8192, 1, false}};
+    for (const auto &r : routers)
+        if (stbl::route_split(r.n_exp, r.t, r.score_fn) != r.split) {
+            printf("router of %d experts, %d tokens, score %d: not %d\n", r.n_exp, r.t, r.score_fn, r.split);
             return 1;
         }
     return 0;

@@ -163,7 +163,7 @@ def _run_check(name, tmp_path):
     assert r.returncode == 0, r.stdout
 
 
-def test_moe_steps_quantize_where_that_is_faster(tmp_path):
+def test_moe_rules_take_the_faster_way(tmp_path):
     _run_check("moe_plan_check", tmp_path)
 
 

@@ -625,6 +625,24 @@ def test_route_random(gpu):
         check_route(np_(ids), np_(w), sc, oids, ow, bias)
 
 
+@pytest.mark.parametrize("e", [64, 65, 256, 257, 320, 512, 513, 1000, 1024])
+@pytest.mark.parametrize("fn", [0, 1])
+def test_route_waves_and_workgroups(gpu, e, fn):
+    # a wave a token, or a workgroup whose waves share the scores: each side of route_split's lines, experts
+    # at and past whole registers and parts; ids, weights and scores
+    for t in (1, 5, 1024, 1025, 2048, 2049):
+        topk = min(e, 32) if t == 5 else 8
+        lg = np.random.default_rng(e + t).normal(0, 3.0, (t, e)).astype(np.float32)
+        lg[0, ::7] = np.nan
+        bias = np.random.default_rng(e).normal(0, 0.01, e).astype(np.float32)
+        ids, w, sc = ops.route(torch.from_numpy(lg).to(gpu), topk, torch.from_numpy(bias).to(gpu), 2.5, want_scores=True, score_fn=fn)
+        osc, oids, ow = oracle.route(lg, topk, bias, 2.5, score_fn=fn)
+        check_route(np_(ids), np_(w), osc, oids, ow, bias)
+        num = ~np.isnan(osc)
+        assert np.array_equal(np.isnan(np_(sc)), ~num)
+        assert np.max(np.abs(np_(sc)[num] - osc[num])) <= 1e-6 * np.max(np.abs(osc[num]))
+
+
 def test_route_nan_logits(gpu):
     # NaN keys rank below every number (the oracle's rule): a token with fewer than k numeric keys
     # takes the lowest unused ids next, and NaN scores make its weights NaN
