@@ -153,7 +153,9 @@ __device__ __forceinline__ bool wave_total(float (&vals)[N], float (*red)[N], fl
 
 // Whether a job of M tokens sums each row over the wave as soon as its products are done, instead of the
 // whole tile's rows together: 4 tokens' tile would hold 32 sums next to 64 registers of x. (The order of
-// a sum does not depend on how many are summed together: wave_sum_rows.)
+// a sum does not depend on how many are summed together: wave_sum_rows.) Launches of one job, which leave
+// registers idle, keep the tile (row by row -> tile, us: one FP4 expert, 3 tokens, 7168 x 2048 13.8 -> 13.5, 1664 x
+// 2432 9.45 -> 9.35; four jobs of 3 tokens 5120 x 2304 39.3 -> 41.4).
 constexpr bool row_sums(int M) { return M >= 3; }
 
 // The lane's products over its CPL chunks of 16 bytes (x words of chunk i: i * CH / 2 on), chunk by
@@ -191,7 +193,7 @@ __device__ __forceinline__ void chunk_dot_lane(float (&s)[M], const u32x4 (&w)[C
 // The body runs in any workgroup of at least ceil(dim / CH / 64) waves: waves past the job's K (in
 // the mixed-format launches, whose workgroups are sized for the format with the most waves) load
 // nothing and add zeros.
-template <WFmt F, int M, int R, bool DW, int CPL = 1>
+template <WFmt F, int M, int R, bool DW, int CPL = 1, bool ROWS = row_sums(M)>
 __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &L, const uint16_t *__restrict__ x,
                                            uint16_t *__restrict__ h, int dim, int inter, float limit, int official) {
     static_assert(CPL == 1 || !WTraits<F>::fp4, "two chunks per lane: FP8 rows");
@@ -208,7 +210,7 @@ __device__ __forceinline__ void gateup_job(const MoeJob &J, const ExpertLayout &
     const int pair_out = J.pair[t_out];
     const float w_out = J.w[t_out];
     __shared__ float red[kMaxWaves][2 * M * R];
-    constexpr bool kRowwise = row_sums(M);
+    constexpr bool kRowwise = ROWS;
     float tot[kRowwise ? 1 : 2 * M * R] = {};
     if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 64 < nch) {
         uint32_t xw[M][CH / 2];
@@ -303,7 +305,7 @@ template <WFmt F, int M, int R, bool DW, int NJ>
 __global__ __launch_bounds__(512) void k_moe_gateup(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ x,
                                                     uint16_t *__restrict__ h, int dim, int inter, float limit,
                                                     int official) {
-    gateup_job<F, M, R, DW>(jobs.j[NJ == 1 ? 0 : blockIdx.y], L, x, h, dim, inter, limit, official);
+    gateup_job<F, M, R, DW, 1, row_sums(M) && NJ != 1>(jobs.j[NJ == 1 ? 0 : blockIdx.y], L, x, h, dim, inter, limit, official);
 }
 
 // Jobs of two formats in one launch (the reference's FP4 routed experts next to its FP8 E8M0 shared
@@ -328,7 +330,7 @@ __global__ __launch_bounds__(512) void k_moe_gateup_mix(MoeTable<NJ> jobs, Exper
 
 // Job blockIdx.y, rows [row0, row0 + R) of down. h bf16 [P][inter] -> o [P][dim] (bf16, or fp32
 // holding the unrounded sum when out_f32). DW as in k_moe_gateup.
-template <WFmt F, int M, int R, bool DW, int CPL = 1>
+template <WFmt F, int M, int R, bool DW, int CPL = 1, bool ROWS = row_sums(M)>
 __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L, const uint16_t *__restrict__ h,
                                          void *__restrict__ o, int dim, int inter, int official, int out_f32) {
     static_assert(CPL == 1 || !WTraits<F>::fp4, "two chunks per lane: FP8 rows");
@@ -341,7 +343,7 @@ __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L,
     const int m = J.m;
     const int pair_out = J.pair[min((int)threadIdx.x / R, M - 1)];  // read early, as in gateup_job
     __shared__ float red[kMaxWaves][M * R];
-    constexpr bool kRowwise = row_sums(M) && R % 2 == 0;
+    constexpr bool kRowwise = ROWS && R % 2 == 0;
     float tot[kRowwise ? 1 : M * R] = {};
     constexpr int NV = pow2_at_least(2 * M);
     float two[kRowwise ? NV : 1] = {};  // two rows' values, summed together
@@ -419,7 +421,7 @@ __device__ __forceinline__ void down_job(const MoeJob &J, const ExpertLayout &L,
 template <WFmt F, int M, int R, bool DW, int NJ>
 __global__ __launch_bounds__(512) void k_moe_down(MoeTable<NJ> jobs, ExpertLayout L, const uint16_t *__restrict__ h,
                                                   void *__restrict__ o, int dim, int inter, int official, int out_f32) {
-    down_job<F, M, R, DW>(jobs.j[NJ == 1 ? 0 : blockIdx.y], L, h, o, dim, inter, official, out_f32);
+    down_job<F, M, R, DW, 1, row_sums(M) && NJ != 1>(jobs.j[NJ == 1 ? 0 : blockIdx.y], L, h, o, dim, inter, official, out_f32);
 }
 
 // Down rows of jobs of two formats in one launch, as k_moe_gateup_mix.
