@@ -15,7 +15,9 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
+#include <initializer_list>
 #include <vector>
 
 namespace {
@@ -63,7 +65,7 @@ struct Lib {
 
 PyObject *other() { Py_RETURN_NOTIMPLEMENTED; }
 
-// A plain tensor (no subclass), or null.
+// A plain tensor or parameter (no other subclass), or null.
 const Tensor *tensor(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
 
 // A contiguous strided device tensor of type `dt`, of `dims` dimensions if that is not 0, or null.
@@ -129,6 +131,19 @@ bool failed(int status, const char *what) {
     return true;
 }
 
+// A tuple of tensors, or null with an error set.
+PyObject *tuple(std::initializer_list<const Tensor *> ts) {
+    THPObjectPtr all(PyTuple_New((Py_ssize_t)ts.size()));
+    if (!all) return nullptr;
+    Py_ssize_t i = 0;
+    for (const Tensor *t : ts) {
+        PyObject *o = THPVariable_Wrap(*t);
+        if (!o) return nullptr;
+        PyTuple_SET_ITEM(all.get(), i++, o);
+    }
+    return all.release();
+}
+
 #define CALL(status, ...)               \
     do {                                \
         Py_BEGIN_ALLOW_THREADS;         \
@@ -189,25 +204,20 @@ PyObject *gemv_batch(PyObject *, PyObject *const *a, Py_ssize_t) {
             y[i] = ptr(*yi);
         }
     }
-    PyObject *ys = a[5];
-    if (given) {
-        Py_INCREF(ys);
-    } else {
-        if (!(ys = PyList_New(n))) return nullptr;
-        for (Py_ssize_t i = 0; i < n; i++) {
-            const Tensor t = empty({m, rows}, out_type(f32), *first);
-            y[i] = ptr(t);
-            PyList_SET_ITEM(ys, i, THPVariable_Wrap(t));
-        }
+    THPObjectPtr ys(given ? Py_NewRef(a[5]) : PyList_New(n));  // freed with its tensors if one cannot be allocated
+    if (!ys) return nullptr;
+    for (Py_ssize_t i = 0; i < n && !given; i++) {
+        const Tensor t = empty({m, rows}, out_type(f32), *first);
+        PyObject *o = THPVariable_Wrap(t);
+        if (!o) return nullptr;
+        y[i] = ptr(t);
+        PyList_SET_ITEM(ys.get(), i, o);
     }
     int st;
     const P sp = stream();
     CALL(st, lib.gemv_batch[fmt](y, c, s, x, (int)n, (int)m, (int)rows, (int)k, f32, sp));
-    if (failed(st, "gemv_batch")) {
-        Py_DECREF(ys);
-        return nullptr;
-    }
-    return ys;
+    if (failed(st, "gemv_batch")) return nullptr;
+    return ys.release();
     END_HANDLE_TH_ERRORS
 }
 
@@ -338,11 +348,7 @@ PyObject *route(PyObject *, PyObject *const *a, Py_ssize_t) {
     const P pl = ptr(*l), pb = bias ? ptr(*bias) : nullptr, pi = ptr(ids), pw = ptr(w), s = stream();
     CALL(st, lib.route(pl, pb, (int)t, (int)e, topk, scale, fn, pi, pw, nullptr, s));
     if (failed(st, "route")) return nullptr;
-    PyObject *i = THPVariable_Wrap(ids), *v = THPVariable_Wrap(w);
-    PyObject *both = i && v ? PyTuple_Pack(2, i, v) : nullptr;
-    Py_XDECREF(i);
-    Py_XDECREF(v);
-    return both;
+    return tuple({&ids, &w});
     END_HANDLE_TH_ERRORS
 }
 
@@ -397,12 +403,7 @@ PyObject *act_quant(PyObject *, PyObject *const *a, Py_ssize_t) {
     const P px = ptr(*x), pc = ptr(codes), ps = ptr(scales), pd = want ? ptr(deq) : nullptr, s = stream();
     CALL(st, lib.act_quant(px, (int)rows, (int)n, block, pow2, pc, ps, pd, s));
     if (failed(st, "act_quant")) return nullptr;
-    PyObject *all = PyTuple_New(want ? 3 : 2);
-    if (!all) return nullptr;
-    PyTuple_SET_ITEM(all, 0, THPVariable_Wrap(codes));
-    PyTuple_SET_ITEM(all, 1, THPVariable_Wrap(scales));
-    if (want) PyTuple_SET_ITEM(all, 2, THPVariable_Wrap(deq));
-    return all;
+    return want ? tuple({&codes, &scales, &deq}) : tuple({&codes, &scales});
     END_HANDLE_TH_ERRORS
 }
 
@@ -419,11 +420,7 @@ PyObject *act_quant_e4m3(PyObject *, PyObject *const *a, Py_ssize_t) {
     const P px = ptr(*x), pc = ptr(codes), ps = ptr(scales), s = stream();
     CALL(st, lib.act_quant_e4m3(px, (int)rows, (int)k, block, pc, ps, s));
     if (failed(st, "act_quant_e4m3")) return nullptr;
-    PyObject *all = PyTuple_New(2);
-    if (!all) return nullptr;
-    PyTuple_SET_ITEM(all, 0, THPVariable_Wrap(codes));
-    PyTuple_SET_ITEM(all, 1, THPVariable_Wrap(scales));
-    return all;
+    return tuple({&codes, &scales});
     END_HANDLE_TH_ERRORS
 }
 
