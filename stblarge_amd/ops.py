@@ -520,10 +520,11 @@ def route_to_host(logits, topk, bias=None, route_scale=1.0, score_fn=SCORE_SIGMO
     if bias is not None:
         _need(bias, torch.float32, "bias", 1)
     stream = torch.cuda.current_stream()
-    status = _lib.load().stbl_amd_route(_ptr(logits), _ptr(bias), t, e, topk, float(route_scale), int(score_fn), _ptr(ids),
-                                        _ptr(w), None, P(stream.cuda_stream))
-    stream.synchronize()  # also before an error is raised: nothing but this call keeps the buffers
-    _lib.check(status, "route")
+    try:
+        _lib.check(_lib.load().stbl_amd_route(_ptr(logits), _ptr(bias), t, e, topk, float(route_scale), int(score_fn),
+                                              _ptr(ids), _ptr(w), None, P(stream.cuda_stream)), "route")
+    finally:
+        stream.synchronize()  # also when an error is raised: nothing but this call keeps the buffers
     return ids.tolist(), w.tolist()
 
 
