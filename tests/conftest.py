@@ -26,3 +26,22 @@ def gpu():
         pytest.skip("no GPU")
     import torch
     return torch.device("cuda:0")
+
+
+@pytest.fixture(scope="session")
+def gemm_plan(tmp_path_factory):
+    """(kernel, chained, steps of a group) of a GEMM call, from the rules the library is built with."""
+    import ctypes
+    import subprocess
+
+    lib = str(tmp_path_factory.mktemp("plan") / "gemm_plan.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "stblarge_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "gemm_plan_check.cpp"), "-o", lib], check=True)
+    fn = ctypes.CDLL(lib).gemm_plan_of
+    kernels = ("split", "waves22", "waves24", "one32", "one64", "tile64", "tile128")
+
+    def plan(fmt, m, n, k, aligned=True):
+        out = (ctypes.c_int * 3)()
+        fn(fmt, m, n, k, int(aligned), out)
+        return kernels[out[0]], bool(out[1]), out[2]
+    return plan

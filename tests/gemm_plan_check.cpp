@@ -1,6 +1,7 @@
 // gemm_plan.hpp's rules against each other, over both formats, aligned and unaligned scales, every m up to 64
 // and larger ones around whole tiles: no tile reads an activation group that the workspace does not hold, and
-// the parts of the workspace fit its size. Prints the first call that breaks a rule.
+// the parts of the workspace fit its size. Prints the first call that breaks a rule. Built as a library, it
+// tells the GPU tests which kernel a call takes.
 #include <cstdio>
 
 #include "gemm_plan.hpp"
@@ -19,6 +20,12 @@ static int check(int fmt, int m, int n, int k, bool aligned) {
     if (front + codes + scales > gemm_work_bytes(m, n, k)) broken = "workspace too small";
     if (broken) printf("%s: kernel %d, fmt %d, %d x %d x %d, aligned %d\n", broken, p.kernel, fmt, m, n, k, aligned);
     return broken ? 1 : 0;
+}
+
+// Per call: the kernel (GemmKernel), whether sums chain, and the steps of a group.
+extern "C" void gemm_plan_of(int fmt, int m, int n, int k, int aligned, int *out) {
+    const GemmPlan p = gemm_plan(fmt, m, n, k, aligned != 0);
+    out[0] = p.kernel, out[1] = p.chain, out[2] = p.group;
 }
 
 int main() {

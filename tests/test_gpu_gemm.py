@@ -76,8 +76,8 @@ def test_gemm_fp8(gpu, m, n, k):
 
 @pytest.mark.parametrize("fmt", [0, 1])
 def test_gemm_more_than_64_rows(gpu, fmt):
-    # M = 150 runs as launches of 64, 64 and 22 rows (ref/kernel.py's GEMMs take any M): against the
-    # oracle, and each 64-row block equal to a call on those rows alone, gemm and gemm_q alike
+    # M = 150 in one call (ref/kernel.py's GEMMs take any M): against the oracle, and each 64-row block, here
+    # also the last 22 rows, equal to a call on those rows alone, gemm and gemm_q alike
     m, n, k = 150, 1024, 2048
     w = data.weight(n, k, seed=91 + fmt)
     q, deq = (oracle.quant_fp4, oracle.dequant_fp4) if fmt == 0 else (oracle.quant_fp8_b128, oracle.dequant_fp8_b128)
@@ -162,11 +162,10 @@ def test_gemm_deterministic_and_work_reuse(gpu):
 @pytest.mark.parametrize("m,n,k,shift", [(16, 7168, 2048, False), (22, 7168, 2048, False), (40, 7168, 2048, False),
                                          (40, 2048, 7168, False), (64, 7168, 2048, True)])
 def test_gemm_tile_plans(gpu, fmt, block, m, n, k, shift):
-    # each tile plan of the GEMM against the oracle: 64 x 32 tiles in one slice (m <= 32 at N >= 6144,
-    # also the 22-row tail of a 150-row call), one-launch 32 x 64 tiles with a partial second row
-    # group (40 rows at 7168x2048), one-launch 16 x 32 tiles with a partial third group (40 rows at
-    # 2048x7168), and two 32-row groups of 64-column tiles when the activation scales are not
-    # 16-byte aligned (the one-launch plans load them 16 bytes at a time)
+    # each tile plan of the GEMM against the oracle: k_gemm_waves with 32 x 32 tiles (m <= 32 at 7168 x 2048),
+    # k_gemm_one with 32 x 64 tiles and a partial second row group (40 rows at 7168 x 2048) and with 16 x
+    # 32 tiles and a partial third group (40 rows at 2048 x 7168), and k_gemm_waves with 32 x 64 tiles when
+    # the activation scales are not 16-byte aligned (k_gemm_one loads them 16 bytes at a time)
     w = data.weight(n, k, seed=n + k + m)
     q, deq = (oracle.quant_fp4, oracle.dequant_fp4) if fmt == 0 else (oracle.quant_fp8_b128, oracle.dequant_fp8_b128)
     codes, scales = q(w.numpy())
@@ -232,8 +231,8 @@ def test_gemm_pack_layout(gpu, fmt, n, k):
                                          (16, 7168, 2048, False), (37, 208, 384, False), (64, 7168, 2048, True),
                                          (150, 1024, 2048, False)])
 def test_gemm_packed_matches_row_major(gpu, fmt, block, m, n, k, shift):
-    # every tile plan (one-launch 16 x 32 and 32 x 64 tiles, 64 x 32 tiles in one slice, split K,
-    # two 32-row groups for unaligned activation scales, 64-row launches) reads packed weights to the
+    # every tile plan of few rows (k_gemm_one with 16 x 32 and 32 x 64 tiles, k_gemm_waves with 32 x 32 and, for
+    # unaligned activation scales, 32 x 64 ones, split K) and a call of 150 rows read packed weights to the
     # same outputs bit for bit, and so against the oracle as the row-major call is checked
     if fmt == 1 and block == 32:
         pytest.skip("FP8 weights pair with act_block 128 in the reference configuration")
@@ -270,17 +269,28 @@ def test_gemm_pack_refuses_bad_shapes(gpu):
         ops.gemm_q_packed(w, s, aq, a_s, 0)
 
 
+def _shifted(t, by):
+    """t's values `by` bytes past an aligned address."""
+    buf = torch.zeros(t.numel() + 16, dtype=t.dtype, device=t.device)
+    return buf[by:by + t.numel()].view(t.shape).copy_(t)
+
+
 @pytest.mark.parametrize("fmt,block", [(0, 32), (0, 128), (1, 128)])
-@pytest.mark.parametrize("m,n,k,shift", [(65, 16, 128, 0), (70, 2048, 7168, 0), (129, 208, 384, 0), (257, 515, 640, 0),
-                                         (300, 2048, 1024, 0), (200, 2050, 2176, 0), (640, 512, 4096, 0),
-                                         (1000, 1040, 512, 0), (321, 6160, 1536, 0), (260, 1664, 2048, 1),
-                                         (8200, 64, 256, 0)])
-def test_gemm_many_rows_equal_64_row_calls(gpu, fmt, block, m, n, k, shift):
-    # one call on many rows against calls on 64 of them, bit for bit on every whole 64 rows: 32 x 32 and
-    # 32 x 64 tiles of waves, 64 x 64 and 64 x 128 tiles through LDS (their counts cross one and two per
-    # CU), partial tiles in both directions, groups of 1 to 8 steps, chained or not, scales that are not
-    # 16-byte aligned, N that is no multiple of 8 (element stores), and more rows than a call takes; the
+@pytest.mark.parametrize("m,n,k,shift,kernel", [
+    (65, 16, 128, 0, "waves22"), (70, 2048, 7168, 0, "waves22"), (129, 208, 384, 0, "waves22"), (257, 515, 640, 0, "waves22"),
+    (300, 2048, 1024, 0, "tile64"), (200, 2050, 2176, 0, "waves24"), (640, 512, 4096, 0, "waves24"),
+    (1000, 1040, 512, 0, "tile128"), (321, 6160, 1536, 0, "tile128"), (260, 1664, 2048, 1, "waves24"), (8200, 64, 256, 0, "waves24"),
+    # the tile kernels with element stores (N % 8 = 2), an odd number of steps in unchained groups of 3, scales off
+    # 16 bytes, and fewer steps than stages
+    (300, 2050, 2176, 0, "tile64"), (600, 2050, 2176, 0, "tile128"), (300, 2050, 2176, 1, "tile64"),
+    (1000, 1040, 128, 0, "tile128"), (300, 2048, 384, 0, "tile64"), (330, 2056, 256, 1, "tile64")])
+def test_gemm_many_rows_equal_64_row_calls(gpu, gemm_plan, fmt, block, m, n, k, shift, kernel):
+    # one call on many rows against calls on 64 of them, bit for bit on every whole 64 rows (of 8200 rows, more
+    # than a call takes, on six blocks): 32 x 32 and 32 x 64 tiles of waves, 64 x 64 and 64 x 128 tiles through LDS (their
+    # counts cross one and two per CU), partial tiles in both directions, groups of 1 to 8 steps, chained or
+    # not, activation scales that are not 16-byte aligned, N that is no multiple of 8 (element stores); the
     # first, last and some middle rows against the oracle
+    assert gemm_plan(fmt, min(m, 8192), n, k, not shift)[0] == kernel
     w = data.weight(n, k, seed=n + k + m)
     q, deq = (oracle.quant_fp4, oracle.dequant_fp4) if fmt == 0 else (oracle.quant_fp8_b128, oracle.dequant_fp8_b128)
     codes, scales = q(w.numpy())
@@ -288,18 +298,68 @@ def test_gemm_many_rows_equal_64_row_calls(gpu, fmt, block, m, n, k, shift):
     dc, ds, xg = torch.from_numpy(codes).to(gpu), torch.from_numpy(scales).to(gpu), x.to(gpu)
     aq, a_s = ops.act_quant_e4m3(xg, block)
     if shift:
-        buf = torch.zeros(a_s.numel() + 16, dtype=a_s.dtype, device=gpu)
-        a_s = buf[shift:shift + a_s.numel()].view(a_s.shape).copy_(a_s)
+        a_s = _shifted(a_s, shift)
     y32 = ops.gemm_q(dc, ds, aq, a_s, fmt, block, out_f32=True)
-    whole = min(m, 640) // 64 * 64
-    want = torch.cat([ops.gemm_q(dc, ds, aq[r:r + 64], a_s[r:r + 64], fmt, block, out_f32=True) for r in range(0, whole, 64)])
-    assert torch.equal(y32[:whole], want)
+    for r in range(0, m // 64 * 64, 64) if m <= 1024 else (0, 64, 4096, 5056, 8064, 8128):
+        assert torch.equal(y32[r:r + 64], ops.gemm_q(dc, ds, aq[r:r + 64], a_s[r:r + 64], fmt, block, out_f32=True)), r
     rows = sorted({0, 63, m // 2, m - 2, m - 1})
     _check(np_(y32)[rows], np_(ops.gemm_q(dc, ds, aq, a_s, fmt, block))[rows], _oracle_gemm(x[rows], deq(codes, scales), block))
     if not shift:
         assert torch.equal(ops.gemm(dc, ds, xg, fmt, block, out_f32=True), y32)
     if n % 16 == 0:
         assert torch.equal(ops.gemm_q_packed(ops.gemm_pack(dc, fmt), ds, aq, a_s, fmt, block, out_f32=True), y32)
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [(100, 2048, 512, "waves22"), (300, 2048, 1024, "tile64"), (600, 2064, 640, "tile128")])
+def test_gemm_weight_scales_off_16_bytes(gpu, gemm_plan, m, n, k, kernel):
+    # FP4 weight scales that start one byte off: k_gemm_prep reads them byte by byte, the waves' kernel as single
+    # bytes; the sums are those of a call of 64 rows on the same scales
+    assert gemm_plan(0, m, n, k, False)[0] == kernel
+    codes, scales = oracle.quant_fp4(data.weight(n, k, seed=m).numpy())
+    x = data.activation(m, k, seed=m + 1)
+    dc, ds, xg = torch.from_numpy(codes).to(gpu), _shifted(torch.from_numpy(scales).to(gpu), 1), x.to(gpu)
+    y32 = ops.gemm(dc, ds, xg, 0, 128, out_f32=True)
+    for r in range(0, m // 64 * 64, 64):
+        assert torch.equal(y32[r:r + 64], ops.gemm(dc, ds, xg[r:r + 64], 0, 128, out_f32=True)), r
+    rows = [0, m // 2, m - 1]
+    _check(np_(y32)[rows], np_(ops.gemm(dc, ds, xg, 0, 128))[rows], _oracle_gemm(x[rows], oracle.dequant_fp4(codes, scales), 128))
+    assert torch.equal(ops.gemm_packed(ops.gemm_pack(dc, 0), ds, xg, 0, 128, out_f32=True), y32)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("m,n,k,kernel", [(40, 512, 640, "waves22"), (200, 512, 1024, "waves22"), (200, 2048, 640, "waves24"),
+                                          (300, 2048, 1024, "tile64"), (1000, 1040, 640, "tile128")])
+def test_gemm_non_finite_rows(gpu, gemm_plan, fmt, m, n, k, kernel):
+    # an infinity in a row makes all its outputs NaN, a NaN none (test_gemm_non_finite_activations); every other row
+    # keeps its bits in the kernels of waves and the tile kernels
+    assert gemm_plan(fmt, m, n, k)[0] == kernel
+    codes, scales = (oracle.quant_fp4 if fmt == 0 else oracle.quant_fp8_b128)(data.weight(n, k, seed=7).numpy())
+    dc, ds = torch.from_numpy(codes).to(gpu), torch.from_numpy(scales).to(gpu)
+    x = data.activation(m, k, seed=8).to(gpu)
+    clean = ops.gemm(dc, ds, x, fmt, 128, out_f32=True)
+    x[0, 5], x[m // 2, k - 1], x[m - 1, 200] = float("inf"), float("-inf"), float("inf")
+    x[1, 7], x[m - 2, k - 2] = float("nan"), float("nan")
+    aq, a_s = ops.act_quant_e4m3(x, 128)
+    other = torch.ones(m, dtype=torch.bool, device=gpu)
+    other[[0, 1, m // 2, m - 2, m - 1]] = False
+    for y in (ops.gemm(dc, ds, x, fmt, 128, out_f32=True), ops.gemm_q(dc, ds, aq, a_s, fmt, 128, out_f32=True)):
+        assert y[[0, m // 2, m - 1]].isnan().all() and y[[1, m - 2]].isfinite().all()
+        assert torch.equal(y[other], clean[other])
+
+
+@pytest.mark.parametrize("fmt,block", [(0, 32), (0, 128), (1, 128)])
+@pytest.mark.parametrize("m", [33, 40, 48, 49])
+def test_gemm_32_row_tiles_past_the_last_group(gpu, gemm_plan, fmt, block, m):
+    # k_gemm_one's second tile of 32 rows with one group of 16 rows in the call, or two: the quantized activations
+    # in operand order (gemm) give the bits of those in rows (gemm_q)
+    n, k = 7168, 2048
+    assert gemm_plan(fmt, m, n, k)[0] == "one64"
+    codes, scales = (oracle.quant_fp4 if fmt == 0 else oracle.quant_fp8_b128)(data.weight(n, k, seed=9).numpy())
+    dc, ds, x = torch.from_numpy(codes).to(gpu), torch.from_numpy(scales).to(gpu), data.activation(m, k, seed=m).to(gpu)
+    aq, a_s = ops.act_quant_e4m3(x, block)
+    want = ops.gemm_q(dc, ds, aq, a_s, fmt, block, out_f32=True)
+    assert torch.equal(ops.gemm(dc, ds, x, fmt, block, out_f32=True), want)
+    assert torch.equal(ops.gemm_packed(ops.gemm_pack(dc, fmt), ds, x, fmt, block, out_f32=True), want)
 
 
 @pytest.mark.parametrize("fmt,block", [(0, 32), (0, 128), (1, 128)])
