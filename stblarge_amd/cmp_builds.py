@@ -9,8 +9,8 @@ moves work between lanes, waves or workgroups must leave every output bit unchan
 Both builds must report the same stbl_amd_version() (the same ABI). Runs on one GPU in seconds; the
 inputs are seeded, random and bf16-valued where the path needs it. Outputs start as NaN (ids as -1),
 and a case that either build rejects (a recorded stbl_amd_last_error, or a v2 status other than 0)
-counts as a difference, so two rejected calls never compare equal. Prints each differing case and
-exits 1 if any output differs.
+counts as a difference, so two rejected calls never compare equal; a case whose entry point one build does
+not have is named and left out. Prints each differing case and exits 1 if any output differs.
 """
 
 import ctypes
@@ -52,7 +52,8 @@ def _out(shape, dev, dtype=torch.float32):
 
 
 def _cases(dev, seed):
-    """(name, function(lib) -> list of output tensors) for one seed."""
+    """(name, function(lib) -> list of output tensors[, an entry point that an older build may lack]) for one
+    seed."""
     g = torch.Generator(device=dev)
     g.manual_seed(seed)
     st = None
@@ -189,6 +190,31 @@ def _cases(dev, seed):
         assert lib.stbl_amd_gemm(ops.FP4, _p(y), _p(gc), _p(gs), _p(xg), 64, 2048, 7168, 32, 1, _p(work), st) == 0
         return [y]
     cases.append(("gemm fp4 m=64", gemm))
+
+    # GEMMs of many rows in one call (tiles of waves, 64 x 64 and 64 x 128 tiles), and an expert into its slot
+    for fmt, m, n, k, quantized in ((ops.FP4, 100, 2048, 1024, True), (ops.FP8, 300, 2048, 7168, False), (ops.FP4, 1024, 7168, 2048, False)):
+        codes, scales = (ops.quant_fp4 if fmt == ops.FP4 else ops.quant_fp8_b128)(data.weight(n, k, seed + 3, dev))
+        xr = bf((m, k))
+        aq, a_s = ops.act_quant_e4m3(xr, 128)
+
+        def rows_(lib, fmt=fmt, m=m, n=n, k=k, quantized=quantized, codes=codes, scales=scales, xr=xr, aq=aq, a_s=a_s):
+            y = _out((m, n), dev)
+            work = torch.empty(int(lib.stbl_amd_gemm_work_bytes(m, n, k)), dtype=torch.uint8, device=dev)
+            if quantized:
+                assert lib.stbl_amd_gemm_q_rows(fmt, 0, _p(y), _p(codes), _p(scales), _p(aq), _p(a_s), m, n, k, 128, 1, _p(work), st) == 0
+            else:
+                assert lib.stbl_amd_gemm_rows(fmt, 0, _p(y), _p(codes), _p(scales), _p(xr), m, n, k, 128, 1, _p(work), st) == 0
+            return [y]
+        name = "gemm_q_rows" if quantized else "gemm_rows"
+        cases.append((f"{name} fmt {fmt} {m}x{n}x{k}", rows_, f"stbl_amd_{name}"))
+    for fmt in (ops.FP4, ops.FP8, ops.FP8_E8M0):
+        ws = [data.weight(r, k, seed + 4 + i, dev) for i, (r, k) in enumerate(((640, 1152), (640, 1152), (1152, 640)))]
+
+        def slot_(lib, fmt=fmt, ws=ws):
+            slot = torch.zeros(ops.expert_layout(fmt, 1152, 640)[0], dtype=torch.uint8, device=dev)
+            assert lib.stbl_amd_quant_expert(fmt, _p(slot), *[_p(w) for w in ws], 1152, 640, st) == 0
+            return [slot]
+        cases.append((f"quant_expert fmt {fmt} 1152x640", slot_, "stbl_amd_quant_expert"))
     return cases
 
 
@@ -214,7 +240,11 @@ def compare(new, old, seeds=3):
     dev = torch.device("cuda", torch.cuda.current_device())
     bad = []
     for seed in range(seeds):
-        for name, fn in _cases(dev, seed):
+        for name, fn, *needs in _cases(dev, seed):
+            without = [who for who, lib in (("new", new), ("old", old)) if not all(hasattr(lib, n) for n in needs)]
+            if without:
+                print(f"{name} seed {seed}: not in the {' and '.join(without)} build", flush=True)
+                continue
             a, b = _run(fn, new), _run(fn, old)
             if a is None or b is None:
                 who = " and ".join(w for w, r in (("the new build", a), ("the old build", b)) if r is None)

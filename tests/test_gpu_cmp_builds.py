@@ -80,3 +80,21 @@ def test_rejected_case_is_reported(gpu):
     bad = cmp_builds.compare(a, b, seeds=1)
     assert [n for n, _ in bad] == ["stbl_gemv_mxfp4 2304x5120 seed 0", "stbl_gemv_mxfp4 5120x2304 seed 0"]
     assert all(r == "rejected by the new build and the old build" for _, r in bad)
+
+
+def test_case_of_a_missing_entry_point_is_left_out(gpu, capsys):
+    # an older build without the many-row GEMMs: those cases are named, not compared
+    _lib.load()
+
+    class Older:
+        def __init__(self, lib):
+            self._lib = lib
+
+        def __getattr__(self, attr):
+            if attr.endswith("_rows"):
+                raise AttributeError(attr)
+            return getattr(self._lib, attr)
+
+    assert cmp_builds.compare(_lib.LIB_PATH, Older(cmp_builds._load(_lib.LIB_PATH)), seeds=1) == []
+    out = capsys.readouterr().out
+    assert out.count("not in the old build") == 3 and "gemm_rows fmt 1 300x2048x7168" in out
