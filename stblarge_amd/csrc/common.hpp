@@ -113,13 +113,6 @@ __device__ __forceinline__ uint32_t f32_to_e4m3(float x) {
     return sign | (uint32_t)(((E + 7) << 3) | (qi - 8));
 }
 
-// e2m1 value table (ref/kernel.py:14-16).
-__device__ __forceinline__ float e2m1_value(uint32_t c) {
-    const uint32_t m = c & 7u;
-    const float mag = m < 4 ? 0.5f * (float)m : (m < 6 ? (float)(m - 2) : (m == 6 ? 4.0f : 6.0f));
-    return (c & 8u) ? -mag : mag;
-}
-
 // ---- wave reductions -----------------------------------------------------------------------------
 
 __device__ __forceinline__ float wave_sum(float v) {

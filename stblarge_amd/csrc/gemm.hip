@@ -173,104 +173,95 @@ __global__ __launch_bounds__(256) void k_gemm_pack(const uint8_t *__restrict__ c
     *(u32x4 *)(packed + 16 * t) = *(const u32x4 *)(codes + src);
 }
 
-// One workgroup owns a 16 MT x 16 NT output tile (MT m-tiles x NT n-tiles of 16 x 16) and a slice of up
-// to NW 128-K steps; wave w takes step w of the slice for all MT * NT tiles, loading its activations and
-// weights straight from global memory (no operand is shared between waves, so nothing is staged
-// through LDS), from addresses clamped into the buffers; a step past the slice gets zero operands
-// instead of a branch. The waves' tiles are summed through LDS in wave order, the workgroup writes its
-// slice's partial tile, and k_gemm_reduce adds the slices in order. (Summing the slices in the last
-// workgroup to finish needs an agent-scope release/acquire per workgroup, which writes back and
-// invalidates the XCD's L2 each time: measured at about 4x the whole GEMM, so the kernel boundary is
-// the synchronization point.) A rows are K bytes apart. Partial tiles and the LDS sum hold f32x4 q = t *
-// 64 + lane with t = m-tile * NT + n-tile.
-template <bool FP4W, int MT, int NT, int NW, bool WOPS>
-__global__ __launch_bounds__(NW * 64) void k_gemm(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
-                                                  const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,
-                                                  f32x4 *__restrict__ part, int M, int N, int K, int act_shift,
-                                                  int ntiles, int slices, int steps_wg) {
-    constexpr int SW = 1;
-    constexpr int kTileVecs = MT * NT * 64;
-    constexpr int kThreads = NW * 64;
+// One workgroup owns a 64 x 64 output tile (MT m-tiles x NT n-tiles of 16 x 16) and a slice of up to NW 128-K
+// steps; wave w takes step w of the slice for all MT * NT tiles, loading its activations and weights
+// straight from global memory (no operand is shared between waves, so nothing is staged through LDS),
+// from addresses clamped into the buffers; a step past the slice gets zero operands instead of a
+// branch. The waves' tiles are summed through LDS in wave order, the workgroup writes its slice's partial
+// tile, and k_gemm_reduce adds the slices in order. (Summing the slices in the last workgroup to finish
+// needs an agent-scope release/acquire per workgroup, which writes back and invalidates the XCD's L2 each
+// time: measured at about 4x the whole GEMM, so the kernel boundary is the synchronization point.) A
+// rows are K bytes apart. Partial tiles and the LDS sum hold f32x4 q = t * 64 + lane with t = m-tile * NT +
+// n-tile.
+template <bool FP4W, bool WOPS>
+__global__ __launch_bounds__(512) void k_gemm(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
+                                              const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,
+                                              f32x4 *__restrict__ part, int M, int N, int K, int act_shift, int ntiles,
+                                              int slices, int steps_wg) {
+    constexpr int MT = 4, NT = 4, NW = 8, kTileVecs = MT * NT * 64, kThreads = NW * 64;
     __shared__ f32x4 red[NW * kTileVecs];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
     const int tile = blockIdx.x % ntiles, slice = blockIdx.x / ntiles;
     const int n0 = tile * 16 * NT, KS = K >> 7;
-    const int s0 = slice * steps_wg + wave;
-    const int nst = max(0, min(1, min(KS, (slice + 1) * steps_wg) - s0));  // wave-uniform
+    const int step = slice * steps_wg + wave;
+    const bool live = step < min(KS, (slice + 1) * steps_wg);  // wave-uniform
 
-    // 1. loads: lane (r, g) holds, per step, rows 16 mt + r of A and columns n0 + 16 nt + r of W
-    u32x4 av[SW][MT][2];
-    uint32_t asc[SW][MT];
-    u32x4 bv[SW][NT][FP4W ? 1 : 2];
-    uint32_t bsc[SW][NT];
-    float wsc[SW];
+    // 1. loads: lane (r, g) holds rows 16 mt + r of A and columns n0 + 16 nt + r of W
+    u32x4 av[MT][2];
+    uint32_t asc[MT];
+    u32x4 bv[NT][FP4W ? 1 : 2];
+    uint32_t bsc[NT];
+    const size_t kb = (size_t)(live ? step : 0) * 128;
 #pragma unroll
-    for (int s = 0; s < SW; s++) {
-        const size_t kb = (size_t)(s < nst ? s0 + s : 0) * 128;
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const int m = min(16 * mt + r, M - 1);
-            const uint8_t *row = aq + (size_t)m * K + kb;
-            av[s][mt][0] = *(const u32x4 *)(row + 16 * g);
-            av[s][mt][1] = *(const u32x4 *)(row + 64 + 16 * g);
-            asc[s][mt] = as_[(size_t)m * (K >> act_shift) + ((kb + 32 * g) >> act_shift)];
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            const int n = min(n0 + 16 * nt + r, N - 1);
-            if constexpr (WOPS) {  // operand order: one contiguous kilobyte (two for FP8) per load
-                const uint8_t *blk = wc + ops_block(min((n0 >> 4) + nt, (N >> 4) - 1), (int)(kb >> 7), KS, FP4W) + 16 * lane;
-                bv[s][nt][0] = *(const u32x4 *)blk;
-                if constexpr (!FP4W) bv[s][nt][1] = *(const u32x4 *)(blk + 1024);
-                if constexpr (FP4W) bsc[s][nt] = ((const uint8_t *)ws)[(size_t)n * (K >> 5) + (kb >> 5) + g];
-            } else if constexpr (FP4W) {
-                bv[s][nt][0] = *(const u32x4 *)(wc + (size_t)n * (K >> 1) + (kb >> 1) + 16 * g);
-                bsc[s][nt] = ((const uint8_t *)ws)[(size_t)n * (K >> 5) + (kb >> 5) + g];
-            } else {
-                const uint8_t *row = wc + (size_t)n * K + kb;
-                bv[s][nt][0] = *(const u32x4 *)(row + 16 * g);
-                bv[s][nt][1] = *(const u32x4 *)(row + 64 + 16 * g);
-            }
-        }
-        if constexpr (!FP4W) wsc[s] = ((const float *)ws)[(size_t)(n0 >> 7) * KS + (kb >> 7)];
+    for (int mt = 0; mt < MT; mt++) {
+        const int m = min(16 * mt + r, M - 1);
+        const uint8_t *row = aq + (size_t)m * K + kb;
+        av[mt][0] = *(const u32x4 *)(row + 16 * g);
+        av[mt][1] = *(const u32x4 *)(row + 64 + 16 * g);
+        asc[mt] = as_[(size_t)m * (K >> act_shift) + ((kb + 32 * g) >> act_shift)];
     }
-    // 2. MFMAs, 4 NT independent accumulators per step
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        const int n = min(n0 + 16 * nt + r, N - 1);
+        if constexpr (WOPS) {  // operand order: one contiguous kilobyte (two for FP8) per load
+            const uint8_t *blk = wc + ops_block(min((n0 >> 4) + nt, (N >> 4) - 1), (int)(kb >> 7), KS, FP4W) + 16 * lane;
+            bv[nt][0] = *(const u32x4 *)blk;
+            if constexpr (!FP4W) bv[nt][1] = *(const u32x4 *)(blk + 1024);
+            if constexpr (FP4W) bsc[nt] = ((const uint8_t *)ws)[(size_t)n * (K >> 5) + (kb >> 5) + g];
+        } else if constexpr (FP4W) {
+            bv[nt][0] = *(const u32x4 *)(wc + (size_t)n * (K >> 1) + (kb >> 1) + 16 * g);
+            bsc[nt] = ((const uint8_t *)ws)[(size_t)n * (K >> 5) + (kb >> 5) + g];
+        } else {
+            const uint8_t *row = wc + (size_t)n * K + kb;
+            bv[nt][0] = *(const u32x4 *)(row + 16 * g);
+            bv[nt][1] = *(const u32x4 *)(row + 64 + 16 * g);
+        }
+    }
+    float wsc = 0.f;
+    if constexpr (!FP4W) wsc = ((const float *)ws)[(size_t)(n0 >> 7) * KS + (kb >> 7)];
+    // 2. MFMAs
     f32x4 acc[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     const u32x4 z4 = {0, 0, 0, 0};
+    i32x8 b[NT];
 #pragma unroll
-    for (int s = 0; s < SW; s++) {
-        const bool live = s < nst;
-        i32x8 b[NT];
+    for (int nt = 0; nt < NT; nt++) {
+        const u32x4 b0 = live ? bv[nt][0] : z4;
+        if constexpr (FP4W) {
+            b[nt] = i32x8{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], 0, 0, 0, 0};
+        } else {
+            const u32x4 b1 = live ? bv[nt][1] : z4;
+            b[nt] = i32x8{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
+        }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        const u32x4 a0 = live ? av[mt][0] : z4, a1 = live ? av[mt][1] : z4;
+        const i32x8 a = {(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            const u32x4 b0 = live ? bv[s][nt][0] : z4;
             if constexpr (FP4W) {
-                b[nt] = i32x8{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], 0, 0, 0, 0};
+                acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[nt], acc[mt][nt], 0, 4, 0, (int)asc[mt],
+                                                                               0, (int)bsc[nt]);
             } else {
-                const u32x4 b1 = live ? bv[s][nt][1] : z4;
-                b[nt] = i32x8{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
-            }
-        }
+                const f32x4 d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[nt], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0,
+                                                                                  0, (int)asc[mt], 0, 127);
+                const float sw = live ? wsc : 0.f;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const u32x4 a0 = live ? av[s][mt][0] : z4, a1 = live ? av[s][mt][1] : z4;
-            const i32x8 a = {(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                if constexpr (FP4W) {
-                    acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[nt], acc[mt][nt], 0, 4, 0,
-                                                                                   (int)asc[s][mt], 0, (int)bsc[s][nt]);
-                } else {
-                    const f32x4 d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[nt], f32x4{0.f, 0.f, 0.f, 0.f},
-                                                                                      0, 0, 0, (int)asc[s][mt], 0, 127);
-                    const float sw = live ? wsc[s] : 0.f;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[mt][nt][e] = fmaf(sw, d[e], acc[mt][nt][e]);
-                }
+                for (int e = 0; e < 4; e++) acc[mt][nt][e] = fmaf(sw, d[e], acc[mt][nt][e]);
             }
         }
     }
@@ -278,11 +269,9 @@ __global__ __launch_bounds__(NW * 64) void k_gemm(const uint8_t *__restrict__ wc
 #pragma unroll
     for (int t = 0; t < MT * NT; t++) red[(wave * MT * NT + t) * 64 + lane] = acc[t / NT][t % NT];
     __syncthreads();
-    constexpr int kPer = (kTileVecs + kThreads - 1) / kThreads;
 #pragma unroll
-    for (int j = 0; j < kPer; j++) {
+    for (int j = 0; j < kTileVecs / kThreads; j++) {
         const int q = tid + kThreads * j;
-        if (q >= kTileVecs) break;
         f32x4 v = red[q];
 #pragma unroll
         for (int w = 1; w < NW; w++) v += red[w * kTileVecs + q];
@@ -292,10 +281,9 @@ __global__ __launch_bounds__(NW * 64) void k_gemm(const uint8_t *__restrict__ wc
 
 // Y = the slices' partial tiles added in slice order; thread i takes f32x4 i of every tile (the
 // layout k_gemm stored them in), so partial reads are contiguous per slice.
-template <int NT>
 __global__ __launch_bounds__(256) void k_gemm_reduce(const f32x4 *__restrict__ part, int slices, int ntiles,
                                                      void *__restrict__ y, int y_f32, int M, int N) {
-    constexpr int kTileVecs = 4 * NT * 64;
+    constexpr int NT = 4, kTileVecs = 4 * NT * 64;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= ntiles * kTileVecs) return;
     const int tile = i / kTileVecs, q = i % kTileVecs;
@@ -343,8 +331,8 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const f32x4 *__restrict__ p
 template <bool FP4W, int MT, int NT, int NW, int QW, bool AARR, bool WOPS>
 __global__ __launch_bounds__(NW * 64) void k_gemm_one(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
                                                       const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,
-                                                      void *__restrict__ y, int y_f32, int M, int N, int K, int lda,
-                                                      int act32, int ntiles) {
+                                                      void *__restrict__ y, int y_f32, int M, int N, int K, int act32,
+                                                      int ntiles) {
     constexpr int SW = 4 * QW;  // steps per wave
     constexpr int kTileVecs = MT * NT * 64;
     constexpr int kThreads = NW * 64;
@@ -435,7 +423,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_one(const uint8_t *__restrict_
                     av[s][mt][0] = *(const u32x4 *)blk;
                     av[s][mt][1] = *(const u32x4 *)(blk + 1024);
                 } else {
-                    const uint8_t *row = aq + (size_t)min(m0 + 16 * mt + r, M - 1) * lda + kb;
+                    const uint8_t *row = aq + (size_t)min(m0 + 16 * mt + r, M - 1) * K + kb;
                     av[s][mt][0] = *(const u32x4 *)(row + h0 + 16 * g);
                     av[s][mt][1] = *(const u32x4 *)(row + h1 + 16 * g);
                 }
@@ -549,7 +537,7 @@ __device__ __forceinline__ void wait_lds_vmem() {
 }
 
 template <bool FP4W, int BM, int BN, int WR, int WC, int S, bool CHAIN, bool WOPS>
-__global__ __launch_bounds__(WR *WC * 64, BM / WR * BN / WC >= 4096 ? 1 : 2) void k_gemm_tile(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
+__global__ __launch_bounds__(WR *WC * 64, 2) void k_gemm_tile(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
                                                       const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as4,
                                                       const uint8_t *__restrict__ ws4, void *__restrict__ y, int y_f32,
                                                       int M, int N, int K, int group, int mtiles, int ntiles) {
@@ -819,13 +807,12 @@ __global__ __launch_bounds__(256) void k_gemm_prep(const void *__restrict__ x, c
 // q form, FP4, against 64 rows a launch, us: 100 x 2048 x 7168 15.9 -> 11.3, 200 x 512 x 7168 38.6 -> 14.8,
 // 700 x 512 x 4096 100.9 -> 19.3 (2 x 4 tiles); against split K and its second launch: 64 x 4096 x 2176
 // 10.4 -> 5.7, 16 x 256 x 512 7.3 -> 3.6, 8 x 7168 x 2048 (64 x 32 tiles over 16 waves) 11.5 -> 6.5.
-template <bool FP4W, int MT, int NT, int NW, bool CHAIN, bool AARR, bool WOPS>
-__global__ __launch_bounds__(NW * 64) void k_gemm_waves(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
+template <bool FP4W, int MT, int NT, bool CHAIN, bool AARR, bool WOPS>
+__global__ __launch_bounds__(512) void k_gemm_waves(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
                                                         const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,
                                                         void *__restrict__ y, int y_f32, int M, int N, int K, int act32,
                                                         int group, int mtiles, int ntiles) {
-    constexpr int kTileVecs = MT * NT * 64, kThreads = NW * 64, kPer = (kTileVecs + kThreads - 1) / kThreads;
-    
+    constexpr int NW = 8, kTileVecs = MT * NT * 64, kThreads = NW * 64, kPer = (kTileVecs + kThreads - 1) / kThreads;
     __shared__ f32x4 red[NW * kTileVecs];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1027,11 +1014,11 @@ template <bool FP4W, bool WOPS>
 static hipError_t launch_split(const GemmPlan &p, const GemmArgs &c, void *work) {
     const int tiles = ceil_div(c.n, 64);
     f32x4 *part = (f32x4 *)work;
-    hipLaunchKernelGGL((k_gemm<FP4W, 4, 4, 8, WOPS>), dim3(tiles * p.slices), dim3(512), 0, c.st, c.codes, c.scales, c.aq,
+    hipLaunchKernelGGL((k_gemm<FP4W, WOPS>), dim3(tiles * p.slices), dim3(512), 0, c.st, c.codes, c.scales, c.aq,
                        c.as_, part, c.m, c.n, c.k, c.act_block == 32 ? 5 : 7, tiles, p.slices, p.group);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_gemm_reduce<4>, dim3(tiles * (4 * 4 * 64) / 256), dim3(256), 0, c.st, part, p.slices, tiles, c.y,
+    hipLaunchKernelGGL(k_gemm_reduce, dim3(tiles * (4 * 4 * 64) / 256), dim3(256), 0, c.st, part, p.slices, tiles, c.y,
                        c.y_f32, c.m, c.n);
     return hipGetLastError();
 }
@@ -1040,7 +1027,7 @@ template <bool FP4W, int MT, int NT, int NW, int QW, bool ARR, bool WOPS>
 static hipError_t launch_one(const GemmArgs &c) {
     const int tiles = ceil_div(c.n, 16 * NT);
     hipLaunchKernelGGL((k_gemm_one<FP4W, MT, NT, NW, QW, ARR, WOPS>), dim3(tiles * ceil_div(c.m, 16 * MT)), dim3(NW * 64), 0,
-                       c.st, c.codes, c.scales, c.aq, c.as_, c.y, c.y_f32, c.m, c.n, c.k, c.k, c.act_block == 32, tiles);
+                       c.st, c.codes, c.scales, c.aq, c.as_, c.y, c.y_f32, c.m, c.n, c.k, c.act_block == 32, tiles);
     return hipGetLastError();
 }
 
@@ -1048,7 +1035,7 @@ template <bool FP4W, int MT, int NT, bool ARR, bool WOPS>
 static hipError_t launch_waves(const GemmPlan &p, const GemmArgs &c) {
     const int mt = ceil_div(c.m, 16 * MT), nt = ceil_div(c.n, 16 * NT);
 #define STBL_WAVES(CHAIN)                                                                                             \
-    hipLaunchKernelGGL((k_gemm_waves<FP4W, MT, NT, 8, CHAIN, ARR, WOPS>), dim3((unsigned)mt * nt), dim3(512), 0, c.st,    \
+    hipLaunchKernelGGL((k_gemm_waves<FP4W, MT, NT, CHAIN, ARR, WOPS>), dim3((unsigned)mt * nt), dim3(512), 0, c.st,    \
                        c.codes, c.scales, c.aq, c.as_, c.y, c.y_f32, c.m, c.n, c.k, c.act_block == 32, p.group, mt, nt)
     if (p.chain) STBL_WAVES(true);
     else STBL_WAVES(false);
