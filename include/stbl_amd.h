@@ -233,7 +233,7 @@ int stbl_amd_gemm(int fmt, void *y, const void *codes, const void *scales, const
                   int act_block, int y_f32, void *work, hipStream_t st);
 
 /* The same GEMM on activations already quantized by stbl_amd_act_quant_e4m3: aq e4m3 codes [m][k]
- * (16-byte aligned), as E8M0 scale bytes [m][k/act_block]. One launch.
+ * (16-byte aligned), as E8M0 scale bytes [m][k/act_block]. One launch, two where K is split.
  * Replaces fp8_gemm(a, a_s, b, b_s) / fp4_gemm(a, a_s, b, b_s) of ref/kernel.py:85-102, which take
  * the quantized activation and its scales as arguments. */
 int stbl_amd_gemm_q(int fmt, void *y, const void *codes, const void *scales, const void *aq, const void *as, int m,
@@ -259,9 +259,9 @@ int stbl_amd_gemm_packed(int fmt, void *y, const void *packed, const void *scale
                          int act_block, int y_f32, void *work, hipStream_t st);
 
 /* stbl_amd_gemm / stbl_amd_gemm_q (packed != 0: on weight codes from stbl_amd_gemm_pack) on up to 8192 rows
- * in one call: the weights pass through the GPU once per 64 or 128 columns, not once per 64 rows. Every
- * full 64 rows' results are those of a call on them alone, bit for bit; a shorter last part is summed
- * as the others are. The rows of ref/kernel.py:85-102's a, whose number is not limited. */
+ * in one call: one launch over all the rows' tiles, 32 to 64 rows high, that read the weights through L2,
+ * not one per 64 rows. Every full 64 rows' results are those of a call on them alone, bit for bit; a
+ * shorter last part is summed as the others are. The rows of ref/kernel.py:85-102's a, whose number is not limited. */
 int stbl_amd_gemm_rows(int fmt, int packed, void *y, const void *codes, const void *scales, const void *x, int m, int n,
                        int k, int act_block, int y_f32, void *work, hipStream_t st);
 int stbl_amd_gemm_q_rows(int fmt, int packed, void *y, const void *codes, const void *scales, const void *aq, const void *as,

@@ -13,7 +13,7 @@
 //                     e2m1 weights. The activation scales (powers of two) and the FP4 weight scales
 //                     (E8M0) are the MFMA's own per-32 scale operands, so the hardware applies them
 //                     exactly; the FP8 weights' fp32 block scale multiplies each 128-K step's product
-//                     in fp32. gemm_plan chooses between them: k_gemm_one (the configurations' shapes)
+//                     in fp32. gemm_plan (gemm_plan.hpp) chooses between them: k_gemm_one (the configurations' shapes)
 //                     and k_gemm_waves, one launch over all of K by waves that each take a part of it;
 //                     k_gemm and k_gemm_reduce, split K; k_gemm_tile, many rows through LDS, on operands
 //                     laid out by k_gemm_prep;
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_one(const uint8_t *__restrict_
 // and a wave reads the next step's operands from LDS while its products of this one run. A and packed W
 // lie in LDS in operand order, row-major W with its 16-byte pieces permuted by the column, so that operand
 // reads hit every bank once.
-// The sum runs as a call of up to 64 rows at the same n and k sums (gemm_sum): steps in groups of `group`;
+// The sum runs as a call of 64 rows at the same n and k sums (gemm_plan): steps in groups of `group`;
 // within a group CHAIN keeps one running sum (FP4: in the MFMA's accumulator, FP8: an FMA per element and
 // step), otherwise each step's product is rounded and added; then the groups' sums are added in order.
 // Measured (FP4 / FP8, with k_gemm_prep, us) against 64 rows a launch: 1024 x 7168 x 2048 84.6 / 107.2 -> 31.1 /
@@ -802,11 +802,11 @@ __global__ __launch_bounds__(256) void k_gemm_prep(const void *__restrict__ x, c
 // owns a 16 MT x 16 NT output tile over all of K; wave w takes the groups w, w + NW, ... of `group` steps
 // each, loads its operands straight from global memory one step ahead of their products, and the groups'
 // sums are added in order through LDS, NW groups at a time. The waves of a tile need no barrier but the
-// sum's and no partial tiles in memory. The order of the sum is gemm_sum's, as in k_gemm_tile; chained
+// sum's and no partial tiles in memory. The order of the sum is gemm_plan's, as in k_gemm_tile; chained
 // groups (a multiple of 4 steps, 4- and 16-byte aligned scales) load their scales four steps at once.
 // q form, FP4, against 64 rows a launch, us: 100 x 2048 x 7168 15.9 -> 11.3, 200 x 512 x 7168 38.6 -> 14.8,
 // 700 x 512 x 4096 100.9 -> 19.3 (2 x 4 tiles); against split K and its second launch: 64 x 4096 x 2176
-// 10.4 -> 5.7, 16 x 256 x 512 7.3 -> 3.6, 8 x 7168 x 2048 (64 x 32 tiles over 16 waves) 11.5 -> 6.5.
+// 10.4 -> 5.9, 16 x 256 x 512 7.3 -> 3.2, 8 x 7168 x 2048 11.5 -> 6.5.
 template <bool FP4W, int MT, int NT, bool CHAIN, bool AARR, bool WOPS>
 __global__ __launch_bounds__(512) void k_gemm_waves(const uint8_t *__restrict__ wc, const void *__restrict__ ws,
                                                         const uint8_t *__restrict__ aq, const uint8_t *__restrict__ as_,

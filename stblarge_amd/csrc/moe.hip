@@ -5,21 +5,23 @@
 //   gemv_mxfp4_batch(gate, up) -> swiglu_batch(route weights) -> act_quant_fp8(mid) ->
 //   gemv_mxfp4_batch(down) -> shared expert -> axpy of every expert output in top-k order, then the
 //   shared one -> round_bf16.
-// Here the same arithmetic runs as three launches over a job table (one job = one expert slot and
-// the <= 4 tokens routed to it, each token with its own route weight):
+// Here the same arithmetic runs over a job table (one job = one expert slot and the <= 4 tokens routed
+// to it, each token with its own route weight), in three launches where one kernel takes every job:
 //   k_moe_gateup  gate and up rows of a job in the same workgroup; the epilogue rounds both to bf16
 //                 and applies SwiGLU with the token's route weight (stbl/kernels.cu:444-459), so
 //                 the gate/up outputs never leave the chip;
 //   k_moe_down    down rows of a job; output rounded to bf16 as the reference's GEMV does;
 //   k_moe_combine per token, the fp32 sum of its experts' outputs in top-k order plus the shared
 //                 expert's, rounded to bf16 (stbl/model.cu:589-592).
-// Jobs are compiled per token class (1, 2 or 3-4 tokens). A step whose jobs of one format span
-// several classes runs them all in one gate/up and one down launch (k_moe_gateup_any /
-// k_moe_down_any); otherwise each class has its launches, one launch holding both formats where a
-// class has FP4 and FP8 E8M0 jobs (k_moe_gateup_mix / k_moe_down_mix).
+// Jobs fall into token classes (1, 2 or 3-4 tokens). A step whose jobs of one format span several
+// classes runs them all in one gate/up and one down launch (k_moe_gateup_any / k_moe_down_any, which
+// have a body per token count); otherwise each class has its launches (3 tokens run the 4-token body),
+// one launch holding both formats where a class has FP4 and FP8 E8M0 jobs (k_moe_gateup_mix /
+// k_moe_down_mix).
 // In the reference's "official" numerics the expert input and the SwiGLU output are quantized to FP8
-// per 32 first (stbl/model.cu:510, :538); both kernels do that quantization in registers on the
-// lane's own chunk of the activation, so it costs no launch and no memory traffic.
+// per 32 first (stbl/model.cu:510, :538): by gate/up and down in registers, on the lane's own chunk
+// of the activation, without a launch or memory traffic; or, in large steps of several tokens, once, by
+// two launches of k_moe_act_quant (quantize_once).
 // The router is k_route: sigmoid scores, top-k by score + bias with ties to the lower id, weights
 // renormalized in top-k order (stbl/model.cu:444-451, :528-530 with sigmoid for sqrt-softplus).
 #include <algorithm>
@@ -702,7 +704,8 @@ static hipError_t launch_down(const MoeJobs &jobs, int n, const ExpertLayout &L,
     return launch_down_r<F, M, M == 4 ? 4 : 8>(jobs, n, L, h, o, dim, inter, official, out_f32, st);
 }
 
-// Token class of a job: 1 (one token), 2 (two) or 3 (three or four: the M = 4 templates).
+// Token class of a job: 1 (one token), 2 (two) or 3 (three or four; launches by class run both in the
+// M = 4 templates, run_jobs_any has one for 3).
 static int token_class(const MoeJob &J) { return J.m == 1 ? 1 : (J.m == 2 ? 2 : 3); }
 
 static bool several_classes(const MoeJob *all, int njobs) {

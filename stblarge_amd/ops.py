@@ -601,8 +601,9 @@ def _gemm_q_rows(packed, codes, scales, aq, a_s, fmt, act_block, out_f32, work):
 
 def gemm(codes, scales, x, fmt, act_block=128, out_f32=False, work=None):
     """Y [M, N] = act_quant(X, act_block) . Wdeq^T (fp4_gemm / fp8_gemm of ref/kernel.py), any M (each
-    output row depends only on its own activation row). `work` (from gemm_work) may be passed to reuse
-    the scratch across calls on one stream."""
+    output row depends only on its own activation row). `work` (from gemm_work, for at least min(M, 8192)
+    rows: a smaller one is left aside and the call allocates) may be passed to reuse the scratch across
+    calls on one stream."""
     _need(x, torch.bfloat16, "x", 2)
     if x.shape[0] < 1:
         raise ValueError("gemm: x has no rows")
