@@ -515,7 +515,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_one(const uint8_t *__restrict_
 // are the products alone (7.5 at the matrix cores' rate; a 64 x 128 tile's 16 steps are short against its
 // start and end), 9.5 the loads and LDS reads alone.
 // 64 lanes x 16 (4) bytes at base + off -> LDS at lds + 16 (4) x lane. The LDS address goes through M0,
-// which is left as it was. Counted by vmcnt (wait_vmem): the compiler's builtin for this load makes it
+// which is left as it was. Counted by vmcnt (wait_lds_vmem): the compiler's builtin for this load makes it
 // wait for every such load before any LDS read that could alias, which is each step's.
 __device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t *base, uint32_t off) {
     uint32_t keep;
